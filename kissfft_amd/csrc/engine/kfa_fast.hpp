@@ -65,6 +65,24 @@ struct Radices {
         return o;
     }
     static constexpr int tw_len() { return tw_off(K); }
+    // Where the stage tables of the second pass of a reference-order split start (kfa_tile.hpp:
+    // stage s has L1 * m(s) rows, so its offsets are L1 times these plus the rotations).
+    static constexpr int rot_len() { return round_up(2, G); }
+    static constexpr int rows_before(int s)
+    {
+        int o = 0;
+        for (int i = 0; i < s; ++i)
+            o += m(i) * PR(i);
+        return o;
+    }
+    static constexpr int gens_before(int s)
+    {
+        int o = 0;
+        for (int i = 0; i < s; ++i)
+            if (gen(i))
+                o += m(i) * GR(i);
+        return o;
+    }
     // Generic radices (any p but 2, 3, 4, 5, 8, 16).  Fixed point runs them as
     // kf_bfly_generic does (kiss_fft.c:191-233): output q1 of column u sums
     // C_MUL(x'_q, table[q * P * (u + q1 * m) mod N]) over q, so after the table above a
@@ -455,6 +473,16 @@ __device__ __forceinline__ void line_sync()
     }
 }
 
+// Entry type of a stage table (make_stage_table_raw: fmt 1 for packed Q15, else 0).
+template <class A>
+struct TwEntry {
+    typedef typename A::store2 type;
+};
+template <>
+struct TwEntry<Q15P> {
+    typedef uint2 type;
+};
+
 template <class A, bool INV, int T, class RS, int S, bool PAIRED>
 struct FastStage {
     typedef typename A::store2 St;
@@ -553,22 +581,37 @@ struct FastStage {
         }
     }
 
+    // Entries of the stage table: word pairs for packed Q15 (see kfa_q15p.hpp), else
+    // stored complex values.
+    typedef typename TwEntry<A>::type Ent;
+
     __device__ __forceinline__ static void compute(C (&v)[J][p], const St *__restrict__ stw, int t)
     {
         // m == 1: every butterfly's twiddles are table entry 0 (see ONE in kfa_arith.hpp)
-        constexpr bool ONE = A::fixed && m == 1;
+        const Ent *tab = reinterpret_cast<const Ent *>(stw);
+        compute_rows<m == 1>(v, tab + TWO, tab + TWO + m * PR, tab + RS::gen_off(S), 0, 1, t);
+    }
+
+    // The stage's butterflies with twiddle row u0 + um * u for column u (rows / grows: row 0
+    // of the stage's table and of its generic entries; rot: the two fixed rotations).
+    // FIRST: every row is row 0, whose twiddles are table entry 0.
+    template <bool FIRST>
+    __device__ __forceinline__ static void compute_rows(C (&v)[J][p], const Ent *__restrict__ rows,
+                                                        const Ent *__restrict__ rot, const Ent *__restrict__ grows,
+                                                        int u0, int um, int t)
+    {
+        constexpr bool ONE = A::fixed && FIRST;
 #pragma unroll
         for (int j = 0; j < J; ++j) {
             if (!live(t, j))
                 break;
             const int b = bidx(t, j);
-            const int u = b / P;
-            const St *row = stw + TWO + u * PR;
+            const int u = u0 + um * (b / P);
             if constexpr (IsPacked<A>::value && RS::gen(S)) {
                 // kf_bfly_generic (kiss_fft.c:191-233) on packed words: C_FIXDIV, then per
                 // output the packed C_MULs with the combined entries (word pairs) summed by
                 // packed 16-bit adds (C_ADDTO into kiss_fft_scalar)
-                const uint2 *grow = reinterpret_cast<const uint2 *>(stw) + RS::gen_off(S) + u * RS::GR(S);
+                const uint2 *grow = grows + u * RS::GR(S);
                 unsigned x[p];
 #pragma unroll
                 for (int q = 0; q < p; ++q)
@@ -585,8 +628,7 @@ struct FastStage {
                 }
             } else if constexpr (IsPacked<A>::value) {
                 // stage table of pre-arranged twiddle word pairs (see kfa_q15p.hpp)
-                const uint2 *tab = reinterpret_cast<const uint2 *>(stw);
-                const uint2 *trow = tab + TWO + u * PR;
+                const uint2 *trow = rows + u * PR;
                 uint2 w[p > 1 ? p - 1 : 1] = {};
                 if constexpr (!ONE) {
 #pragma unroll
@@ -602,10 +644,10 @@ struct FastStage {
                 } else if constexpr (p == 4) {
                     q15p::bfly4<INV, ONE>(x, w);
                 } else if constexpr (p == 3) {
-                    const uint2 ya = tab[TWO + m * PR];
+                    const uint2 ya = rot[0];
                     q15p::bfly3<ONE>(x, w, q15p::scal(q15p::lo16(ya.y)));
                 } else {
-                    const uint2 ya = tab[TWO + m * PR], yb = tab[TWO + m * PR + 1];
+                    const uint2 ya = rot[0], yb = rot[1];
                     q15p::Y5 y{q15p::scal(q15p::lo16(ya.x)), q15p::scal(q15p::lo16(ya.y)),
                                q15p::scal(q15p::lo16(yb.x)), q15p::scal(q15p::lo16(yb.y))};
                     q15p::bfly5<ONE>(x, w, y);
@@ -617,7 +659,7 @@ struct FastStage {
                 // kf_bfly_generic (kiss_fft.c:191-233): every input divided by p, then each
                 // output the first input plus the rounded products of the others with
                 // their table entries, summed in kiss_fft_scalar (C_ADDTO)
-                const St *grow = stw + RS::gen_off(S) + u * RS::GR(S);
+                const St *grow = grows + u * RS::GR(S);
                 C x[p];
 #pragma unroll
                 for (int q = 0; q < p; ++q)
@@ -631,14 +673,15 @@ struct FastStage {
                     v[j][q1] = acc;
                 }
             } else if constexpr (A::fixed) {
+                const St *row = rows + u * PR;
                 C w[p > 1 ? p - 1 : 1] = {};
                 if constexpr (!ONE) {
 #pragma unroll
                     for (int r = 1; r < p; ++r)
                         w[r - 1] = O::load(row[r - 1]);
                 }
-                const C ya = O::load(stw[TWO + m * PR]);
-                const C yb = O::load(stw[TWO + m * PR + 1]);
+                const C ya = O::load(rot[0]);
+                const C yb = O::load(rot[1]);
                 if constexpr (p == 2)
                     bfly2<A, ONE>(v[j], w);
                 else if constexpr (p == 3)
@@ -649,7 +692,8 @@ struct FastStage {
                     bfly5<A, ONE>(v[j], w, ya, yb);
                 (void)yb;
             } else {
-                if constexpr (m > 1) {
+                if constexpr (!FIRST) {
+                    const St *row = rows + u * PR;
 #pragma unroll
                     for (int r = 1; r < p; ++r)
                         v[j][r] = O::cmul(v[j][r], O::load(row[r - 1]));

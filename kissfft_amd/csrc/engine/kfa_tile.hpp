@@ -2,24 +2,32 @@
 //
 // A workgroup owns a tile of TL lines of N points.  Line l = (hi, lo), lo = l % nlo, reads
 // element e at in[hi*in_hi + lo*in_lo + e*in_el] and writes it at
-// out[hi*out_hi + lo*out_lo + e*out_el].  The tile moves between HBM and LDS in two
-// phases of its own, each with the thread mapping that makes wave accesses contiguous:
-//   * "column" phases (LCOL / SCOL): consecutive lanes take consecutive lines at the same
-//     element -- the layout of the non-last axes of an N-D array (kiss_fftnd.c:172-177
-//     walks the same columns) and of the first pass of the four-step split;
-//   * "row" phases: consecutive lanes take consecutive elements of one line.
-// In between, the stages of the radix schedule RS run LDS -> registers -> LDS exactly as
-// in the fast line kernel (FastStage, T threads per line).  Lines sit tile_pitch() values
-// apart in LDS so that lanes working on neighbouring lines fall in different banks.
+// out[hi*out_hi + lo*out_lo + e*out_el].  T threads work on a line.  The first stage reads
+// its inputs from HBM into registers, the last one writes its outputs from registers to
+// HBM, and only the hand-overs between stages go through LDS (a schedule of K stages
+// writes and reads the tile K - 1 times).  Consecutive lanes take consecutive lines at the
+// same element, so that wave accesses are contiguous where lines are neighbours in HBM:
+//   * column loads and stores: the non-last axes of an N-D array (kiss_fftnd.c:172-177
+//     walks the same columns), the first pass of the four-step split;
+//   * row loads (ROWS): the first stage alone maps consecutive lanes to consecutive
+//     elements of one line, for passes whose input lines are contiguous.
+// A thread's line is the lane's for every stage but a ROWS first stage, so a butterfly's
+// operands sit TL values apart in LDS and a wave touches TL neighbouring values per
+// element: the LDS rows are as free of bank conflicts as the HBM rows are contiguous
+// (tile_pos).
 //
 // TWID multiplies element e of line l by W^(lo*e), W = exp(-+2*pi*i/tw_n), on the way out:
 // the twiddle step between the two passes of the four-step split (Bailey, "FFTs in
 // external or hierarchical memory", 1990):  with n = n1 + N1*n2 and k = k2 + N2*k1,
 //   X[k2 + N2*k1] = sum_n1 W_N1^(n1*k1) * W_N^(n1*k2) * sum_n2 x[n1 + N1*n2] W_N2^(n2*k2).
 // W^a is read as hi[a >> 10] * lo[a & 1023] from two small tables (computed in FP64,
-// rounded once); a thread's IT elements share one such product and a per-line table of
-// W^(lo*T*k) in LDS.  The float path only: fixed-point long lines keep the reference's own
-// stage order (the general line kernel's two-pass split).
+// rounded once); a thread's outputs share one such product and a per-line table of the
+// steps between them in LDS.  The float path only.
+//
+// REF is the second pass of a fixed-point line longer than one LDS line, which keeps the
+// reference's own stage order: column u of a stage is column lo + L1*u of the full
+// transform (L1 = the product of the first pass's radices), so every line reads its own
+// rows of the full-length stage tables.  Neighbouring lines read neighbouring rows.
 #pragma once
 
 #include "kfa_fast.hpp"
@@ -36,6 +44,7 @@ struct TileArgs {
     long long in_hi, in_lo, in_el;
     long long out_hi, out_lo, out_el;
     int xcd_group;       // > 1: tiles g*G .. g*G+G-1 (which share cache lines) run on one XCD
+    int l1;              // REF: product of the first pass's radices
 };
 
 template <class A, bool INV, int T, class RS, int S>
@@ -59,14 +68,17 @@ __device__ __forceinline__ void tile_stages(std::integer_sequence<int, S...>, ty
 
 // Workgroup -> tile.  Workgroups are dealt to the 8 XCDs round-robin; with G tiles sharing
 // each cache line, the G tiles of a group go to one XCD back to back, so the line is
-// fetched into that XCD's L2 once.
+// fetched into that XCD's L2 once.  Every round of groups starts one XCD further: with rows
+// of a power of two values an XCD would otherwise read the same columns of every row,
+// which fall in few of its L2's channels (copying columns of 8 values of a 1024 x 1024
+// array, x64: 4.82 against 4.71 TB/s; 64 rows of 256 columns 5.67 against 5.46).
 __device__ __forceinline__ long long tile_of_block(long long b, long long ntiles, int G)
 {
     const long long full = ntiles / (8LL * G) * (8LL * G);  // complete groups; the tail in order
     if (G <= 1 || b >= full)
         return b;
     const long long x = b % 8, s = b / 8;
-    return ((s / G) * 8 + x) * G + s % G;
+    return ((s / G) * 8 + (x + s / G) % 8) * G + s % G;
 }
 
 // Line pitch in LDS.  The column phases put lanes ln = 0..TL-1 on neighbouring lines and
@@ -79,96 +91,221 @@ constexpr int tile_pitch()
     return N + (TL < 32 ? 32 / TL : 1);
 }
 
-template <class A, bool INV, int T, int TL, bool LCOL, bool SCOL, bool TWID, class RS>
+// The kernel streams: what bounds it is the access pattern of its column side.  Measured
+// against the form that staged the tile through LDS on both sides of the stages (same
+// sizes, alternating runs): 64x96x120 x16 74.3 -> 72.0 us, real 1024x1000 x32 forward and
+// inverse 270 -> 263 us, c2c 2^20 x64 488 -> 483 us.
+//
+// What a tile's mapping is made of (template argument MODE of k_tile).
+enum { TM_ROWS = 1, TM_TWID = 2, TM_REF = 4 };
+
+// LDS index of element e of tile line ln.  Column tiles: element rows of TL lines, back to
+// back; where such a row is shorter than the 128 bytes that one LDS access of 16 lanes
+// covers (TL < 16 values of 8 bytes), one more row is left free after every G elements,
+// G the last stage's even radix: its inputs are G elements apart, and with G + 1 rows
+// between them neighbouring butterflies fall in different banks.  A ROWS tile is written
+// with lanes along the elements: an odd row of TL + 1 values.
+template <int TL, int CB, bool ROWS, int G>
+struct TilePos {
+    static constexpr bool padded = !ROWS && TL * CB < 128 && G % 2 == 0;
+    static constexpr int row = ROWS ? TL + 1 : TL;
+    static constexpr int size(int n) { return (padded ? n + n / G : n) * row; }
+    __device__ __forceinline__ static int at(int e, int ln) { return (padded ? e + e / G : e) * row + ln; }
+};
+
+template <class A, bool INV, int T, int TL, int MODE, class RS>
+struct TileStages {
+    typedef typename A::store2 St;
+    typedef Ops<A> O;
+    typedef Cx<A> C;
+    static constexpr int K = RS::K;
+    static constexpr bool ROWS = (MODE & TM_ROWS) != 0;
+    typedef TilePos<TL, (int)sizeof(St), ROWS, RS::p(RS::K - 1)> Pos;
+    template <int S>
+    using Stage = FastStage<A, INV, T, RS, S, false>;
+
+    // stage S's butterflies on v; lo: the line's index (REF)
+    template <int S>
+    __device__ __forceinline__ static void compute(typename Stage<S>::C (&v)[Stage<S>::J][Stage<S>::p],
+                                                   const St *stw, int t, int l1, int lo)
+    {
+        typedef Stage<S> F;
+        if constexpr ((MODE & TM_REF) != 0) {
+            const typename F::Ent *tab = reinterpret_cast<const typename F::Ent *>(stw);
+            const typename F::Ent *rows = tab + (long long)l1 * RS::rows_before(S) + S * RS::rot_len();
+            const typename F::Ent *gens = tab + (long long)l1 * (RS::rows_before(K) + RS::gens_before(S)) +
+                                          K * RS::rot_len();
+            F::template compute_rows<false>(v, rows, rows + (long long)l1 * F::m * F::PR, gens, lo, l1, t);
+        } else {
+            F::compute(v, stw, t);
+        }
+    }
+
+    // Stages S .. K-1 from LDS; the last stage's outputs are left in `out`.
+    template <int S, class Last>
+    __device__ __forceinline__ static void from(St *buf, const St *stw, int ln, int t, int l1, int lo, Last &out)
+    {
+        typedef Stage<S> F;
+        auto gather = [&](auto &v) {
+#pragma unroll
+            for (int j = 0; j < F::J; ++j) {
+                if (!F::live(t, j))
+                    break;
+                const int b = F::bidx(t, j);
+                const int u = b / F::P, o = b - (b / F::P) * F::P;
+#pragma unroll
+                for (int r = 0; r < F::p; ++r)
+                    v[j][r] = O::load(buf[Pos::at(u * F::P * F::p + r * F::P + o, ln)]);
+            }
+        };
+        if constexpr (S == K - 1) {
+            gather(out);
+            compute<S>(out, stw, t, l1, lo);
+        } else {
+            C v[F::J][F::p];
+            gather(v);
+            compute<S>(v, stw, t, l1, lo);
+            __syncthreads();  // every input read before the tile is overwritten
+            put<S>(v, buf, ln, t);
+            __syncthreads();
+            from<S + 1>(buf, stw, ln, t, l1, lo, out);
+        }
+    }
+
+    template <int S, class V>
+    __device__ __forceinline__ static void put(V &v, St *buf, int ln, int t)
+    {
+        typedef Stage<S> F;
+#pragma unroll
+        for (int j = 0; j < F::J; ++j) {
+            if (!F::live(t, j))
+                break;
+#pragma unroll
+            for (int q = 0; q < F::p; ++q)
+                buf[Pos::at(F::bidx(t, j) + q * F::NB, ln)] = O::pack(v[j][q]);
+        }
+    }
+};
+
+// a / b and a % b, a, b >= 0: 32-bit where the launch allows it (small: nlines < 2^31)
+__device__ __forceinline__ void tile_divmod(long long a, long long b, bool small, long long &q, long long &r)
+{
+    if (small) {
+        const unsigned d = (unsigned)a / (unsigned)b;
+        q = d;
+        r = (unsigned)a - d * (unsigned)b;
+    } else {
+        q = a / b;
+        r = a - q * b;
+    }
+}
+
+template <class A, bool INV, int T, int TL, int MODE, class RS>
 __global__ void __launch_bounds__(T *TL) k_tile(TileArgs a)
 {
     typedef typename A::store2 St;
     typedef Ops<A> O;
     typedef Cx<A> C;
-    constexpr int N = RS::N();
-    constexpr int NS = tile_pitch<N, TL>();
-    constexpr int IT = N / T;  // elements per thread in the HBM phases
-    static_assert(N % T == 0, "threads per line must divide the length");
-    static_assert(!TWID || SCOL, "the four-step twiddle is applied on column stores");
-    extern __shared__ __align__(16) unsigned char kfa_tile_smem[];
-    St *buf = reinterpret_cast<St *>(kfa_tile_smem);
-    // TWID: per line, W^(lo*T*k) for k < IT; a thread's element e = e0 + k*T then takes
-    // W^(lo*e) = W^(lo*e0) * W^(lo*T*k) (one table product per thread, one per line and k)
+    typedef TileStages<A, INV, T, TL, MODE, RS> TS;
+    constexpr int N = RS::N(), K = RS::K;
+    constexpr bool ROWS = TS::ROWS, TWID = (MODE & TM_TWID) != 0;
+    typedef typename TS::template Stage<0> F0;
+    typedef typename TS::template Stage<K - 1> FL;
+    static_assert(K > 1 || !ROWS, "a one-stage tile has one mapping");
+    static_assert(!(TWID && A::fixed), "the four-step twiddle is float");
+    // outputs per thread, and the W^(lo*step) between them
+    constexpr int IT = FL::J * FL::p;
+    __shared__ __align__(16) St buf[K > 1 ? TS::Pos::size(N) : 1];
     __shared__ St s_step[TWID ? TL * IT : 1];
 
     const int tid = threadIdx.x;
     const long long ntiles = (a.nlines + TL - 1) / TL;
     const long long l0 = tile_of_block(blockIdx.x, ntiles, a.xcd_group) * TL;
     const int nl = (int)((a.nlines - l0) < TL ? (a.nlines - l0) : TL);
+    const bool small = a.nlines < 0x7fffffffLL && a.nlo < 0x7fffffffLL;
+    const St *stw = reinterpret_cast<const St *>(__builtin_assume_aligned(a.stw, 16));
 
-    // HBM phases: each thread owns one line and IT of its elements.  Column mapping:
-    // lanes take consecutive lines (line = tid % TL), element e0 + k*T; row mapping:
-    // T lanes take consecutive elements of one line (line = tid / T).
-    auto line_of = [&](bool col) { return col ? tid % TL : tid / T; };
-    auto elem0 = [&](bool col) { return col ? tid / TL : tid % T; };
+    // the thread's line in the column mapping
+    const int ln = tid % TL, t = tid / TL;
+    const bool ok = ln < nl;
+    long long hi, lo;
+    tile_divmod(l0 + (ok ? ln : 0), a.nlo, small, hi, lo);
 
-    {
-        const int ln = line_of(LCOL), e0 = elem0(LCOL);
-        const bool ok = ln < nl;
-        const long long gl = l0 + (ok ? ln : 0);
-        const long long hi = gl / a.nlo, lo = gl - hi * a.nlo;
-        const St *src = reinterpret_cast<const St *>(a.in) + hi * a.in_hi + lo * a.in_lo + e0 * a.in_el;
-        const long long step = (long long)T * a.in_el;
-        St v[IT];
-#pragma unroll
-        for (int k = 0; k < IT; ++k)
-            if (ok)
-                v[k] = src[k * step];
-#pragma unroll
-        for (int k = 0; k < IT; ++k)
-            if (ok)
-                buf[ln * NS + e0 + k * T] = v[k];
-    }
-    if constexpr (TWID) {
-        const St *whi = reinterpret_cast<const St *>(a.tw_hi);
-        const St *wlo = reinterpret_cast<const St *>(a.tw_lo);
-        for (int w = tid; w < TL * IT; w += T * TL) {
-            const int ln = w / IT, k = w - (w / IT) * IT;
-            const long long gl = l0 + (ln < nl ? ln : 0);
-            const unsigned long long lo = (unsigned long long)(gl % a.nlo);
-            const unsigned long long ex = lo * (unsigned)(k * T);  // < tw_n
-            s_step[w] = O::pack(O::cmul(O::load(whi[ex >> 10]), O::load(wlo[ex & 1023])));
+    C out[FL::J][FL::p];
+    {   // first stage: HBM -> registers (m == 1: input r of butterfly b is element r*NB + b)
+        const int t0 = ROWS ? tid % T : t;
+        long long h0 = hi, o0 = lo;
+        bool ok0 = ok;
+        if constexpr (ROWS) {
+            ok0 = tid / T < nl;
+            tile_divmod(l0 + (ok0 ? tid / T : 0), a.nlo, small, h0, o0);
         }
-    }
-    __syncthreads();
-
-    {
-        const int line = tid / T, t = tid - line * T;
-        tile_stages<A, INV, T, RS>(std::make_integer_sequence<int, RS::K>{}, buf + line * NS,
-                                   reinterpret_cast<const St *>(a.stw), t);
-    }
-    if constexpr (64 % T == 0)
-        __syncthreads();  // every line done before the store phase reads across lines
-
-    {
-        const int ln = line_of(SCOL), e0 = elem0(SCOL);
-        if (ln >= nl)
-            return;
-        const long long gl = l0 + ln;
-        const long long hi = gl / a.nlo, lo = gl - hi * a.nlo;
-        St *dst = reinterpret_cast<St *>(a.out) + hi * a.out_hi + lo * a.out_lo + e0 * a.out_el;
-        const long long step = (long long)T * a.out_el;
-        C v[IT];
+        const St *src = reinterpret_cast<const St *>(a.in) + h0 * a.in_hi + o0 * a.in_lo;
+        const long long step = (long long)F0::NB * a.in_el;
+        C v[F0::J][F0::p];
 #pragma unroll
-        for (int k = 0; k < IT; ++k)
-            v[k] = O::load(buf[ln * NS + e0 + k * T]);
+        for (int j = 0; j < F0::J; ++j) {
+            const St *p0 = src + (long long)(t0 + j * T) * a.in_el;
+            const bool get = ok0 && F0::live(t0, j);
+#pragma unroll
+            for (int r = 0; r < F0::p; ++r)
+                v[j][r] = get ? O::load(p0[r * step]) : O::zero();
+        }
         if constexpr (TWID) {
             const St *whi = reinterpret_cast<const St *>(a.tw_hi);
             const St *wlo = reinterpret_cast<const St *>(a.tw_lo);
-            const unsigned long long ex = (unsigned long long)lo * (unsigned)e0;  // < tw_n
-            const C base = O::cmul(O::load(whi[ex >> 10]), O::load(wlo[ex & 1023]));
-#pragma unroll
-            for (int k = 0; k < IT; ++k)
-                v[k] = O::cmul(v[k], O::cmul(base, O::load(s_step[ln * IT + k])));
+            for (int w = tid; w < TL * IT; w += T * TL) {
+                const int l = w / IT, i = w - (w / IT) * IT;
+                long long h, o;
+                tile_divmod(l0 + (l < nl ? l : 0), a.nlo, small, h, o);
+                // element jT + q*NB of the thread's first, i = j*p + q (< tw_n: lo < tw_n / N)
+                const unsigned long long ex =
+                    (unsigned long long)o * (unsigned)((i / FL::p) * T + (i % FL::p) * FL::NB);
+                s_step[w] = O::pack(O::cmul(O::load(whi[ex >> 10]), O::load(wlo[ex & 1023])));
+            }
         }
+        if constexpr (K == 1) {
+            TS::template compute<0>(v, stw, t0, a.l1, (int)lo);
 #pragma unroll
-        for (int k = 0; k < IT; ++k)
-            dst[k * step] = O::pack(v[k]);
+            for (int j = 0; j < F0::J; ++j)
+#pragma unroll
+                for (int r = 0; r < F0::p; ++r)
+                    out[j][r] = v[j][r];
+            if constexpr (TWID)
+                __syncthreads();  // the step table
+        } else {
+            TS::template compute<0>(v, stw, t0, a.l1, (int)o0);
+            TS::template put<0>(v, buf, ROWS ? tid / T : ln, t0);
+            __syncthreads();
+        }
+    }
+    if constexpr (K > 1)
+        TS::template from<1>(buf, stw, ln, t, a.l1, (int)lo, out);
+
+    if (!ok)
+        return;
+    St *dst = reinterpret_cast<St *>(a.out) + hi * a.out_hi + lo * a.out_lo;
+    const long long step = (long long)FL::NB * a.out_el;
+    if constexpr (TWID) {
+        const St *whi = reinterpret_cast<const St *>(a.tw_hi);
+        const St *wlo = reinterpret_cast<const St *>(a.tw_lo);
+        const unsigned long long ex = (unsigned long long)lo * (unsigned)t;  // < tw_n
+        const C base = O::cmul(O::load(whi[ex >> 10]), O::load(wlo[ex & 1023]));
+#pragma unroll
+        for (int j = 0; j < FL::J; ++j)
+#pragma unroll
+            for (int q = 0; q < FL::p; ++q)
+                if (FL::live(t, j))
+                    out[j][q] = O::cmul(out[j][q], O::cmul(base, O::load(s_step[ln * IT + j * FL::p + q])));
+    }
+#pragma unroll
+    for (int j = 0; j < FL::J; ++j) {
+        if (!FL::live(t, j))
+            break;
+        St *p0 = dst + (long long)(t + j * T) * a.out_el;
+#pragma unroll
+        for (int q = 0; q < FL::p; ++q)
+            p0[q * step] = O::pack(out[j][q]);
     }
 }
 

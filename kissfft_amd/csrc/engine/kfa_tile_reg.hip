@@ -18,19 +18,12 @@
 
 namespace kfa {
 
-template <bool INV, int T, int TL, bool LCOL, bool SCOL, bool TWID, class RS>
+template <bool INV, int T, int TL, int MODE, class RS>
 static int launch_tile(const TileArgs &a, long long blocks, hipStream_t s)
 {
-    const size_t lds = (size_t)TL * tile_pitch<RS::N(), TL>() * sizeof(float2);
-    static std::once_flag once;
-    std::call_once(once, [=] {
-        (void)hipFuncSetAttribute((const void *)k_tile<F32, INV, T, TL, LCOL, SCOL, TWID, RS>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    });
     if (blocks <= 0)
         return 0;
-    hipLaunchKernelGGL((k_tile<F32, INV, T, TL, LCOL, SCOL, TWID, RS>), dim3((unsigned)blocks), dim3(T * TL), lds,
-                       s, a);
+    hipLaunchKernelGGL((k_tile<F32, INV, T, TL, MODE, RS>), dim3((unsigned)blocks), dim3(T * TL), 0, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
@@ -40,9 +33,10 @@ static void add_tile(std::vector<TileVariant> &v, const char *name)
     constexpr int G = 2;  // 16-byte stage-table rows of float2
     typedef Radices<G, R...> RS;
     static_assert(T * TL <= 1024, "workgroup too large");
-    static_assert((size_t)TL * tile_pitch<RS::N(), TL>() * 8 <= 160 * 1024, "tile exceeds LDS");
     for (int mode = 0; mode < 3; ++mode)
         for (int inv = 0; inv < 2; ++inv) {
+            if (mode == TILE_ROWS_TO_COLS && RS::K == 1)
+                continue;  // (such lines are never the second pass of a four-step split)
             TileVariant f;
             f.n = RS::N();
             f.inverse = inv;
@@ -52,18 +46,15 @@ static void add_tile(std::vector<TileVariant> &v, const char *name)
             f.radices = {R...};
             f.tw_pad = G;
             f.tw_len = RS::tw_len();
-            f.lds = (size_t)TL * tile_pitch<RS::N(), TL>() * 8;
+            f.lds = 0;
             f.name = name;
             f.launch_real = nullptr;
             if (mode == TILE_COLS)
-                f.launch = inv ? &launch_tile<true, T, TL, true, true, false, RS>
-                               : &launch_tile<false, T, TL, true, true, false, RS>;
+                f.launch = inv ? &launch_tile<true, T, TL, 0, RS> : &launch_tile<false, T, TL, 0, RS>;
             else if (mode == TILE_COLS_TWID)
-                f.launch = inv ? &launch_tile<true, T, TL, true, true, true, RS>
-                               : &launch_tile<false, T, TL, true, true, true, RS>;
-            else
-                f.launch = inv ? &launch_tile<true, T, TL, false, true, false, RS>
-                               : &launch_tile<false, T, TL, false, true, false, RS>;
+                f.launch = inv ? &launch_tile<true, T, TL, TM_TWID, RS> : &launch_tile<false, T, TL, TM_TWID, RS>;
+            else if constexpr (RS::K > 1)
+                f.launch = inv ? &launch_tile<true, T, TL, TM_ROWS, RS> : &launch_tile<false, T, TL, TM_ROWS, RS>;
             v.push_back(f);
         }
 }
@@ -117,16 +108,19 @@ const std::vector<TileVariant> &tile_registry()
     static std::vector<TileVariant> *reg = [] {
         auto *v = new std::vector<TileVariant>();
         add_tile<8, 64, 8, 8>(*v, "tile64_88_t8x64");
-        add_tile<16, 32, 8, 4, 3>(*v, "tile96_843_t16x32");
+        // 64x96x120 x16, the 96 axis: t8x32 30.8 us, t16x32 32.5, t12x32 31.7, t8x16 31.5
+        add_tile<8, 32, 8, 4, 3>(*v, "tile96_843_t8x32");
         add_tile<16, 32, 8, 16>(*v, "tile128_816_t16x32");
         add_tile<16, 16, 16, 16>(*v, "tile256_1616_t16x16");
         // first registered = preferred unless another wins the HBM-sized tuning by 4 %
         // (t64x8 is the fastest of the 512 and 1024 tiles on multi-GiB batches)
         add_tile<64, 8, 8, 8, 8>(*v, "tile512_888_t64x8");
         add_tile<64, 16, 8, 8, 8>(*v, "tile512_888_t64x16");
-        add_tile<64, 8, 16, 16, 4>(*v, "tile1024_16164_t64x8");
-        add_tile<64, 4, 16, 16, 4>(*v, "tile1024_16164_t64x4");
-        add_tile<64, 16, 16, 16, 4>(*v, "tile1024_16164_t64x16");
+        // c2c 2^20 x64, column pass: 4, 16, 16 241 us, 16, 8, 8 244, 16, 16, 4 276 (its
+        // last stage's padding leaves LDS for one workgroup per CU); four lines 314 us
+        add_tile<64, 8, 4, 16, 16>(*v, "tile1024_41616_t64x8");
+        add_tile<64, 8, 16, 8, 8>(*v, "tile1024_1688_t64x8");
+        add_tile<64, 16, 16, 8, 8>(*v, "tile1024_1688_t64x16");
         add_tile<16, 32, 16, 16>(*v, "tile256_1616_t16x32");
         add_tile<16, 16, 8, 16>(*v, "tile128_816_t16x16");
         add_tile<8, 32, 8, 8>(*v, "tile64_88_t8x32");
