@@ -96,18 +96,27 @@ constexpr int tile_pitch()
 // sizes, alternating runs): 64x96x120 x16 74.3 -> 72.0 us, real 1024x1000 x32 forward and
 // inverse 270 -> 263 us, c2c 2^20 x64 488 -> 483 us.
 //
+// HALF hands one component over at a time (real parts, then imaginary parts through the
+// same space): half the LDS per line, so twice the lines fit a workgroup.  For lengths whose
+// rows would otherwise be shorter than a 128-byte line (8 lines of 8-byte values) that
+// is worth the extra barriers: the copy of 1024 rows of 8 columns runs at 4.8 TB/s, of 16
+// columns at 5.2-5.4.
+//
 // What a tile's mapping is made of (template argument MODE of k_tile).
-enum { TM_ROWS = 1, TM_TWID = 2, TM_REF = 4 };
+enum { TM_ROWS = 1, TM_TWID = 2, TM_REF = 4, TM_HALF = 8 };
 
 // LDS index of element e of tile line ln.  Column tiles: element rows of TL lines, back to
-// back; where such a row is shorter than the 128 bytes that one LDS access of 16 lanes
-// covers (TL < 16 values of 8 bytes), one more row is left free after every G elements,
-// G the last stage's even radix: its inputs are G elements apart, and with G + 1 rows
-// between them neighbouring butterflies fall in different banks.  A ROWS tile is written
-// with lanes along the elements: an odd row of TL + 1 values.
+// back; where such a row of 8-byte values is shorter than the 128 bytes that one LDS access
+// of 16 lanes covers (TL < 16), one more row is left free after every G elements, G the
+// last stage's even radix: its inputs are G elements apart, and with G + 1 rows between
+// them neighbouring butterflies fall in different banks.  (Not for 4-byte slots: the
+// padded index needs an address register per access, 77 instead of 63 registers for 1024
+// points, and a second workgroup per CU is worth more than the two-way conflict of the
+// last gather.)  A ROWS tile is written with lanes along the elements: an odd row of
+// TL + 1 values.
 template <int TL, int CB, bool ROWS, int G>
 struct TilePos {
-    static constexpr bool padded = !ROWS && TL * CB < 128 && G % 2 == 0;
+    static constexpr bool padded = !ROWS && CB >= 8 && TL * CB < 128 && G % 2 == 0;
     static constexpr int row = ROWS ? TL + 1 : TL;
     static constexpr int size(int n) { return (padded ? n + n / G : n) * row; }
     __device__ __forceinline__ static int at(int e, int ln) { return (padded ? e + e / G : e) * row + ln; }
@@ -119,15 +128,24 @@ struct TileStages {
     typedef Ops<A> O;
     typedef Cx<A> C;
     static constexpr int K = RS::K;
-    static constexpr bool ROWS = (MODE & TM_ROWS) != 0;
-    typedef TilePos<TL, (int)sizeof(St), ROWS, RS::p(RS::K - 1)> Pos;
+    static constexpr bool ROWS = (MODE & TM_ROWS) != 0, HALF = (MODE & TM_HALF) != 0;
+    // what LDS holds: whole values, or (HALF) one component of every value at a time
+    template <bool H, class X>
+    struct Slot {
+        typedef typename X::store2 type;
+    };
+    template <class X>
+    struct Slot<true, X> {
+        typedef typename X::scalar type;
+    };
+    typedef typename Slot<HALF, A>::type L;
+    typedef TilePos<TL, (int)sizeof(L), ROWS, RS::p(RS::K - 1)> Pos;
     template <int S>
     using Stage = FastStage<A, INV, T, RS, S, false>;
 
     // stage S's butterflies on v; lo: the line's index (REF)
-    template <int S>
-    __device__ __forceinline__ static void compute(typename Stage<S>::C (&v)[Stage<S>::J][Stage<S>::p],
-                                                   const St *stw, int t, int l1, int lo)
+    template <int S, class V>
+    __device__ __forceinline__ static void compute(V &v, const St *stw, int t, int l1, int lo)
     {
         typedef Stage<S> F;
         if constexpr ((MODE & TM_REF) != 0) {
@@ -141,48 +159,57 @@ struct TileStages {
         }
     }
 
-    // Stages S .. K-1 from LDS; the last stage's outputs are left in `out`.
-    template <int S, class Last>
-    __device__ __forceinline__ static void from(St *buf, const St *stw, int ln, int t, int l1, int lo, Last &out)
-    {
-        typedef Stage<S> F;
-        auto gather = [&](auto &v) {
-#pragma unroll
-            for (int j = 0; j < F::J; ++j) {
-                if (!F::live(t, j))
-                    break;
-                const int b = F::bidx(t, j);
-                const int u = b / F::P, o = b - (b / F::P) * F::P;
-#pragma unroll
-                for (int r = 0; r < F::p; ++r)
-                    v[j][r] = O::load(buf[Pos::at(u * F::P * F::p + r * F::P + o, ln)]);
-            }
-        };
-        if constexpr (S == K - 1) {
-            gather(out);
-            compute<S>(out, stw, t, l1, lo);
-        } else {
-            C v[F::J][F::p];
-            gather(v);
-            compute<S>(v, stw, t, l1, lo);
-            __syncthreads();  // every input read before the tile is overwritten
-            put<S>(v, buf, ln, t);
-            __syncthreads();
-            from<S + 1>(buf, stw, ln, t, l1, lo, out);
-        }
-    }
-
-    template <int S, class V>
-    __device__ __forceinline__ static void put(V &v, St *buf, int ln, int t)
+    // f(j, r, element) for every input (IN) or output of the thread's stage-S butterflies
+    template <int S, bool IN, class Fn>
+    __device__ __forceinline__ static void each(int t, Fn f)
     {
         typedef Stage<S> F;
 #pragma unroll
         for (int j = 0; j < F::J; ++j) {
             if (!F::live(t, j))
                 break;
+            const int b = F::bidx(t, j);
+            const int u = b / F::P, o = b - (b / F::P) * F::P;
 #pragma unroll
-            for (int q = 0; q < F::p; ++q)
-                buf[Pos::at(F::bidx(t, j) + q * F::NB, ln)] = O::pack(v[j][q]);
+            for (int r = 0; r < F::p; ++r)
+                f(j, r, IN ? u * F::P * F::p + r * F::P + o : b + r * F::NB);
+        }
+    }
+
+    // Outputs v of stage S (line lw, thread tw of it) through LDS to the inputs n of stage
+    // S + 1 (line ln, thread t).  HALF: real parts first, then the imaginary ones through
+    // the same space, so that a tile of twice the lines fits.
+    template <int S, class V, class W>
+    __device__ __forceinline__ static void hand_over(V &v, W &n, L *buf, int lw, int tw, int ln, int t)
+    {
+        if constexpr (HALF) {
+            each<S, false>(tw, [&](int j, int r, int e) { buf[Pos::at(e, lw)] = v[j][r].r; });
+            __syncthreads();
+            each<S + 1, true>(t, [&](int j, int r, int e) { n[j][r].r = buf[Pos::at(e, ln)]; });
+            __syncthreads();
+            each<S, false>(tw, [&](int j, int r, int e) { buf[Pos::at(e, lw)] = v[j][r].i; });
+            __syncthreads();
+            each<S + 1, true>(t, [&](int j, int r, int e) { n[j][r].i = buf[Pos::at(e, ln)]; });
+        } else {
+            each<S, false>(tw, [&](int j, int r, int e) { buf[Pos::at(e, lw)] = O::pack(v[j][r]); });
+            __syncthreads();
+            each<S + 1, true>(t, [&](int j, int r, int e) { n[j][r] = O::load(buf[Pos::at(e, ln)]); });
+        }
+    }
+
+    // Stages S .. K-1 on v, the inputs of stage S; the last stage's outputs are left in `out`.
+    template <int S, class V, class Last>
+    __device__ __forceinline__ static void from(V &v, L *buf, const St *stw, int ln, int t, int l1, int lo, Last &out)
+    {
+        compute<S>(v, stw, t, l1, lo);
+        __syncthreads();  // every input read before the tile is overwritten
+        if constexpr (S + 1 == K - 1) {
+            hand_over<S>(v, out, buf, ln, t, ln, t);
+            compute<K - 1>(out, stw, t, l1, lo);
+        } else {
+            C n[Stage<S + 1>::J][Stage<S + 1>::p];
+            hand_over<S>(v, n, buf, ln, t, ln, t);
+            from<S + 1>(n, buf, stw, ln, t, l1, lo, out);
         }
     }
 };
@@ -201,7 +228,7 @@ __device__ __forceinline__ void tile_divmod(long long a, long long b, bool small
 }
 
 template <class A, bool INV, int T, int TL, int MODE, class RS>
-__global__ void __launch_bounds__(T *TL) k_tile(TileArgs a)
+__global__ void __launch_bounds__(T *TL, (MODE & TM_HALF) ? 2 * T * TL / 256 : 1) k_tile(TileArgs a)
 {
     typedef typename A::store2 St;
     typedef Ops<A> O;
@@ -215,7 +242,7 @@ __global__ void __launch_bounds__(T *TL) k_tile(TileArgs a)
     static_assert(!(TWID && A::fixed), "the four-step twiddle is float");
     // outputs per thread, and the W^(lo*step) between them
     constexpr int IT = FL::J * FL::p;
-    __shared__ __align__(16) St buf[K > 1 ? TS::Pos::size(N) : 1];
+    __shared__ __align__(16) typename TS::L buf[K > 1 ? TS::Pos::size(N) : 1];
     __shared__ St s_step[TWID ? TL * IT : 1];
 
     const int tid = threadIdx.x;
@@ -264,8 +291,9 @@ __global__ void __launch_bounds__(T *TL) k_tile(TileArgs a)
                 s_step[w] = O::pack(O::cmul(O::load(whi[ex >> 10]), O::load(wlo[ex & 1023])));
             }
         }
+        TS::template compute<0>(v, stw, t0, a.l1, (int)o0);
+        const int lw = ROWS ? tid / T : ln;
         if constexpr (K == 1) {
-            TS::template compute<0>(v, stw, t0, a.l1, (int)lo);
 #pragma unroll
             for (int j = 0; j < F0::J; ++j)
 #pragma unroll
@@ -273,14 +301,16 @@ __global__ void __launch_bounds__(T *TL) k_tile(TileArgs a)
                     out[j][r] = v[j][r];
             if constexpr (TWID)
                 __syncthreads();  // the step table
+        } else if constexpr (K == 2) {
+            TS::template hand_over<0>(v, out, buf, lw, t0, ln, t);
+            TS::template compute<1>(out, stw, t, a.l1, (int)lo);
         } else {
-            TS::template compute<0>(v, stw, t0, a.l1, (int)o0);
-            TS::template put<0>(v, buf, ROWS ? tid / T : ln, t0);
-            __syncthreads();
+            typedef typename TS::template Stage<1> F1;
+            C n[F1::J][F1::p];
+            TS::template hand_over<0>(v, n, buf, lw, t0, ln, t);
+            TS::template from<1>(n, buf, stw, ln, t, a.l1, (int)lo, out);
         }
     }
-    if constexpr (K > 1)
-        TS::template from<1>(buf, stw, ln, t, a.l1, (int)lo, out);
 
     if (!ok)
         return;

@@ -27,8 +27,8 @@ static int launch_tile(const TileArgs &a, long long blocks, hipStream_t s)
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-template <int T, int TL, int... R>
-static void add_tile(std::vector<TileVariant> &v, const char *name)
+template <int HALF, int T, int TL, int... R>
+static void add_tile_mode(std::vector<TileVariant> &v, const char *name)
 {
     constexpr int G = 2;  // 16-byte stage-table rows of float2
     typedef Radices<G, R...> RS;
@@ -50,13 +50,26 @@ static void add_tile(std::vector<TileVariant> &v, const char *name)
             f.name = name;
             f.launch_real = nullptr;
             if (mode == TILE_COLS)
-                f.launch = inv ? &launch_tile<true, T, TL, 0, RS> : &launch_tile<false, T, TL, 0, RS>;
+                f.launch = inv ? &launch_tile<true, T, TL, HALF, RS> : &launch_tile<false, T, TL, HALF, RS>;
             else if (mode == TILE_COLS_TWID)
-                f.launch = inv ? &launch_tile<true, T, TL, TM_TWID, RS> : &launch_tile<false, T, TL, TM_TWID, RS>;
+                f.launch = inv ? &launch_tile<true, T, TL, HALF + TM_TWID, RS> : &launch_tile<false, T, TL, HALF + TM_TWID, RS>;
             else if constexpr (RS::K > 1)
-                f.launch = inv ? &launch_tile<true, T, TL, TM_ROWS, RS> : &launch_tile<false, T, TL, TM_ROWS, RS>;
+                f.launch = inv ? &launch_tile<true, T, TL, HALF + TM_ROWS, RS> : &launch_tile<false, T, TL, HALF + TM_ROWS, RS>;
             v.push_back(f);
         }
+}
+
+template <int T, int TL, int... R>
+static void add_tile(std::vector<TileVariant> &v, const char *name)
+{
+    add_tile_mode<0, T, TL, R...>(v, name);
+}
+
+// The same with component-wise hand-overs (TM_HALF).
+template <int T, int TL, int... R>
+static void add_htile(std::vector<TileVariant> &v, const char *name)
+{
+    add_tile_mode<TM_HALF, T, TL, R...>(v, name);
 }
 
 template <bool MERGE, int T, int TL, class RS>
@@ -116,11 +129,13 @@ const std::vector<TileVariant> &tile_registry()
         // (t64x8 is the fastest of the 512 and 1024 tiles on multi-GiB batches)
         add_tile<64, 8, 8, 8, 8>(*v, "tile512_888_t64x8");
         add_tile<64, 16, 8, 8, 8>(*v, "tile512_888_t64x16");
-        // c2c 2^20 x64, column pass: 4, 16, 16 241 us, 16, 8, 8 244, 16, 16, 4 276 (its
-        // last stage's padding leaves LDS for one workgroup per CU); four lines 314 us
+        // 1024 lines of 16 values would leave LDS for one workgroup per CU: one component at
+        // a time, two workgroups of 1024 threads (63 registers) fill it.  c2c 2^20 x64,
+        // column / row pass: 227 / 213 us against 246 / 220 with 8 lines of whole values;
+        // 1024 x 501 columns x32 53 against 59 us.  32 threads a line 231-237 us, radices
+        // 8, 8, 4, 4 235 us, 16 lines of whole values 272 us.
+        add_htile<64, 16, 16, 8, 8>(*v, "htile1024_1688_t64x16");
         add_tile<64, 8, 4, 16, 16>(*v, "tile1024_41616_t64x8");
-        add_tile<64, 8, 16, 8, 8>(*v, "tile1024_1688_t64x8");
-        add_tile<64, 16, 16, 8, 8>(*v, "tile1024_1688_t64x16");
         add_tile<16, 32, 16, 16>(*v, "tile256_1616_t16x32");
         add_tile<16, 16, 8, 16>(*v, "tile128_816_t16x16");
         add_tile<8, 32, 8, 8>(*v, "tile64_88_t8x32");

@@ -210,3 +210,19 @@ def test_forced_rtile(n, name, monkeypatch):
         assert rel_l2(y, np.fft.irfft(cplx(Xin), n=N, axis=-1) * N) <= ABS_FLOAT_BOUND, name
     finally:
         lib.L.kiss_fft_cleanup()
+
+
+def htile_registry():
+    out = []
+    for m in re.finditer(r"add_htile<([^>]*)>\(\*v,\s*\"(\w+)\"\)", open(TREG).read()):
+        a = [int(x) for x in m.group(1).split(",")]
+        out.append((int(np.prod(a[2:])), m.group(2)))
+    return out
+
+
+@pytest.mark.parametrize("n,name", htile_registry(), ids=[t[1] for t in htile_registry()])
+def test_forced_htile(n, name, monkeypatch, capfd):
+    """The tiles with component-wise hand-overs, as the tiles above; 40 columns leave the last
+    tile of 16 lines half empty."""
+    test_forced_tile(n, name, monkeypatch)
+    assert f": {name}\n" in capfd.readouterr().err
