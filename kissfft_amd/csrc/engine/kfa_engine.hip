@@ -439,12 +439,12 @@ bool env_flag(const char *name, bool dflt)
 // holds table[r*u*P_s] for r = 1..p-1, padded to a multiple of `pad` entries; then
 // table[P_s*m_s] and table[2*P_s*m_s], padded likewise (the layout of Radices<G, ...>).
 int make_stage_table_raw(const unsigned char *h_tw, int type, long long n, const std::vector<int> &rad,
-                                int pad, int fmt, DevBuf &out)
+                                int pad, int fmt, DevBuf &out, long long m0)
 {
     // fmt 1: a Q15 entry w becomes the word pair (w.r, -w.i), (w.i, w.r) (8 bytes)
     const size_t cb = fmt == 1 ? 8 : cpx_bytes(type);
     std::vector<unsigned char> h;
-    long long m = 1;
+    long long m = m0;
     auto put = [&](long long idx) {
         const unsigned char *src = h_tw + cpx_bytes(type) * (size_t)(idx % n);
         if (fmt == 1) {
@@ -484,7 +484,7 @@ int make_stage_table_raw(const unsigned char *h_tw, int type, long long n, const
     // fixed point: the generic stages' combined entries (Radices::gen_off / GR in
     // kfa_fast.hpp: row u of stage s holds table[q * P * (u + q1 * m) mod n], q1 major)
     if (type != KFA_F32) {
-        m = 1;
+        m = m0;
         for (int p : rad) {
             const bool gen = !(p == 2 || p == 3 || p == 4 || p == 5 || p == 8 || p == 16);
             const long long Pst = n / (p * m);
@@ -755,6 +755,19 @@ static int tile_choice(int n, int inverse, int mode, hipStream_t s, std::shared_
                     break;
                 }
     }
+    // lengths without a built-in tile: compiled at run time (not while the caller's stream
+    // is being captured: that call takes the general kernel, and the choice stays open)
+    const bool real = mode == TILE_RSPLIT || mode == TILE_RMERGE;
+    if (cand.empty() && !real && env_flag("KISSFFT_AMD_FAST", true)) {
+        if (stream_capturing(s)) {
+            out = std::make_shared<const TileChoice>();
+            return 0;
+        }
+        const std::vector<int> rad = float_schedule(n, true);
+        const int tm = mode == TILE_COLS ? 0 : mode == TILE_COLS_TWID ? TM_TWID : TM_ROWS;
+        if (const TileVariant *v = rad.empty() ? nullptr : rtc_tile(KFA_F32, rad, inverse, tm))
+            cand.push_back(std::make_shared<TileChoice>(TileChoice{v, nullptr, nullptr}));
+    }
     const std::vector<unsigned char> tw = float_twiddles(n, inverse, n, 1);
     for (auto &c : cand) {
         if ((rc = make_stage_table_raw(tw.data(), KFA_F32, n, c->v->radices, c->v->tw_pad, 0, c->stw_mem)))
@@ -851,7 +864,7 @@ static int launch_tile(const TileChoice &tc, TileArgs a, hipStream_t s)
     if (tiles > 0x7fffffffLL)
         return fail(-2, "too many lines (%lld) for one launch", a.nlines);
     ++g_launches;
-    return tc.v->launch(a, tiles, s) ? fail(-3, "tile kernel launch failed") : 0;
+    return tile_launch(*tc.v, a, tiles, s) ? fail(-3, "tile kernel launch failed") : 0;
 }
 
 // A fused real pass over `howmany` transforms: a.other / 2 line pairs each, TL / 2 per
@@ -2224,6 +2237,41 @@ int kfa_c2r(const kfa_rplan *pl, const void *in, long long idist, void *out, lon
     return real_common(pl, in, idist, out, odist, howmany, stream, sync, 1);
 }
 
+// The compiled tile kernel for the lines of fixed-point plan P as strided columns, decided
+// once per plan (null: the general kernel).  While the caller's stream is being captured
+// an undecided plan takes the general kernel for that call.
+static int fixed_axis(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoice> &out)
+{
+    std::lock_guard<std::mutex> g(P.mu);
+    out = P.axis;
+    if (P.axis_decided)
+        return 0;
+    if (thread_noalloc())
+        return noalloc_refuse("a tile kernel's tables");
+    if (stream_capturing(s))
+        return 0;
+    if (env_flag("KISSFFT_AMD_FAST", true)) {
+        if (const TileVariant *v = rtc_tile(P.type, P.radix, P.inverse, 0)) {
+            auto tc = std::make_shared<TileChoice>();
+            tc->v = v;
+            if (int rc = make_stage_table_raw(P.h_tw.data(), P.type, P.n, v->radices, v->tw_pad, v->tw_fmt, tc->stw_mem))
+                return rc;
+            tc->d_stw = tc->stw_mem.get();
+            P.axis = tc;
+            if (env_flag("KISSFFT_AMD_VERBOSE", false))
+                fprintf(stderr, "[kissfft_amd] tile n=%d inverse=%d type=%d: %s\n", P.n, P.inverse, P.type, v->name);
+        }
+    }
+    P.axis_decided = true;
+    out = P.axis;
+    return 0;
+}
+
+// Whether a column pass of `values` values over lines of n points is worth a kernel
+// compiled for its length on first use (a fraction of a second): any length from 16 points,
+// as for rows, and shorter ones when there is more than a handful of them.
+static bool axis_compiles(long long n, long long values) { return n >= 16 || values >= (1LL << 16); }
+
 // One axis of an N-D array batch, dims[k] long, between device buffers (in may equal out).
 static int run_axis(DevPlan &P, const void *in, void *out, long long outer, long long inner,
                     hipStream_t s)
@@ -2242,12 +2290,13 @@ static int run_axis(DevPlan &P, const void *in, void *out, long long outer, long
         }
         return 0;
     }
-    if (P.type == KFA_F32) {
+    if (axis_compiles(len, outer * inner * len)) {
         std::shared_ptr<const TileChoice> tc;
-        int rc = tile_choice((int)len, P.inverse, TILE_COLS, s, tc, inner, outer);
+        int rc = P.type == KFA_F32 ? tile_choice((int)len, P.inverse, TILE_COLS, s, tc, inner, outer)
+                                   : fixed_axis(P, s, tc);
         if (rc)
             return rc;
-        if (tc->v) {
+        if (tc && tc->v) {
             TileArgs a{};
             a.in = in;
             a.out = out;

@@ -44,11 +44,12 @@ namespace kfa {
 struct TileArgs;
 struct RealTileArgs;
 
-// Tile-kernel variants (kfa_tile.hpp, kfa_tile_real.hpp): float, one length, direction
-// and HBM mapping.
+// Tile-kernel variants (kfa_tile.hpp, kfa_tile_real.hpp): one length, direction and HBM
+// mapping.  Built in: float; compiled at run time (kfa_rtc.hip): any scalar kind.
 enum { TILE_COLS = 0, TILE_COLS_TWID = 1, TILE_ROWS_TO_COLS = 2, TILE_RSPLIT = 3, TILE_RMERGE = 4 };
 
 struct TileVariant {
+    int type = 0;  // KFA_F32 / KFA_Q15 / KFA_Q31
     int n;
     int inverse;
     int mode;     // TILE_COLS: column load / column store (N-D axes)
@@ -59,14 +60,18 @@ struct TileVariant {
     int T, TL;    // threads per line, lines per workgroup
     std::vector<int> radices;
     int tw_pad;
+    int tw_fmt = 0;  // see FastVariant
     int tw_len;
     size_t lds;   // dynamic LDS bytes
     const char *name;
+    const void *rtc = nullptr;  // runtime-compiled variant: launched through it
     int (*launch)(const TileArgs &, long long blocks, hipStream_t);            // modes 0-2
     int (*launch_real)(const RealTileArgs &, long long blocks, hipStream_t);  // modes 3-4
 };
 
 const std::vector<TileVariant> &tile_registry();
+// launches variant v (modes 0-2, built in or runtime-compiled) on `blocks` workgroups
+int tile_launch(const TileVariant &v, const TileArgs &a, long long blocks, hipStream_t s);
 
 }  // namespace kfa
 

@@ -79,6 +79,9 @@ struct DevPlan {
     std::shared_ptr<const RealFusedPlan> rfused[2];  // per direction
     bool blue_decided = false;
     std::shared_ptr<const BlueChoice> blue;
+    // fixed point: the line as strided columns (N-D axes; null: the general kernel)
+    bool axis_decided = false;
+    std::shared_ptr<const TileChoice> axis;
 };
 
 struct RealTables {
@@ -142,6 +145,12 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
 
 // runtime-compiled variants of a plan's length and kind (kfa_rtc.hip), when none is built in
 int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> &out);
+// the runtime-compiled tile kernel of schedule `radices` (kfa_tile.hpp; tm: TM_* mapping
+// bits), or null: radix outside 2-5, 7, 11, 13 (float also 8, 16), no shape without
+// scratch, or the runtime compiler off
+const TileVariant *rtc_tile(int type, const std::vector<int> &radices, int inverse, int tm);
+// the float schedule of length n (empty: a factor above 13)
+std::vector<int> float_schedule(int n, bool even = false);
 // the persisted table of tuned choices (kfa_rtc.hip): key of a decision, lookup, store
 std::string tuned_key(const DevPlan &P, int kind, long long tune_lines);
 bool tuned_lookup(const std::string &key, std::string &name);
@@ -189,8 +198,9 @@ bool env_flag(const char *name, bool dflt);
 // float twiddles exp(-+2*pi*i*(j*step mod n)/n), j < count, FP64 rounded once (8 bytes each)
 std::vector<unsigned char> float_twiddles(long long n, int inverse, long long count, long long step);
 // per-stage twiddle table of schedule `rad` (the fast kernels' layout) from a full table
+// (m0: product of the radices executed before rad's first, for a part of a schedule)
 int make_stage_table_raw(const unsigned char *h_tw, int type, long long n, const std::vector<int> &rad, int pad,
-                         int fmt, DevBuf &out);
+                         int fmt, DevBuf &out, long long m0 = 1);
 
 // whether a float plan runs Bluestein's kernel (its tables built on return; the caller may
 // hold them in `keep`)

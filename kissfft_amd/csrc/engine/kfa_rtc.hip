@@ -18,6 +18,11 @@
 //     the options and the device architecture; KISSFFT_AMD_RTC=0 turns the path off;
 //   * a kernel that would use scratch memory (spilled registers) is not used;
 //   * lines shorter than 16 points (KISSFFT_AMD_RTC_MIN) keep the general kernel.
+// The tile kernel k_tile (kfa_tile.hpp) is compiled the same way for the strided lines of
+// N-D axes without a built-in tile, all three scalar kinds, in one shape chosen by rule
+// (tile_shapes), so an axis costs one compilation per direction.  Against the general line
+// kernel: Q15 64x96x120 x16 500 -> 63 us, float 24x25x128 x93 252 -> 53 us, Q31 real
+// 45x48x120 x61 there and back 722 -> 193 us.
 // The tuned choice of every (device, scalar kind, transform kind, length, direction,
 // timing batch) is kept in a table on disk beside the code objects (tuned.txt, or
 // KISSFFT_AMD_TUNE_TABLE; "0" turns it off), so later processes skip the timing.
@@ -45,6 +50,7 @@
 #include "../kfa_engine.h"
 #include "kfa_fast.hpp"
 #include "kfa_internal.hpp"
+#include "kfa_tile.hpp"
 
 // embedded header sources (generated at build time)
 extern "C" const int kfa_rtc_nheaders;
@@ -153,7 +159,7 @@ std::map<std::string, std::unique_ptr<RtcVariant>> g_variants;  // by name expre
 
 // Compiles (or reads from the disk cache) the kernel `expr` of source `src`; 0 on success.
 int build_kernel(const std::string &expr, const std::string &arch, std::string &code, std::string &lowered,
-                 const std::string &src = "#include \"kfa_fast.hpp\"\n")
+                 const std::string &src)
 {
     const std::vector<std::string> opts = {"--offload-arch=" + arch, "-O3", "-std=c++17", "-Xclang",
                                            "-target-feature", "-Xclang", "-packed-fp32-ops"};
@@ -253,42 +259,6 @@ const char *arith_name(int type, int kind)
     return kind == FK_C2C ? "kfa::Q15P" : "kfa::Q15";
 }
 
-// float: 16s, then one 8 / 4 / 2 for the rest of the power of two, then 5s, then 3s,
-// then the generic odd radices 7, 11, 13 (kfa_fast.hpp's Dft<P>); empty for other factors
-std::vector<int> float_schedule(int n)
-{
-    int a = 0, b = 0, c = 0;
-    while (n % 2 == 0) {
-        n /= 2;
-        ++a;
-    }
-    while (n % 3 == 0) {
-        n /= 3;
-        ++b;
-    }
-    while (n % 5 == 0) {
-        n /= 5;
-        ++c;
-    }
-    std::vector<int> g;
-    for (int p : {7, 11, 13})
-        while (n % p == 0) {
-            n /= p;
-            g.push_back(p);
-        }
-    std::vector<int> r;
-    if (n != 1)
-        return r;
-    for (; a >= 4; a -= 4)
-        r.push_back(16);
-    if (a)
-        r.push_back(1 << a);
-    r.insert(r.end(), c, 5);
-    r.insert(r.end(), b, 3);
-    r.insert(r.end(), g.begin(), g.end());
-    return r;
-}
-
 std::map<std::string, std::string> g_tuned;  // tuned-choice table: key -> variant name
 bool g_tuned_loaded = false;
 
@@ -318,7 +288,225 @@ void tuned_load()
     }
 }
 
+// Builds and loads kernel `expr` of source `src`; 0 when it runs without scratch memory.
+int load_kernel(const std::string &expr, const std::string &arch, const std::string &src, hipModule_t *mod,
+                hipFunction_t *fn)
+{
+    std::string code, lowered;
+    int scratch = 0;
+    *mod = nullptr;
+    if (build_kernel(expr, arch, code, lowered, src) == 0 && hipModuleLoadData(mod, code.data()) == hipSuccess &&
+        hipModuleGetFunction(fn, *mod, lowered.c_str()) == hipSuccess &&
+        hipFuncGetAttribute(&scratch, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, *fn) == hipSuccess && scratch == 0)
+        return 0;
+    (void)hipGetLastError();
+    if (*mod)
+        (void)hipModuleUnload(*mod);
+    *mod = nullptr;
+    if (env_flag("KISSFFT_AMD_VERBOSE", false))
+        fprintf(stderr, "[kissfft_amd] runtime kernel %s unusable (scratch %d): %s\n", expr.c_str(), scratch,
+                kfa_last_error());
+    return -3;
+}
+
+// One runtime-compiled tile: its variant and its loaded kernel.
+struct RtcTile {
+    TileVariant v;
+    std::string name;
+    hipModule_t mod = nullptr;
+    hipFunction_t fn = nullptr;
+};
+
+std::map<std::string, std::unique_ptr<RtcTile>> g_tiles;  // by name expression, arch, device
+
+// Shapes of a tile of n-point lines, cb bytes a value, preferred first.
+struct TileShape {
+    int T, TL;
+    bool half;
+};
+
+// Threads per line: the count that leaves the fewest idle butterfly slots over the stages
+// (T * sum of ceil(n / p / T) * p), with at most `most` values per thread in any stage.
+int tile_threads(int n, const std::vector<int> &rad, int TL, int most)
+{
+    int best = 0;
+    double best_cost = 0;
+    for (int T = 1; T <= n && T * TL <= 1024; ++T) {
+        long long slots = 0;
+        int widest = 0;
+        for (int p : rad) {
+            const int el = (n / p + T - 1) / T * p;
+            slots += el;
+            widest = std::max(widest, el);
+        }
+        if (widest > most && widest > *std::max_element(rad.begin(), rad.end()))
+            continue;
+        // whole waves; fewer values per thread cost an address each
+        const int waves = (T * TL + 63) / 64;
+        const double cost = (double)slots * waves * 64 / TL * (widest < 8 ? 1.1 : 1.0);
+        if (!best || cost < 0.995 * best_cost) {
+            best = T;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+// Rows of a full 128-byte line wherever LDS holds two such workgroups per CU: whole values,
+// else one component at a time (8-byte values only: Q15 moves packed words), else rows half
+// as long, and so on.  Short lines take more lines, up to 256 threads.
+std::vector<TileShape> tile_shapes(int n, const std::vector<int> &rad, int type, bool rows)
+{
+    const int cb = type == KFA_Q15 ? 4 : 8;
+    const size_t room = 78 * 1024;
+    std::vector<TileShape> out;
+    auto fits = [&](int TL, int slot) {
+        const bool padded = !rows && slot == 8 && TL * slot < 128 && rad.back() % 2 == 0;  // TilePos
+        return (size_t)(padded ? n + n / rad.back() : n) * (TL + (rows ? 1 : 0)) * slot <= room;
+    };
+    for (int TL = 128 / cb; TL >= 1 && out.size() < 3; TL /= 2)
+        for (int half = 0; half < (cb == 8 && rad.size() > 1 ? 2 : 1); ++half) {
+            if (!fits(TL, half ? 4 : cb))
+                continue;
+            // half: two workgroups of 1024 threads have 64 registers, 16 values a thread (Q31,
+            // whose products take register pairs, spills above 10)
+            int tl = TL, T = tile_threads(n, rad, tl, half && type == KFA_Q31 ? 10 : 16);
+            if (!T && !half)
+                T = tile_threads(n, rad, tl, 32);
+            if (!T)
+                continue;
+            while (!half && T * tl < 256 && (size_t)n * (2 * tl + 1) * cb <= 40 * 1024)
+                tl *= 2;
+            out.push_back({tl == TL ? T : std::max(1, tile_threads(n, rad, tl, 16)), tl, half != 0});
+            if (!half)
+                break;
+        }
+    return out;
+}
+
 }  // namespace
+
+// float: 16s, then one 8 / 4 / 2 for the rest of the power of two, then 5s, then 3s,
+// then the generic odd radices 7, 11, 13 (kfa_fast.hpp's Dft<P>); empty for other factors.
+// even: 8 and 4 in the place of a 16 and a 2 (a tile's threads hold all of a stage's values
+// at once: a stage of radix 2 moves the tile through LDS for little work)
+std::vector<int> float_schedule(int n, bool even)
+{
+    int a = 0, b = 0, c = 0;
+    while (n % 2 == 0) {
+        n /= 2;
+        ++a;
+    }
+    while (n % 3 == 0) {
+        n /= 3;
+        ++b;
+    }
+    while (n % 5 == 0) {
+        n /= 5;
+        ++c;
+    }
+    std::vector<int> g;
+    for (int p : {7, 11, 13})
+        while (n % p == 0) {
+            n /= p;
+            g.push_back(p);
+        }
+    std::vector<int> r;
+    if (n != 1)
+        return r;
+    for (; a >= 4 && !(even && a == 5); a -= 4)
+        r.push_back(16);
+    if (a == 5) {
+        r.push_back(8);
+        a = 2;
+    }
+    if (a)
+        r.push_back(1 << a);
+    r.insert(r.end(), c, 5);
+    r.insert(r.end(), b, 3);
+    r.insert(r.end(), g.begin(), g.end());
+    return r;
+}
+
+int tile_launch(const TileVariant &v, const TileArgs &a, long long blocks, hipStream_t s)
+{
+    if (!v.rtc)
+        return v.launch(a, blocks, s);
+    if (blocks <= 0)
+        return 0;
+    TileArgs copy = a;
+    void *params[] = {&copy};
+    return hipModuleLaunchKernel(static_cast<const RtcTile *>(v.rtc)->fn, (unsigned)blocks, 1, 1, v.T * v.TL, 1, 1, 0,
+                                 s, params, nullptr) == hipSuccess
+               ? 0
+               : -3;
+}
+
+const TileVariant *rtc_tile(int type, const std::vector<int> &radices, int inverse, int tm)
+{
+    if (!env_flag("KISSFFT_AMD_RTC", true) || radices.empty() || ((tm & TM_ROWS) && radices.size() < 2))
+        return nullptr;
+    long long n = 1;
+    bool generic = false;
+    for (int p : radices) {
+        if (!(p == 2 || p == 3 || p == 4 || p == 5 || p == 7 || p == 11 || p == 13 ||
+              (type == KFA_F32 && (p == 8 || p == 16))))
+            return nullptr;
+        generic |= p == 7 || p == 11 || p == 13;
+        n *= p;
+        if (n > 16384)
+            return nullptr;
+    }
+    const std::string arch = arch_name();
+    std::lock_guard<std::mutex> g(g_rtc_mu);
+    // Q15: packed words; with a generic radix the unpacked form when the packed one spills
+    for (int packed = type == KFA_Q15; packed >= 0; packed -= (type == KFA_Q15 && generic) ? 1 : 2)
+        for (const TileShape &sh : tile_shapes((int)n, radices, type, (tm & TM_ROWS) != 0)) {
+            const int mode = tm | (sh.half ? TM_HALF : 0);
+            const int pad = (type == KFA_Q15 && !packed) ? 4 : 2;  // 16-byte stage-table rows
+            std::string rs;
+            for (int p : radices)
+                rs += ", " + std::to_string(p);
+            const char *arith = type == KFA_F32 ? "kfa::F32" : type == KFA_Q31 ? "kfa::Q31"
+                                : packed ? "kfa::Q15P" : "kfa::Q15";
+            const std::string expr = std::string("&kfa::k_tile<") + arith + ", " + (inverse ? "true" : "false") + ", " +
+                                     std::to_string(sh.T) + ", " + std::to_string(sh.TL) + ", " +
+                                     std::to_string(mode) + ", kfa::Radices<" + std::to_string(pad) + rs + ">>";
+            const std::string key = expr + "|" + arch + "|" + std::to_string(current_dev());
+            auto it = g_tiles.find(key);
+            if (it == g_tiles.end()) {
+                auto rt = std::make_unique<RtcTile>();
+                if (load_kernel(expr, arch, "#include \"kfa_tile.hpp\"\n", &rt->mod, &rt->fn) == 0) {
+                    char nm[160];
+                    snprintf(nm, sizeof nm, "rtc_tile%lld_t%dx%d%s%s", n, sh.T, sh.TL, sh.half ? "h" : "",
+                             type == KFA_Q15 && !packed ? "_u" : "");
+                    rt->name = nm;
+                    TileVariant &v = rt->v;
+                    v.type = type;
+                    v.n = (int)n;
+                    v.inverse = inverse;
+                    v.mode = -1;  // (the caller's mapping is in the kernel)
+                    v.T = sh.T;
+                    v.TL = sh.TL;
+                    v.radices = radices;
+                    v.tw_pad = pad;
+                    v.tw_fmt = packed ? 1 : 0;
+                    v.tw_len = 1;
+                    v.lds = 0;
+                    v.name = rt->name.c_str();
+                    v.rtc = rt.get();
+                    v.launch = nullptr;
+                    v.launch_real = nullptr;
+                } else {
+                    rt.reset();  // remembered as unusable
+                }
+                it = g_tiles.emplace(key, std::move(rt)).first;
+            }
+            if (it->second)
+                return &it->second->v;
+        }
+    return nullptr;
+}
 
 std::string tuned_key(const DevPlan &P, int kind, long long tune_lines)
 {
@@ -418,13 +606,7 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
             auto it = g_variants.find(key);
             if (it == g_variants.end()) {
                 auto rv = std::make_unique<RtcVariant>();
-                std::string code, lowered;
-                int rc = build_kernel(expr, arch, code, lowered);
-                int scratch = 0;
-                if (rc == 0 && hipModuleLoadData(&rv->mod, code.data()) == hipSuccess &&
-                    hipModuleGetFunction(&rv->fn, rv->mod, lowered.c_str()) == hipSuccess &&
-                    hipFuncGetAttribute(&scratch, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, rv->fn) == hipSuccess &&
-                    scratch == 0) {
+                if (load_kernel(expr, arch, "#include \"kfa_fast.hpp\"\n", &rv->mod, &rv->fn) == 0) {
                     char nm[160];
                     // (Q15 complex lines in the unpacked form: suffix _u)
                     snprintf(nm, sizeof nm, "rtc_%s%d_t%dx%d%s",
@@ -449,13 +631,7 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
                     v.arith = arith;
                     v.db = v.fuse = false;
                 } else {
-                    (void)hipGetLastError();
-                    if (rv->mod)
-                        (void)hipModuleUnload(rv->mod);
                     rv.reset();  // remembered as unusable
-                    if (env_flag("KISSFFT_AMD_VERBOSE", false))
-                        fprintf(stderr, "[kissfft_amd] runtime kernel %s unusable (scratch %d): %s\n",
-                                expr.c_str(), scratch, kfa_last_error());
                 }
                 it = g_variants.emplace(key, std::move(rv)).first;
             }
@@ -529,23 +705,10 @@ int rtc_fused(const std::vector<FusedMember> &m, int NT, hipFunction_t *fn)
     const std::string key = src + "|" + arch + "|" + std::to_string(current_dev());
     auto it = fused.find(key);
     if (it == fused.end()) {
-        std::string code, lowered;
         hipModule_t mod = nullptr;
         hipFunction_t f = nullptr;
-        int scratch = 0;
-        int rc = build_kernel(expr, arch, code, lowered, src);
-        if (rc == 0 && hipModuleLoadData(&mod, code.data()) == hipSuccess &&
-            hipModuleGetFunction(&f, mod, lowered.c_str()) == hipSuccess &&
-            hipFuncGetAttribute(&scratch, HIP_FUNC_ATTRIBUTE_LOCAL_SIZE_BYTES, f) == hipSuccess && scratch == 0) {
-            // kept
-        } else {
-            (void)hipGetLastError();
-            if (mod)
-                (void)hipModuleUnload(mod);
+        if (load_kernel(expr, arch, src, &mod, &f))
             f = nullptr;  // remembered as unusable
-            if (env_flag("KISSFFT_AMD_VERBOSE", false))
-                fprintf(stderr, "[kissfft_amd] fused kernel unusable (scratch %d): %s\n", scratch, kfa_last_error());
-        }
         it = fused.emplace(key, f).first;
     }
     if (!it->second)
