@@ -539,7 +539,7 @@ struct TileCache {
     std::mutex mu;
     // dev, n, inv, mode, inner, small (see tile_choice)
     std::map<std::tuple<int, int, int, int, long long, int>, std::shared_ptr<const TileChoice>> choice;
-    std::map<std::tuple<int, long long, int>, BufPair> fs;                                // dev, N, inv -> hi, lo
+    std::map<std::tuple<int, long long, int, int>, BufPair> fs;                           // dev, N, inv, wide -> hi, lo
     std::map<std::tuple<int, long long, int, int>, BufPair> rs;                           // dev, nc, n, inv
     // dev, A, B, inv, slab, small (see plane_choice)
     std::map<std::tuple<int, int, int, int, int, int>, std::shared_ptr<const PlaneChoice>> plane;
@@ -677,13 +677,13 @@ static size_t tune_tiles(int n, int mode, const std::vector<std::shared_ptr<Tile
         if (geo)
             outer = std::min(outer, outer_max);
         const size_t bytes = 8 * (size_t)(n * C + 1) * (size_t)outer;
-        const size_t hib = 8 * (size_t)((long long)n * C / 1024 + 1);
+        const size_t hib = 16 * (size_t)((long long)n * C / 1024 + 1);
         const size_t rtb = 8 * (size_t)(n + C);
-        TuneBuf bin(bytes, ts), bout(bytes, ts), whi(hib, ts), wlo(8 * 1024, ts), rtw(rtb, ts);
+        TuneBuf bin(bytes, ts), bout(bytes, ts), whi(hib, ts), wlo(16 * 1024, ts), rtw(rtb, ts);
         if (!bin.p || !bout.p || !whi.p || !wlo.p || !rtw.p)
             continue;
         if (fill_tune(bin.p, bytes, KFA_F32, ts) || hipMemsetAsync(whi.p, 0x3c, hib, ts) != hipSuccess ||
-            hipMemsetAsync(wlo.p, 0x3c, 8 * 1024, ts) != hipSuccess || hipMemsetAsync(rtw.p, 0x3c, rtb, ts) != hipSuccess)
+            hipMemsetAsync(wlo.p, 0x3c, 16 * 1024, ts) != hipSuccess || hipMemsetAsync(rtw.p, 0x3c, rtb, ts) != hipSuccess)
             return 0;
         TileArgs a{};
         a.in = bin.p;
@@ -785,8 +785,22 @@ static int tile_choice(int n, int inverse, int mode, hipStream_t s, std::shared_
     return 0;
 }
 
-// W^(q*1024) for q <= N/1024 and W^r for r < 1024, W = exp(-+2*pi*i/N)
-static int fourstep_twiddles(long long N, int inverse, BufPair &out)
+// The tables' values in FP64.
+static std::vector<double> double_twiddles(long long n, int inverse, long long count, long long step)
+{
+    const double pi = 3.14159265358979323846264338327950288;
+    std::vector<double> h(2 * (size_t)count);
+    for (long long i = 0; i < count; ++i) {
+        const double phase = (inverse ? 2 : -2) * pi * (double)(i * step % n) / (double)n;
+        h[2 * i] = cos(phase);
+        h[2 * i + 1] = sin(phase);
+    }
+    return h;
+}
+
+// W^(q*1024) for q <= N/1024 and W^r for r < 1024, W = exp(-+2*pi*i/N): FP64 for the
+// complex passes (wide), float for the fused real merge.
+static int fourstep_twiddles(long long N, int inverse, bool wide, BufPair &out)
 {
     int dev;
     int rc = current_device(&dev);
@@ -794,15 +808,22 @@ static int fourstep_twiddles(long long N, int inverse, BufPair &out)
         return rc;
     auto &C = tile_cache();
     std::lock_guard<std::mutex> g(C.mu);
-    const auto key = std::make_tuple(dev, N, inverse);
+    const auto key = std::make_tuple(dev, N, inverse, (int)wide);
     auto it = C.fs.find(key);
     if (it == C.fs.end()) {
-        const std::vector<unsigned char> h = float_twiddles(N, inverse, N / 1024 + 1, 1024);
-        const std::vector<unsigned char> l = float_twiddles(N, inverse, 1024, 1);
         BufPair bp;
         RelaxCapture relax;
-        if ((rc = dev_upload(h.data(), h.size(), bp.first)) || (rc = dev_upload(l.data(), l.size(), bp.second)))
-            return rc;
+        if (wide) {
+            const std::vector<double> h = double_twiddles(N, inverse, N / 1024 + 1, 1024);
+            const std::vector<double> l = double_twiddles(N, inverse, 1024, 1);
+            if ((rc = dev_upload(h.data(), h.size() * 8, bp.first)) || (rc = dev_upload(l.data(), l.size() * 8, bp.second)))
+                return rc;
+        } else {
+            const std::vector<unsigned char> h = float_twiddles(N, inverse, N / 1024 + 1, 1024);
+            const std::vector<unsigned char> l = float_twiddles(N, inverse, 1024, 1);
+            if ((rc = dev_upload(h.data(), h.size(), bp.first)) || (rc = dev_upload(l.data(), l.size(), bp.second)))
+                return rc;
+        }
         it = C.fs.emplace(key, bp).first;
     }
     out = it->second;
@@ -1119,8 +1140,12 @@ static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long 
     return 0;
 }
 
-// Float four-step (Bailey) for n = N1*N2 with both halves registered as tile variants,
-// decided once per plan: pass 1 transforms the N1 columns (length N2, stride N1) and
+// Longest half of a four-step split that a tile is compiled for: 8 of its lines (rows of 64
+// bytes) fit a workgroup.
+constexpr long long kTileLongest = 2048;
+
+// Float four-step (Bailey) for n = N1*N2 with both halves tile lengths (built in, or
+// compiled at run time), decided once per plan: pass 1 transforms the N1 columns (length N2, stride N1) and
 // applies W_N^(n1*k2); pass 2 transforms the N2 rows (length N1) and writes them as
 // columns (k = k2 + N2*k1).  P.bailey stays null when no such split exists.
 static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPlan> &out)
@@ -1138,7 +1163,10 @@ static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPl
     if (thread_noalloc())
         return noalloc_refuse("the four-step plan");
     const long long n = P.n;
-    long long best1 = 0;
+    // the most balanced split, among the built-in lengths and among those that a tile can be
+    // compiled for; a built-in one is taken unless its longer half is over 1.5 times the other's
+    auto score = [&](long long a) { return a > n / a ? a : n / a; };
+    long long best1 = 0, made1 = 0;
     for (const TileVariant &v : tile_registry()) {
         if (v.mode != TILE_ROWS_TO_COLS || v.inverse != P.inverse || n % v.n != 0)
             continue;
@@ -1146,12 +1174,17 @@ static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPl
         bool have2 = false;
         for (const TileVariant &w : tile_registry())
             have2 |= w.mode == TILE_COLS_TWID && w.inverse == P.inverse && w.n == N2;
-        if (!have2)
-            continue;
-        // most balanced split
-        auto score = [&](long long a) { return a > n / a ? a : n / a; };
-        if (best1 == 0 || score(N1) < score(best1))
+        if (have2 && (best1 == 0 || score(N1) < score(best1)))
             best1 = N1;
+    }
+    for (long long N1 = 17; N1 <= kTileLongest && N1 <= n / 16; ++N1)  // (rows: two stages or more)
+        if (n % N1 == 0 && n / N1 <= kTileLongest && (made1 == 0 || score(N1) < score(made1)) &&
+            float_schedule((int)N1, true).size() > 1 && !float_schedule((int)(n / N1), true).empty())
+            made1 = N1;
+    if (made1 && (best1 == 0 || score(best1) > 1.5 * score(made1))) {
+        if (stream_capturing(s))
+            return 0;  // nothing is compiled now: the choice stays open
+        best1 = made1;
     }
     if (best1) {
         auto bp = std::make_shared<BaileyPlan>();
@@ -1161,7 +1194,7 @@ static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPl
         int rc;
         if ((rc = tile_choice((int)bp->N1, P.inverse, TILE_ROWS_TO_COLS, s, bp->c2)) ||
             (rc = tile_choice((int)bp->N2, P.inverse, TILE_COLS_TWID, s, bp->c1)) ||
-            (rc = fourstep_twiddles(n, P.inverse, tw)))
+            (rc = fourstep_twiddles(n, P.inverse, true, tw)))
             return rc;
         bp->tw_hi = tw.first;
         bp->tw_lo = tw.second;
@@ -1548,6 +1581,89 @@ size_t multipass_bytes_per_transform(DevPlan &P, int fk)
     return cb * (size_t)(P.n + 16) + 256 + c2c;
 }
 
+// The tile kernel compiled for the stages `rad` of fixed-point plan P (mapping tm), with its
+// stage table; m0: product of the radices of the stages before them.  Null: none.
+static int fixed_tile(const DevPlan &P, const std::vector<int> &rad, long long m0, int tm,
+                      std::shared_ptr<const TileChoice> &out)
+{
+    out = nullptr;
+    const TileVariant *v = rtc_tile(P.type, rad, P.inverse, tm);
+    if (!v)
+        return 0;
+    auto tc = std::make_shared<TileChoice>();
+    tc->v = v;
+    if (int rc = make_stage_table_raw(P.h_tw.data(), P.type, P.n, rad, v->tw_pad, v->tw_fmt, tc->stw_mem, m0))
+        return rc;
+    tc->d_stw = tc->stw_mem.get();
+    if (env_flag("KISSFFT_AMD_VERBOSE", false))
+        fprintf(stderr, "[kissfft_amd] tile n=%d of %d inverse=%d type=%d: %s\n", v->n, P.n, P.inverse, P.type, v->name);
+    out = tc;
+    return 0;
+}
+
+// The tile kernel for the lines of fixed-point plan P as strided columns, decided once per
+// plan (null: the general kernel).  While the caller's stream is being captured an
+// undecided plan takes the general kernel for that call.
+static int fixed_axis(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoice> &out)
+{
+    std::lock_guard<std::mutex> g(P.mu);
+    out = P.axis;
+    if (P.axis_decided)
+        return 0;
+    if (thread_noalloc())
+        return noalloc_refuse("a tile kernel's tables");
+    if (stream_capturing(s))
+        return 0;
+    if (env_flag("KISSFFT_AMD_FAST", true))
+        if (int rc = fixed_tile(P, P.radix, 1, 0, P.axis))
+            return rc;
+    P.axis_decided = true;
+    out = P.axis;
+    return 0;
+}
+
+// The tile kernels of a multi-pass fixed-point plan's two passes, decided once per plan (as
+// fixed_axis; null: the general kernel).  The second pass reads stage tables of the full
+// length, about 1.3 entries a point, so very long lines keep the general kernel, which
+// reads the one n-point table.
+constexpr int kSplitTableLongest = 1 << 23;
+
+static int fixed_split(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoice> &t1,
+                       std::shared_ptr<const TileChoice> &t2)
+{
+    std::lock_guard<std::mutex> g(P.mu);
+    if (!P.split_decided) {
+        t1 = t2 = nullptr;
+        if (P.type != KFA_F32 && !P.single && !P.bigp && P.n <= kSplitTableLongest &&
+            env_flag("KISSFFT_AMD_FAST", true)) {
+            if (thread_noalloc())
+                return noalloc_refuse("the two-pass plan");
+            if (stream_capturing(s))
+                return 0;
+            std::vector<int> r1, r2;
+            long long m = 1;
+            for (int p : P.radix) {
+                (m < P.L1 ? r1 : r2).push_back(p);
+                m *= p;
+            }
+            std::shared_ptr<const TileChoice> a, b;
+            if (int rc = fixed_tile(P, r1, 1, 0, a))
+                return rc;
+            if (a)
+                if (int rc = fixed_tile(P, r2, P.L1, TM_ROWS | TM_REF, b))
+                    return rc;
+            if (a && b) {
+                P.split1 = a;
+                P.split2 = b;
+            }
+        }
+        P.split_decided = true;
+    }
+    t1 = P.split1;
+    t2 = P.split2;
+    return 0;
+}
+
 // Runs `howmany` complex transforms of plan P between two device buffers.
 // in: element t of item b at in + (b*idist + t*istride); out: out + (b*odist + t*ostride).
 int run_c2c(DevPlan &P, const void *in, long long istride, long long idist, void *out,
@@ -1673,6 +1789,37 @@ int run_c2c(DevPlan &P, const void *in, long long istride, long long idist, void
     if (int rc = tmp.get(cpx_bytes(P.type) * (size_t)n * (size_t)howmany, s))
         return rc;
     int rc;
+    std::shared_ptr<const TileChoice> t1, t2;
+    if ((rc = fixed_split(P, s, t1, t2)))
+        return rc;
+    if (t1 && t2) {
+        TileArgs a{};
+        a.in = in;
+        a.out = tmp.p;
+        a.nlines = howmany * P.Q;
+        a.nlo = P.Q;
+        a.in_hi = idist;
+        a.in_lo = istride;
+        a.in_el = (long long)P.Q * istride;
+        a.out_hi = n;
+        a.out_lo = 1;
+        a.out_el = P.Q;
+        if ((rc = launch_tile(*t1, a, s)))
+            return rc;
+        TileArgs b{};
+        b.in = tmp.p;
+        b.out = out;
+        b.nlines = howmany * P.L1;
+        b.nlo = P.L1;
+        b.in_hi = n;
+        b.in_lo = P.Q;
+        b.in_el = 1;
+        b.out_hi = odist;
+        b.out_lo = ostride;
+        b.out_el = (long long)P.L1 * ostride;
+        b.l1 = P.L1;
+        return launch_tile(*t2, b, s);
+    }
     if (P.bigp) {
         d.out = tmp.p;
         d.out_hi = n;
@@ -1780,7 +1927,7 @@ static int real_fused_plan(DevPlan &H, int inverse, hipStream_t s, std::shared_p
         int rc;
         if ((rc = tile_choice((int)bestf, inverse, fused_mode, s, rp->cf)) ||
             (rc = tile_choice((int)rp->other, inverse, plain_mode, s, rp->cp)) ||
-            (rc = fourstep_twiddles(nc, inverse, fs)) || (rc = real_split_twiddles(nc, (int)bestf, inverse, rs)))
+            (rc = fourstep_twiddles(nc, inverse, !inverse, fs)) || (rc = real_split_twiddles(nc, (int)bestf, inverse, rs)))
             return rc;
         rp->tw_hi = fs.first;
         rp->tw_lo = fs.second;
@@ -1870,7 +2017,10 @@ int prepare_multipass(DevPlan &P, int fk, hipStream_t s)
         return 0;
     std::shared_ptr<const BaileyPlan> bp;
     std::shared_ptr<const RealFusedPlan> fp;
+    std::shared_ptr<const TileChoice> t1, t2;
     int rc = bailey_plan(P, s, bp);
+    if (rc == 0)
+        rc = fixed_split(P, s, t1, t2);
     if (rc == 0 && fk != FK_C2C)
         rc = real_fused_plan(P, fk == FK_C2R, s, fp);
     return rc;
@@ -2235,36 +2385,6 @@ int kfa_c2r(const kfa_rplan *pl, const void *in, long long idist, void *out, lon
             long long howmany, void *stream, int sync)
 {
     return real_common(pl, in, idist, out, odist, howmany, stream, sync, 1);
-}
-
-// The compiled tile kernel for the lines of fixed-point plan P as strided columns, decided
-// once per plan (null: the general kernel).  While the caller's stream is being captured
-// an undecided plan takes the general kernel for that call.
-static int fixed_axis(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoice> &out)
-{
-    std::lock_guard<std::mutex> g(P.mu);
-    out = P.axis;
-    if (P.axis_decided)
-        return 0;
-    if (thread_noalloc())
-        return noalloc_refuse("a tile kernel's tables");
-    if (stream_capturing(s))
-        return 0;
-    if (env_flag("KISSFFT_AMD_FAST", true)) {
-        if (const TileVariant *v = rtc_tile(P.type, P.radix, P.inverse, 0)) {
-            auto tc = std::make_shared<TileChoice>();
-            tc->v = v;
-            if (int rc = make_stage_table_raw(P.h_tw.data(), P.type, P.n, v->radices, v->tw_pad, v->tw_fmt, tc->stw_mem))
-                return rc;
-            tc->d_stw = tc->stw_mem.get();
-            P.axis = tc;
-            if (env_flag("KISSFFT_AMD_VERBOSE", false))
-                fprintf(stderr, "[kissfft_amd] tile n=%d inverse=%d type=%d: %s\n", P.n, P.inverse, P.type, v->name);
-        }
-    }
-    P.axis_decided = true;
-    out = P.axis;
-    return 0;
 }
 
 // Whether a column pass of `values` values over lines of n points is worth a kernel

@@ -82,6 +82,9 @@ struct DevPlan {
     // fixed point: the line as strided columns (N-D axes; null: the general kernel)
     bool axis_decided = false;
     std::shared_ptr<const TileChoice> axis;
+    // fixed point, multi-pass: the two passes of the reference-order split (both or neither)
+    bool split_decided = false;
+    std::shared_ptr<const TileChoice> split1, split2;
 };
 
 struct RealTables {
@@ -149,8 +152,8 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
 // bits), or null: radix outside 2-5, 7, 11, 13 (float also 8, 16), no shape without
 // scratch, or the runtime compiler off
 const TileVariant *rtc_tile(int type, const std::vector<int> &radices, int inverse, int tm);
-// the float schedule of length n (empty: a factor above 13)
-std::vector<int> float_schedule(int n, bool even = false);
+// the float schedule of length n (empty: a factor above 13), for a row or a tile kernel
+std::vector<int> float_schedule(int n, bool tile = false);
 // the persisted table of tuned choices (kfa_rtc.hip): key of a decision, lookup, store
 std::string tuned_key(const DevPlan &P, int kind, long long tune_lines);
 bool tuned_lookup(const std::string &key, std::string &name);

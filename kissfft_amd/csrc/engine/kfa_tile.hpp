@@ -20,9 +20,11 @@
 // the twiddle step between the two passes of the four-step split (Bailey, "FFTs in
 // external or hierarchical memory", 1990):  with n = n1 + N1*n2 and k = k2 + N2*k1,
 //   X[k2 + N2*k1] = sum_n1 W_N1^(n1*k1) * W_N^(n1*k2) * sum_n2 x[n1 + N1*n2] W_N2^(n2*k2).
-// W^a is read as hi[a >> 10] * lo[a & 1023] from two small tables (computed in FP64,
-// rounded once); a thread's outputs share one such product and a per-line table of the
-// steps between them in LDS.  The float path only.
+// W^a is hi[a >> 10] * lo[a & 1023] from two small FP64 tables; a thread's outputs share one
+// such product and a per-line table of the steps between them in LDS.  The factors and
+// the products with the values are FP64, rounded once per output: in float their roundings
+// made the split less exact than a single schedule (c2c 10^6 1.80e-7 rel-L2 against 1.74e-7).
+// The float path only.
 //
 // REF is the second pass of a fixed-point line longer than one LDS line, which keeps the
 // reference's own stage order: column u of a stage is column lo + L1*u of the full
@@ -38,8 +40,8 @@ struct TileArgs {
     const void *in;
     void *out;
     const void *stw;     // stage table of the schedule (the fast kernels' layout)
-    const void *tw_hi;   // TWID: W^(q*1024), q <= tw_n/1024
-    const void *tw_lo;   // TWID: W^r, r < 1024
+    const void *tw_hi;   // TWID: W^(q*1024), q <= tw_n/1024 (FP64)
+    const void *tw_lo;   // TWID: W^r, r < 1024 (FP64)
     long long nlines, nlo;
     long long in_hi, in_lo, in_el;
     long long out_hi, out_lo, out_el;
@@ -214,6 +216,21 @@ struct TileStages {
     }
 };
 
+// Complex FP64 values of the four-step twiddles.
+struct Cd {
+    double r, i;
+};
+__device__ __forceinline__ Cd cd_mul(Cd a, Cd b) { return Cd{a.r * b.r - a.i * b.i, a.r * b.i + a.i * b.r}; }
+// W^ex from the two tables
+__device__ __forceinline__ Cd cd_root(const void *hi, const void *lo, unsigned long long ex)
+{
+    return cd_mul(reinterpret_cast<const Cd *>(hi)[ex >> 10], reinterpret_cast<const Cd *>(lo)[ex & 1023]);
+}
+__device__ __forceinline__ Cf cd_apply(Cf v, Cd w)
+{
+    return Cf{(float)((double)v.r * w.r - (double)v.i * w.i), (float)((double)v.r * w.i + (double)v.i * w.r)};
+}
+
 // a / b and a % b, a, b >= 0: 32-bit where the launch allows it (small: nlines < 2^31)
 __device__ __forceinline__ void tile_divmod(long long a, long long b, bool small, long long &q, long long &r)
 {
@@ -243,7 +260,7 @@ __global__ void __launch_bounds__(T *TL, (MODE & TM_HALF) ? 2 * T * TL / 256 : 1
     // outputs per thread, and the W^(lo*step) between them
     constexpr int IT = FL::J * FL::p;
     __shared__ __align__(16) typename TS::L buf[K > 1 ? TS::Pos::size(N) : 1];
-    __shared__ St s_step[TWID ? TL * IT : 1];
+    __shared__ Cd s_step[TWID ? TL * IT : 1];
 
     const int tid = threadIdx.x;
     const long long ntiles = (a.nlines + TL - 1) / TL;
@@ -279,16 +296,14 @@ __global__ void __launch_bounds__(T *TL, (MODE & TM_HALF) ? 2 * T * TL / 256 : 1
                 v[j][r] = get ? O::load(p0[r * step]) : O::zero();
         }
         if constexpr (TWID) {
-            const St *whi = reinterpret_cast<const St *>(a.tw_hi);
-            const St *wlo = reinterpret_cast<const St *>(a.tw_lo);
             for (int w = tid; w < TL * IT; w += T * TL) {
-                const int l = w / IT, i = w - (w / IT) * IT;
+                const int l = w % TL, i = w / TL;
                 long long h, o;
                 tile_divmod(l0 + (l < nl ? l : 0), a.nlo, small, h, o);
                 // element jT + q*NB of the thread's first, i = j*p + q (< tw_n: lo < tw_n / N)
                 const unsigned long long ex =
                     (unsigned long long)o * (unsigned)((i / FL::p) * T + (i % FL::p) * FL::NB);
-                s_step[w] = O::pack(O::cmul(O::load(whi[ex >> 10]), O::load(wlo[ex & 1023])));
+                s_step[w] = cd_root(a.tw_hi, a.tw_lo, ex);
             }
         }
         TS::template compute<0>(v, stw, t0, a.l1, (int)o0);
@@ -317,16 +332,13 @@ __global__ void __launch_bounds__(T *TL, (MODE & TM_HALF) ? 2 * T * TL / 256 : 1
     St *dst = reinterpret_cast<St *>(a.out) + hi * a.out_hi + lo * a.out_lo;
     const long long step = (long long)FL::NB * a.out_el;
     if constexpr (TWID) {
-        const St *whi = reinterpret_cast<const St *>(a.tw_hi);
-        const St *wlo = reinterpret_cast<const St *>(a.tw_lo);
-        const unsigned long long ex = (unsigned long long)lo * (unsigned)t;  // < tw_n
-        const C base = O::cmul(O::load(whi[ex >> 10]), O::load(wlo[ex & 1023]));
+        const Cd base = cd_root(a.tw_hi, a.tw_lo, (unsigned long long)lo * (unsigned)t);  // (< tw_n)
 #pragma unroll
         for (int j = 0; j < FL::J; ++j)
 #pragma unroll
             for (int q = 0; q < FL::p; ++q)
                 if (FL::live(t, j))
-                    out[j][q] = O::cmul(out[j][q], O::cmul(base, O::load(s_step[ln * IT + j * FL::p + q])));
+                    out[j][q] = cd_apply(out[j][q], cd_mul(base, s_step[(j * FL::p + q) * TL + ln]));
     }
 #pragma unroll
     for (int j = 0; j < FL::J; ++j) {

@@ -1,0 +1,55 @@
+"""GPU tests of multi-pass lines whose two passes run on tile kernels compiled at run time.
+
+Float lengths without a built-in four-step split (kfa_engine.hip bailey_plan), and the
+fixed-point builds' reference-order split, whose second pass reads its own rows of the
+full-length twiddle tables (TM_REF in kfa_tile.hpp).  Fixed point is bit-exact against the
+oracle, float within the float bar of FP64; contiguous and strided input, both directions.
+"""
+import numpy as np
+import pytest
+
+import kissfft_amd
+from helpers import ABS_FLOAT_BOUND, cplx, rel_l2
+from oracle import Oracle
+
+pytestmark = pytest.mark.gpu
+
+# halves of equal and of very different radices, odd lengths, a generic radix, a half with
+# component-wise hand-overs
+LENGTHS = [18750, 19683, 16807 * 2, 65536, 98304, 118098, 218700, 2 ** 18 * 3]
+
+
+def rnd(rng, dtype, shape):
+    if dtype == "float":
+        return rng.uniform(-1, 1, shape).astype(np.float32)
+    if dtype == "int16_t":
+        return rng.integers(-32768, 32768, shape).astype(np.int16)
+    return rng.integers(-(1 << 31), 1 << 31, shape, dtype=np.int64).astype(np.int32)
+
+
+@pytest.mark.parametrize("dtype", ["float", "int16_t", "int32_t"])
+@pytest.mark.parametrize("n", LENGTHS)
+def test_two_pass_lines(n, dtype, monkeypatch, capfd):
+    lib = kissfft_amd.load(dtype)
+    monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    lib.L.kiss_fft_cleanup()
+    b = 3
+    x = rnd(np.random.default_rng(n), dtype, (b, n, 2))
+    for inv in (False, True):
+        print("case", dtype, n, inv, flush=True)
+        y = np.zeros_like(x)
+        lib.fft_batch(lib.fft_alloc(n, inv), x, y, b, n, n)
+        if dtype == "float":
+            want = np.fft.ifft(cplx(x), axis=-1) * n if inv else np.fft.fft(cplx(x), axis=-1)
+            assert rel_l2(cplx(y), want) <= ABS_FLOAT_BOUND
+        else:
+            np.testing.assert_array_equal(y, Oracle(dtype).fft(x, inv))
+    xs = rnd(np.random.default_rng(n + 1), dtype, (1, 2 * n, 2))  # every other element
+    ys = np.zeros((1, n, 2), lib.scalar)
+    lib.fft_batch(lib.fft_alloc(n), xs, ys, 1, 2 * n, n, in_stride=2)
+    xd = np.ascontiguousarray(xs[:, ::2])
+    if dtype == "float":
+        assert rel_l2(cplx(ys), np.fft.fft(cplx(xd), axis=-1)) <= ABS_FLOAT_BOUND
+    else:
+        np.testing.assert_array_equal(ys, Oracle(dtype).fft(xd))
+    assert "tile" in capfd.readouterr().err
