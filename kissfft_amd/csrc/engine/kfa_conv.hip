@@ -101,7 +101,7 @@ extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, const vo
         if (rc == 0)
             rc = finish_out(O, s);
     }
-    release(I, s);
-    release(O, s);
+    release(I);
+    release(O);
     return call_end(s, sync || I.staged || O.staged, rc);
 }

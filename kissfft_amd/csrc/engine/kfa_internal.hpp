@@ -100,9 +100,25 @@ int current_device(int *dev);
 // stream-ordered scratch from the engine's per-device pool (free with hipFreeAsync)
 hipError_t scratch_alloc(void **p, size_t bytes, hipStream_t s);
 
+// Device memory for one call on stream s, from the engine's cache of blocks (kfa_engine.hip);
+// put() or the destructor gives it back once the call's work is queued.
+struct StreamMem {
+    void *p = nullptr;
+    StreamMem() = default;
+    StreamMem(const StreamMem &) = delete;
+    StreamMem &operator=(const StreamMem &) = delete;
+    int get(size_t bytes, hipStream_t s);
+    void put();
+    ~StreamMem() { put(); }
+
+  private:
+    hipStream_t s_ = nullptr;
+    struct MemBlock *block_ = nullptr;  // null: from the pool
+};
+
 // Scratch of one call: carved from the calling thread's current workspace when one is set
 // (a multi-batch's, allocated at its creation; the no-allocation entry point's static
-// device array), else stream-ordered from the device pool.  Released when the object
+// device array), else from the block cache (StreamMem).  Released when the object
 // goes out of scope (workspace carving is a stack: releases come in reverse order).
 struct Workspace {
     char *base = nullptr;
@@ -121,10 +137,9 @@ struct Scratch {
     ~Scratch();
 
   private:
-    hipStream_t s_ = nullptr;
+    StreamMem mem_;
     Workspace *ws_ = nullptr;
     size_t mark_ = 0;
-    bool pooled_ = false;
 };
 // Multi-pass batches run in chunks whose temporaries fit this many bytes: the free part
 // of the thread's workspace, else the chunk limit (KISSFFT_AMD_CHUNK_MB, default below:
@@ -173,29 +188,20 @@ int run_ndr(DevPlan &H, const RealTables &R, const std::vector<std::shared_ptr<D
 
 // A caller buffer: used in place when the device can access it, else staged through a
 // stream-ordered device copy (stage_in copies host -> device; finish_out device -> host).
-// The staging copy is returned to the pool by release() or, on an early return, by the
-// destructor.
+// The staging copy is given back by release() or, on an early return, by the destructor.
 struct Operand {
     const void *host = nullptr;  // non-null when staged
     void *dev = nullptr;
     size_t bytes = 0;
     bool staged = false;
-    hipStream_t s = nullptr;     // the stream the staging copy is ordered on
-    Operand() = default;
-    Operand(const Operand &) = delete;
-    Operand &operator=(const Operand &) = delete;
-    ~Operand()
-    {
-        if (staged && dev)
-            (void)hipFreeAsync(dev, s);
-    }
+    StreamMem mem;               // the staging copy
 };
 int stage_in(const void *p, size_t bytes, hipStream_t s, Operand &op);
 // gaps: the output span holds values the call must not touch (rows further apart than
 // their length); a staged copy then starts from the caller's bytes.
 int stage_out(void *p, size_t bytes, hipStream_t s, Operand &op, bool gaps = false);
 int finish_out(Operand &op, hipStream_t s);
-void release(Operand &op, hipStream_t s);
+void release(Operand &op);
 
 bool env_flag(const char *name, bool dflt);
 // float twiddles exp(-+2*pi*i*(j*step mod n)/n), j < count, FP64 rounded once (8 bytes each)
