@@ -17,10 +17,109 @@
 
 namespace kfa {
 
+// ------------------------------------------------------------------------------------
+// The cyclic convolution both kernels are made of: x -> IFFT_N(FFT_N(x) * H) on one line of
+// N = RS::N() points (a power of two), T threads a line.  The inputs arrive in registers
+// as the inputs of the forward schedule's first stage (element r*NB + b of butterfly b),
+// the results leave as the outputs of the inverse's last one.  The inverse runs the
+// schedule backwards, so its first stage takes exactly the values that the thread's
+// forward last stage left, and the product with H happens in registers between the two.
+// Only the 2 (K - 1) hand-overs between stages go through LDS.  What bounds the kernels is
+// vector arithmetic, then these hand-overs and their barriers.  Against the form that
+// staged the line through LDS before, between and after the two transforms (16 trips a
+// value with three stages; now 8) and had its inputs 8-way conflicting in LDS banks:
+// real FIR of 2^26 samples, 1000 taps (2048-point blocks) 303 -> 250 us (kernel); c2c 1009 x4096
+// 36.7 -> 30.9 us.
+//
+// LDS index of element e: one slot free after every 16, so that the last stage's inputs,
+// p = 4 .. 16 elements apart, fall in different banks (N + N/16 slots a line).
+// ------------------------------------------------------------------------------------
+__device__ __forceinline__ int conv_pos(int e) { return e + (e >> 4); }
+constexpr int conv_slots(int n) { return n + n / 16; }
+
+template <class Done, int... X>
+struct Reversed;
+template <int G, int... Y>
+struct Reversed<Radices<G, Y...>> {
+    typedef Radices<G, Y...> type;
+};
+template <int G, int... Y, int X, int... Xs>
+struct Reversed<Radices<G, Y...>, X, Xs...> {
+    typedef typename Reversed<Radices<G, X, Y...>, Xs...>::type type;
+};
+template <class RS>
+struct Backwards;
+template <int G, int R0, int... R>
+struct Backwards<Radices<G, R0, R...>> {
+    typedef typename Reversed<Radices<G, R0>, R...>::type type;
+};
+
+// Stages S .. K-1 of schedule RS on v, the inputs of stage S; the last stage's outputs in
+// `out`.  FRESH: the line's LDS holds nothing another thread still reads.
+template <bool INV, int T, class RS, int S, bool FRESH, class V, class W>
+__device__ __forceinline__ void conv_stages(V &v, W &out, F32::store2 *buf, const F32::store2 *stw, int t)
+{
+    typedef FastStage<F32, INV, T, RS, S, false> F;
+    typedef Ops<F32> O;
+    F::compute(v, stw, t);
+    if constexpr (S == RS::K - 1) {
+#pragma unroll
+        for (int j = 0; j < F::J; ++j)
+#pragma unroll
+            for (int q = 0; q < F::p; ++q)
+                out[j][q] = v[j][q];
+    } else {
+        typedef FastStage<F32, INV, T, RS, S + 1, false> Fn;
+        static_assert(F::NB % T == 0 && Fn::NB % T == 0, "whole butterflies per thread");
+        if constexpr (!FRESH)
+            line_sync<T>();
+#pragma unroll
+        for (int j = 0; j < F::J; ++j)
+#pragma unroll
+            for (int q = 0; q < F::p; ++q)
+                buf[conv_pos(t + j * T + q * F::NB)] = O::pack(v[j][q]);
+        line_sync<T>();
+        Cf n[Fn::J][Fn::p];
+#pragma unroll
+        for (int j = 0; j < Fn::J; ++j) {
+            const int b = t + j * T, u = b / Fn::P, o = b - u * Fn::P;
+#pragma unroll
+            for (int r = 0; r < Fn::p; ++r)
+                n[j][r] = O::load(buf[conv_pos(u * Fn::P * Fn::p + r * Fn::P + o)]);
+        }
+        conv_stages<INV, T, RS, S + 1, false>(n, out, buf, stw, t);
+    }
+}
+
+template <int T, class RS>
+struct Conv {
+    typedef typename Backwards<RS>::type RI;
+    typedef FastStage<F32, false, T, RS, 0, false> In;          // layout of the inputs
+    typedef FastStage<F32, false, T, RS, RS::K - 1, false> Mid;  // ... of the spectrum
+    typedef FastStage<F32, true, T, RI, RS::K - 1, false> Out;   // ... of the results
+    static_assert(RS::N() % T == 0 && RS::K > 1, "threads per line must divide the length");
+
+    __device__ __forceinline__ static void run(Cf (&v)[In::J][In::p], Cf (&out)[Out::J][Out::p], F32::store2 *buf,
+                                               const F32::store2 *stw_f, const F32::store2 *stw_i,
+                                               const F32::store2 *H, int t)
+    {
+        typedef Ops<F32> O;
+        Cf m[Mid::J][Mid::p];
+        conv_stages<false, T, RS, 0, true>(v, m, buf, stw_f, t);
+#pragma unroll
+        for (int j = 0; j < Mid::J; ++j)
+#pragma unroll
+            for (int q = 0; q < Mid::p; ++q)
+                m[j][q] = O::cmul(m[j][q], O::load(H[t + j * T + q * Mid::NB]));
+        // (the inverse's first stage reads element r*NB + b as the forward's last one left it)
+        conv_stages<true, T, RI, 0, false>(m, out, buf, stw_i, t);
+    }
+};
+
 struct BlueArgs {
     const void *in;
     void *out;
-    const void *stw_f, *stw_i;  // stage tables of the M-point schedule, forward and inverse
+    const void *stw_f, *stw_i;  // stage tables of the M-point schedule, and of it backwards
     const void *chirp;          // w[n], n < N
     const void *bfft;           // B[m], m < M
     int n;
@@ -37,51 +136,41 @@ __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
     typedef F32::store2 St;
     typedef Ops<F32> O;
     typedef Cx<F32> C;
+    typedef Conv<T, RS> CV;
+    typedef typename CV::In In;
+    typedef typename CV::Out Out;
     constexpr int M = RS::N();
-    constexpr int IT = M / T;
-    static_assert(M % T == 0, "threads per line must divide M");
     extern __shared__ __align__(16) unsigned char kfa_blue_smem[];
     const int line = threadIdx.x / T, t = threadIdx.x - line * T;
-    St *buf = reinterpret_cast<St *>(kfa_blue_smem) + line * (M + 1);
+    St *buf = reinterpret_cast<St *>(kfa_blue_smem) + line * conv_slots(M);
     const long long gl = blk * LPB + line;
     const bool ok = gl < a.nlines;
     const int n = a.n;
     const St *chirp = reinterpret_cast<const St *>(a.chirp);
-    const St *bf = reinterpret_cast<const St *>(a.bfft);
 
     const St *src;
     St *dst;
     line_base<St>(a, ok ? gl : 0, src, dst);
-    {
-        C v[IT];
+    C v[In::J][In::p], out[Out::J][Out::p];
 #pragma unroll
-        for (int k = 0; k < IT; ++k) {
-            const int i = t + k * T;
-            v[k] = (ok && i < n) ? O::cmul(O::load(src[(long long)i * a.in_el]), O::load(chirp[i])) : O::zero();
+    for (int j = 0; j < In::J; ++j)
+#pragma unroll
+        for (int r = 0; r < In::p; ++r) {
+            const int i = t + j * T + r * In::NB;
+            v[j][r] = (ok && i < n) ? O::cmul(O::load(src[(long long)i * a.in_el]), O::load(chirp[i])) : O::zero();
         }
-#pragma unroll
-        for (int k = 0; k < IT; ++k)
-            buf[t + k * T] = O::pack(v[k]);
-    }
-    __syncthreads();
-    tile_stages<F32, false, T, RS>(std::make_integer_sequence<int, RS::K>{}, buf,
-                                   reinterpret_cast<const St *>(a.stw_f), t);
-#pragma unroll
-    for (int k = 0; k < IT; ++k) {
-        const int i = t + k * T;
-        buf[i] = O::pack(O::cmul(O::load(buf[i]), O::load(bf[i])));
-    }
-    __syncthreads();
-    tile_stages<F32, true, T, RS>(std::make_integer_sequence<int, RS::K>{}, buf,
-                                  reinterpret_cast<const St *>(a.stw_i), t);
+    CV::run(v, out, buf, reinterpret_cast<const St *>(a.stw_f), reinterpret_cast<const St *>(a.stw_i),
+            reinterpret_cast<const St *>(a.bfft), t);
     if (!ok)
         return;
 #pragma unroll
-    for (int k = 0; k < IT; ++k) {
-        const int i = t + k * T;
-        if (i < n)
-            dst[(long long)i * a.out_el] = O::pack(O::cmul(O::load(buf[i]), O::load(chirp[i])));
-    }
+    for (int j = 0; j < Out::J; ++j)
+#pragma unroll
+        for (int q = 0; q < Out::p; ++q) {
+            const int i = t + j * T + q * Out::NB;
+            if (i < n)
+                dst[(long long)i * a.out_el] = O::pack(O::cmul(out[j][q], O::load(chirp[i])));
+        }
 }
 
 template <int T, int LPB, class RS>
@@ -104,7 +193,7 @@ namespace kfa {
 struct ConvArgs {
     const void *in;
     void *out;
-    const void *stw_f, *stw_i;  // stage tables of the N-point schedule
+    const void *stw_f, *stw_i;  // stage tables of the N-point schedule, and of it backwards
     const void *H;              // N complex
     long long nlines;           // complex blocks (REAL: ceil(nblocks / 2))
     long long nblocks;          // blocks of samples
@@ -117,73 +206,57 @@ __global__ void __launch_bounds__(T *LPB) k_conv(ConvArgs a)
     typedef F32::store2 St;
     typedef Ops<F32> O;
     typedef Cx<F32> C;
+    typedef Conv<T, RS> CV;
+    typedef typename CV::In In;
+    typedef typename CV::Out Out;
     constexpr int N = RS::N();
-    constexpr int IT = N / T;
-    static_assert(N % T == 0, "threads per line must divide N");
     extern __shared__ __align__(16) unsigned char kfa_conv_smem[];
     const int line = threadIdx.x / T, t = threadIdx.x - line * T;
-    St *buf = reinterpret_cast<St *>(kfa_conv_smem) + line * (N + 1);
+    St *buf = reinterpret_cast<St *>(kfa_conv_smem) + line * conv_slots(N);
     const long long gl = (long long)blockIdx.x * LPB + line;
     const bool ok = gl < a.nlines;
     const long long b0 = REAL ? 2 * gl : gl;          // first block of this line
     const bool two = REAL && b0 + 1 < a.nblocks;      // second block (imaginary part)
-    const St *H = reinterpret_cast<const St *>(a.H);
 
-    {
-        C v[IT];
-        if constexpr (REAL) {
-            const float *x = reinterpret_cast<const float *>(a.in);
-            const float *xa = x + (ok ? b0 : 0) * a.ngood, *xb = x + (two ? b0 + 1 : 0) * a.ngood;
+    C v[In::J][In::p], out[Out::J][Out::p];
+    if constexpr (REAL) {
+        const float *x = reinterpret_cast<const float *>(a.in);
+        const float *xa = x + (ok ? b0 : 0) * a.ngood, *xb = x + (two ? b0 + 1 : 0) * a.ngood;
 #pragma unroll
-            for (int k = 0; k < IT; ++k) {
-                const int i = t + k * T;
-                v[k] = C{ok ? xa[i] : 0.0f, two ? xb[i] : 0.0f};
+        for (int j = 0; j < In::J; ++j)
+#pragma unroll
+            for (int r = 0; r < In::p; ++r) {
+                const int i = t + j * T + r * In::NB;
+                v[j][r] = C{ok ? xa[i] : 0.0f, two ? xb[i] : 0.0f};
             }
-        } else {
-            const St *x = reinterpret_cast<const St *>(a.in) + (ok ? gl : 0) * a.ngood;
+    } else {
+        const St *x = reinterpret_cast<const St *>(a.in) + (ok ? gl : 0) * a.ngood;
 #pragma unroll
-            for (int k = 0; k < IT; ++k)
-                v[k] = ok ? O::load(x[t + k * T]) : O::zero();
-        }
+        for (int j = 0; j < In::J; ++j)
 #pragma unroll
-        for (int k = 0; k < IT; ++k)
-            buf[t + k * T] = O::pack(v[k]);
+            for (int r = 0; r < In::p; ++r)
+                v[j][r] = ok ? O::load(x[t + j * T + r * In::NB]) : O::zero();
     }
-    __syncthreads();
-    tile_stages<F32, false, T, RS>(std::make_integer_sequence<int, RS::K>{}, buf,
-                                   reinterpret_cast<const St *>(a.stw_f), t);
-#pragma unroll
-    for (int k = 0; k < IT; ++k) {
-        const int i = t + k * T;
-        buf[i] = O::pack(O::cmul(O::load(buf[i]), O::load(H[i])));
-    }
-    __syncthreads();
-    tile_stages<F32, true, T, RS>(std::make_integer_sequence<int, RS::K>{}, buf,
-                                  reinterpret_cast<const St *>(a.stw_i), t);
+    CV::run(v, out, buf, reinterpret_cast<const St *>(a.stw_f), reinterpret_cast<const St *>(a.stw_i),
+            reinterpret_cast<const St *>(a.H), t);
     if (!ok)
         return;
-    if constexpr (REAL) {
-        float *y = reinterpret_cast<float *>(a.out);
-        float *ya = y + b0 * a.ngood, *yb = y + (b0 + 1) * a.ngood;
 #pragma unroll
-        for (int k = 0; k < IT; ++k) {
-            const int i = t + k * T;
-            if (i < a.ngood) {
-                const C c = O::load(buf[i]);
-                ya[i] = c.r;
+    for (int j = 0; j < Out::J; ++j)
+#pragma unroll
+        for (int q = 0; q < Out::p; ++q) {
+            const int i = t + j * T + q * Out::NB;
+            if (i >= a.ngood)
+                continue;
+            if constexpr (REAL) {
+                float *y = reinterpret_cast<float *>(a.out) + b0 * a.ngood;
+                y[i] = out[j][q].r;
                 if (two)
-                    yb[i] = c.i;
+                    y[a.ngood + i] = out[j][q].i;
+            } else {
+                (reinterpret_cast<St *>(a.out) + gl * a.ngood)[i] = O::pack(out[j][q]);
             }
         }
-    } else {
-        St *y = reinterpret_cast<St *>(a.out) + gl * a.ngood;
-#pragma unroll
-        for (int k = 0; k < IT; ++k) {
-            const int i = t + k * T;
-            if (i < a.ngood)
-                y[i] = buf[i];
-        }
-    }
 }
 
 }  // namespace kfa

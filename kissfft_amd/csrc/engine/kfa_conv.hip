@@ -48,7 +48,8 @@ static int conv_plan(int dev, int nfft, int real, const void *H, std::shared_ptr
     const std::vector<unsigned char> tf = float_twiddles(nfft, 0, nfft, 1), ti = float_twiddles(nfft, 1, nfft, 1);
     int rc;
     if ((rc = make_stage_table_raw(tf.data(), KFA_F32, nfft, cp->v->radices, cp->v->tw_pad, 0, cp->mem_f)) ||
-        (rc = make_stage_table_raw(ti.data(), KFA_F32, nfft, cp->v->radices, cp->v->tw_pad, 0, cp->mem_i)) ||
+        (rc = make_stage_table_raw(ti.data(), KFA_F32, nfft, {cp->v->radices.rbegin(), cp->v->radices.rend()},
+                                   cp->v->tw_pad, 0, cp->mem_i)) ||
         (rc = dev_upload(H, (size_t)nfft * 8, cp->mem_h)))
         return rc;
     g_conv[key] = cp;

@@ -1184,7 +1184,8 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
         int rc;
         RelaxCapture relax;
         if ((rc = make_stage_table_raw(tf.data(), KFA_F32, M, bc->v->radices, bc->v->tw_pad, 0, bc->mem_f)) ||
-            (rc = make_stage_table_raw(ti.data(), KFA_F32, M, bc->v->radices, bc->v->tw_pad, 0, bc->mem_i)) ||
+            (rc = make_stage_table_raw(ti.data(), KFA_F32, M, {bc->v->radices.rbegin(), bc->v->radices.rend()},
+                                       bc->v->tw_pad, 0, bc->mem_i)) ||
             (rc = dev_upload(hw.data(), hw.size() * 4, bc->mem_chirp)) ||
             (rc = dev_upload(hb.data(), hb.size() * 4, bc->mem_bfft)))
             return rc;

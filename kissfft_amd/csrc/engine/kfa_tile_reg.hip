@@ -265,7 +265,7 @@ const std::vector<PlaneVariant> &plane_registry()
 template <int T, int LPB, class RS>
 static int launch_blue(const BlueArgs &a, hipStream_t s)
 {
-    const size_t lds = (size_t)LPB * (RS::N() + 1) * sizeof(float2);
+    const size_t lds = (size_t)LPB * conv_slots(RS::N()) * sizeof(float2);
     static std::once_flag once;
     std::call_once(once, [=] {
         (void)hipFuncSetAttribute((const void *)k_blue<T, LPB, RS>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -289,7 +289,7 @@ static void add_blue(std::vector<BlueVariant> &v, const char *name)
     f.LPB = LPB;
     f.radices = {R...};
     f.tw_pad = 2;
-    f.lds = (size_t)LPB * (RS::N() + 1) * 8;
+    f.lds = (size_t)LPB * conv_slots(RS::N()) * 8;
     f.name = name;
     f.launch = &launch_blue<T, LPB, RS>;
     v.push_back(f);
@@ -300,7 +300,7 @@ const std::vector<BlueVariant> &blue_registry()
     static std::vector<BlueVariant> *reg = [] {
         auto *v = new std::vector<BlueVariant>();
         add_blue<8, 8, 8, 8>(*v, "blue64_88_t8x8");
-        add_blue<16, 4, 8, 16>(*v, "blue128_816_t16x4");
+        add_blue<8, 8, 8, 16>(*v, "blue128_816_t8x8");
         add_blue<16, 4, 16, 16>(*v, "blue256_1616_t16x4");
         add_blue<64, 2, 8, 8, 8>(*v, "blue512_888_t64x2");
         add_blue<64, 2, 16, 16, 4>(*v, "blue1024_16164_t64x2");
@@ -314,7 +314,7 @@ const std::vector<BlueVariant> &blue_registry()
 template <int T, int LPB, bool REAL, class RS>
 static int launch_conv(const ConvArgs &a, hipStream_t s)
 {
-    const size_t lds = (size_t)LPB * (RS::N() + 1) * sizeof(float2);
+    const size_t lds = (size_t)LPB * conv_slots(RS::N()) * sizeof(float2);
     static std::once_flag once;
     std::call_once(once, [=] {
         (void)hipFuncSetAttribute((const void *)k_conv<T, LPB, REAL, RS>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -339,7 +339,7 @@ static void add_conv(std::vector<ConvVariant> &v, const char *name)
         f.LPB = LPB;
         f.radices = {R...};
         f.tw_pad = 2;
-        f.lds = (size_t)LPB * (RS::N() + 1) * 8;
+        f.lds = (size_t)LPB * conv_slots(RS::N()) * 8;
         f.name = name;
         f.launch = real ? &launch_conv<T, LPB, true, RS> : &launch_conv<T, LPB, false, RS>;
         v.push_back(f);
