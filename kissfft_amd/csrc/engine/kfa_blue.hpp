@@ -91,7 +91,11 @@ __device__ __forceinline__ void conv_stages(V &v, W &out, F32::store2 *buf, cons
     }
 }
 
-template <int T, class RS>
+__device__ __forceinline__ Cf conv_mul(Cf v, float2 h) { return Ops<F32>::cmul(v, Ops<F32>::load(h)); }
+__device__ __forceinline__ Cf conv_mul(Cf v, Cd h) { return cd_apply(v, h); }
+
+// HT: the spectrum's entries, float2 or FP64 (Cd).
+template <int T, class RS, class HT>
 struct Conv {
     typedef typename Backwards<RS>::type RI;
     typedef FastStage<F32, false, T, RS, 0, false> In;          // layout of the inputs
@@ -100,17 +104,16 @@ struct Conv {
     static_assert(RS::N() % T == 0 && RS::K > 1, "threads per line must divide the length");
 
     __device__ __forceinline__ static void run(Cf (&v)[In::J][In::p], Cf (&out)[Out::J][Out::p], F32::store2 *buf,
-                                               const F32::store2 *stw_f, const F32::store2 *stw_i,
-                                               const F32::store2 *H, int t)
+                                               const F32::store2 *stw_f, const F32::store2 *stw_i, const HT *H,
+                                               int t)
     {
-        typedef Ops<F32> O;
         Cf m[Mid::J][Mid::p];
         conv_stages<false, T, RS, 0, true>(v, m, buf, stw_f, t);
 #pragma unroll
         for (int j = 0; j < Mid::J; ++j)
 #pragma unroll
             for (int q = 0; q < Mid::p; ++q)
-                m[j][q] = O::cmul(m[j][q], O::load(H[t + j * T + q * Mid::NB]));
+                m[j][q] = conv_mul(m[j][q], H[t + j * T + q * Mid::NB]);
         // (the inverse's first stage reads element r*NB + b as the forward's last one left it)
         conv_stages<true, T, RI, 0, false>(m, out, buf, stw_i, t);
     }
@@ -136,7 +139,7 @@ __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
     typedef F32::store2 St;
     typedef Ops<F32> O;
     typedef Cx<F32> C;
-    typedef Conv<T, RS> CV;
+    typedef Conv<T, RS, St> CV;
     typedef typename CV::In In;
     typedef typename CV::Out Out;
     constexpr int M = RS::N();
@@ -187,17 +190,19 @@ namespace kfa {
 // k reads the window in[k*ngood .. k*ngood + N), is transformed, multiplied by the filter
 // spectrum H (already scaled by 1/N), transformed back, and its first ngood samples --
 // the ones the rotated impulse response leaves free of wrap-around -- are written to
-// out[k*ngood ..].  One block per T threads, entirely in LDS.  REAL: the samples are
+// out[k*ngood ..].  The last block may reach past the nin input samples (read as zeros) and
+// the nout output samples (not written).  One block per T threads.  REAL: the samples are
 // real and two consecutive blocks travel as the real and imaginary parts of one complex
 // block; with a real impulse response the two convolutions stay separate.
 struct ConvArgs {
     const void *in;
     void *out;
     const void *stw_f, *stw_i;  // stage tables of the N-point schedule, and of it backwards
-    const void *H;              // N complex
-    long long nlines;           // complex blocks (REAL: ceil(nblocks / 2))
-    long long nblocks;          // blocks of samples
-    long long ngood;
+    const void *H;              // N complex FP64: the product is rounded once, which makes up for
+                                // the roundings of a longer block (4096 for 2048 points)
+    long long nlines;           // complex blocks (REAL: two blocks of samples each)
+    long long ngood;            // samples a block yields
+    long long nin, nout;
 };
 
 template <int T, int LPB, bool REAL, class RS>
@@ -206,7 +211,7 @@ __global__ void __launch_bounds__(T *LPB) k_conv(ConvArgs a)
     typedef F32::store2 St;
     typedef Ops<F32> O;
     typedef Cx<F32> C;
-    typedef Conv<T, RS> CV;
+    typedef Conv<T, RS, Cd> CV;
     typedef typename CV::In In;
     typedef typename CV::Out Out;
     constexpr int N = RS::N();
@@ -215,46 +220,54 @@ __global__ void __launch_bounds__(T *LPB) k_conv(ConvArgs a)
     St *buf = reinterpret_cast<St *>(kfa_conv_smem) + line * conv_slots(N);
     const long long gl = (long long)blockIdx.x * LPB + line;
     const bool ok = gl < a.nlines;
-    const long long b0 = REAL ? 2 * gl : gl;          // first block of this line
-    const bool two = REAL && b0 + 1 < a.nblocks;      // second block (imaginary part)
+    // the line's first sample, its second block's (REAL), and what is left of the input there
+    const long long s0 = (REAL ? 2 * gl : gl) * a.ngood, s1 = s0 + a.ngood;
+    auto left = [](long long end, long long at) {
+        const long long d = end - at;
+        return (int)(d < 0 ? 0 : d < N ? d : N);
+    };
+    const int in0 = ok ? left(a.nin, s0) : 0, in1 = ok && REAL ? left(a.nin, s1) : 0;
 
     C v[In::J][In::p], out[Out::J][Out::p];
     if constexpr (REAL) {
-        const float *x = reinterpret_cast<const float *>(a.in);
-        const float *xa = x + (ok ? b0 : 0) * a.ngood, *xb = x + (two ? b0 + 1 : 0) * a.ngood;
+        const float *x = reinterpret_cast<const float *>(a.in) + (ok ? s0 : 0);
 #pragma unroll
         for (int j = 0; j < In::J; ++j)
 #pragma unroll
             for (int r = 0; r < In::p; ++r) {
                 const int i = t + j * T + r * In::NB;
-                v[j][r] = C{ok ? xa[i] : 0.0f, two ? xb[i] : 0.0f};
+                v[j][r] = C{i < in0 ? x[i] : 0.0f, i < in1 ? x[a.ngood + i] : 0.0f};
             }
     } else {
-        const St *x = reinterpret_cast<const St *>(a.in) + (ok ? gl : 0) * a.ngood;
+        const St *x = reinterpret_cast<const St *>(a.in) + (ok ? s0 : 0);
 #pragma unroll
         for (int j = 0; j < In::J; ++j)
 #pragma unroll
-            for (int r = 0; r < In::p; ++r)
-                v[j][r] = ok ? O::load(x[t + j * T + r * In::NB]) : O::zero();
+            for (int r = 0; r < In::p; ++r) {
+                const int i = t + j * T + r * In::NB;
+                v[j][r] = i < in0 ? O::load(x[i]) : O::zero();
+            }
     }
     CV::run(v, out, buf, reinterpret_cast<const St *>(a.stw_f), reinterpret_cast<const St *>(a.stw_i),
-            reinterpret_cast<const St *>(a.H), t);
+            reinterpret_cast<const Cd *>(a.H), t);
     if (!ok)
         return;
+    const int good = (int)a.ngood, out0 = left(a.nout, s0), out1 = REAL ? left(a.nout, s1) : 0;
 #pragma unroll
     for (int j = 0; j < Out::J; ++j)
 #pragma unroll
         for (int q = 0; q < Out::p; ++q) {
             const int i = t + j * T + q * Out::NB;
-            if (i >= a.ngood)
+            if (i >= good)
                 continue;
             if constexpr (REAL) {
-                float *y = reinterpret_cast<float *>(a.out) + b0 * a.ngood;
-                y[i] = out[j][q].r;
-                if (two)
-                    y[a.ngood + i] = out[j][q].i;
-            } else {
-                (reinterpret_cast<St *>(a.out) + gl * a.ngood)[i] = O::pack(out[j][q]);
+                float *y = reinterpret_cast<float *>(a.out) + s0;
+                if (i < out0)
+                    y[i] = out[j][q].r;
+                if (i < out1)
+                    y[good + i] = out[j][q].i;
+            } else if (i < out0) {
+                (reinterpret_cast<St *>(a.out) + s0)[i] = O::pack(out[j][q]);
             }
         }
 }

@@ -1,6 +1,6 @@
 // kfa_conv.hip -- fast FIR filtering by overlap-scrap (k_conv in kfa_blue.hpp).
 //
-// The filter spectrum (N complex, scaled by 1/N) comes from the host layer; the engine
+// The filter spectrum (N complex FP64, scaled by 1/N) comes from the host layer; the engine
 // keeps a device copy per (device, N, spectrum contents) together with the stage tables
 // of the N-point schedule, and runs every complete block of a call in one launch.
 #include <hip/hip_runtime.h>
@@ -29,7 +29,7 @@ static std::map<std::tuple<int, int, int, std::string>, std::shared_ptr<const Co
 
 static int conv_plan(int dev, int nfft, int real, const void *H, std::shared_ptr<const ConvPlan> &out)
 {
-    const std::string key_h((const char *)H, (size_t)nfft * 8);
+    const std::string key_h((const char *)H, (size_t)nfft * 16);
     std::lock_guard<std::mutex> g(g_conv_mu);
     const auto key = std::make_tuple(dev, nfft, real, key_h);
     auto it = g_conv.find(key);
@@ -50,11 +50,33 @@ static int conv_plan(int dev, int nfft, int real, const void *H, std::shared_ptr
     if ((rc = make_stage_table_raw(tf.data(), KFA_F32, nfft, cp->v->radices, cp->v->tw_pad, 0, cp->mem_f)) ||
         (rc = make_stage_table_raw(ti.data(), KFA_F32, nfft, {cp->v->radices.rbegin(), cp->v->radices.rend()},
                                    cp->v->tw_pad, 0, cp->mem_i)) ||
-        (rc = dev_upload(H, (size_t)nfft * 8, cp->mem_h)))
+        (rc = dev_upload(H, (size_t)nfft * 16, cp->mem_h)))
         return rc;
     g_conv[key] = cp;
     out = cp;
     return 0;
+}
+
+// Moves `words` 4-byte words from buf[from ..] to buf[0 ..], the spans overlapping or not: one
+// workgroup reads them all before it writes any.  (The host's memmove over the bus took
+// about 0.1 us a word: a call of 2^26 samples and 1000 taps 434 -> 250 us, of 228398 samples
+// and 239 taps 89 -> 25 us.)
+constexpr int kMoveThreads = 1024, kMoveWords = 16 * kMoveThreads;
+static __global__ void __launch_bounds__(kMoveThreads) k_move_front(unsigned *buf, long long from, int words)
+{
+    unsigned v[kMoveWords / kMoveThreads];
+#pragma unroll
+    for (int k = 0; k < kMoveWords / kMoveThreads; ++k) {
+        const int i = threadIdx.x + k * kMoveThreads;
+        v[k] = i < words ? buf[from + i] : 0u;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kMoveWords / kMoveThreads; ++k) {
+        const int i = threadIdx.x + k * kMoveThreads;
+        if (i < words)
+            buf[i] = v[k];
+    }
 }
 
 void conv_release()
@@ -67,26 +89,27 @@ void conv_release()
 
 using namespace kfa;
 
-extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, const void *in, void *out, long long nblocks,
-                           long long ngood, void *stream, int sync)
+extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, long long nh, void *in, void *out,
+                           long long nout, long long keep, int *moved, void *stream, int sync)
 {
+    *moved = 0;
     if (type != KFA_F32)
         return fail(-2, "fast convolution is float only (the reference scales by 1/nfft in float)");
-    if (nfft <= 0 || ngood <= 0 || ngood > nfft || nblocks < 0)
+    if (nfft <= 0 || nh <= 0 || nh > nfft || nout < 0 || keep < 0)
         return fail(-2, "fast convolution: bad sizes");
     hipStream_t s;
     int dev;
     int rc = call_begin(stream, &s, &dev);
-    if (rc || nblocks == 0)
+    if (rc || nout == 0)
         return rc;
     std::shared_ptr<const ConvPlan> cp;
     if ((rc = conv_plan(dev, nfft, real, H, cp)))
         return rc;
     const size_t sb = real ? 4 : 8;
     Operand I, O;
-    rc = stage_in(in, sb * (size_t)((nblocks - 1) * ngood + nfft), s, I);
+    rc = stage_in(in, sb * (size_t)(nout + nh - 1), s, I);
     if (rc == 0)
-        rc = stage_out(out, sb * (size_t)(nblocks * ngood), s, O);
+        rc = stage_out(out, sb * (size_t)nout, s, O);
     if (rc == 0) {
         ConvArgs a{};
         a.in = I.dev;
@@ -94,11 +117,25 @@ extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, const vo
         a.stw_f = cp->mem_f.get();
         a.stw_i = cp->mem_i.get();
         a.H = cp->mem_h.get();
-        a.nblocks = nblocks;
-        a.nlines = real ? (nblocks + 1) / 2 : nblocks;
-        a.ngood = ngood;
+        a.ngood = nfft - nh + 1;
+        a.nin = nout + nh - 1;
+        a.nout = nout;
+        const long long blocks = (nout + a.ngood - 1) / a.ngood;
+        a.nlines = real ? (blocks + 1) / 2 : blocks;
         ++g_launches;
         rc = cp->v->launch(a, s) ? fail(-3, "fast convolution launch failed") : 0;
+        const long long words = keep * (long long)(sb / 4);
+        if (rc == 0 && !I.staged && words > 0 && words <= kMoveWords) {
+            // the samples not used yet go to the front of the caller's device buffer, behind
+            // the convolution (from the host each word would cross the bus on its own)
+            hipLaunchKernelGGL(k_move_front, dim3(1), dim3(kMoveThreads), 0, s, (unsigned *)I.dev,
+                               nout * (long long)(sb / 4), (int)words);
+            ++g_launches;
+            if (hipGetLastError() != hipSuccess)
+                rc = fail(-3, "fast convolution: moving the rest failed");
+            else
+                *moved = 1;
+        }
         if (rc == 0)
             rc = finish_out(O, s);
     }

@@ -352,11 +352,13 @@ const std::vector<ConvVariant> &conv_registry()
         auto *v = new std::vector<ConvVariant>();
         add_conv<16, 4, 16, 16>(*v, "conv256_1616_t16x4");
         add_conv<64, 2, 8, 8, 8>(*v, "conv512_888_t64x2");
-        add_conv<64, 2, 16, 16, 4>(*v, "conv1024_16164_t64x2");
-        add_conv<128, 2, 16, 16, 8>(*v, "conv2048_16168_t128x2");
-        add_conv<256, 1, 16, 16, 16>(*v, "conv4096_161616_t256");
-        add_conv<512, 1, 16, 16, 8, 4>(*v, "conv8192_161684_t512");
-        add_conv<256, 1, 16, 16, 8, 4>(*v, "conv8192_161684_t256");
+        add_conv<128, 2, 8, 8, 4, 4>(*v, "conv1024_8844_t128x2");
+        // 8 values a thread (64 registers, twice the waves of 16 values): 2^26 real samples,
+        // 1000 taps, 2048 points 227 us against 255 with 16, 16, 8 at 128 threads (359 at 64,
+        // a wave a line without barriers), 4096 points 194 against 208 with 16, 16, 16
+        add_conv<256, 2, 8, 8, 8, 4>(*v, "conv2048_8884_t256x2");
+        add_conv<512, 1, 8, 8, 8, 8>(*v, "conv4096_8888_t512");
+        add_conv<512, 1, 8, 8, 8, 4, 4>(*v, "conv8192_88844_t512");
         return v;
     }();
     return *reg;

@@ -6,9 +6,9 @@
  * Plan (kiss_fastfir.c:65-153): block length nfft, ngood = nfft - nh + 1 good samples per
  * block; the impulse response is rotated left by nh-1 (h[nh-1] first, then zeros, then
  * h[0..nh-2] at the end) so that the wrap-around lands in the block's tail; its spectrum,
- * scaled by 1/nfft, is computed here in FP64 and rounded once.  For the real filter the
- * full complex spectrum of the real response is kept: the GPU filters two real blocks per
- * complex transform.
+ * scaled by 1/length, is computed here in FP64 and kept so.  For the real filter the full
+ * complex spectrum of the real response is kept: the GPU filters two real blocks per
+ * complex transform.  The GPU's blocks have a length of their own (ff_block).
  */
 #include <math.h>
 #include <string.h>
@@ -19,14 +19,16 @@
 struct kiss_fastfir_state {
     size_t nfft;
     size_t ngood;
+    size_t nh;
+    size_t nblk;      /* points of the GPU's transforms (ff_block) */
     int real;
-    kiss_fft_cpx *H;  /* nfft complex, spectrum / nfft */
+    double *H;        /* nblk FP64 pairs, spectrum / nblk */
     void *tmpbuf;     /* nfft samples, the flush block */
 };
 
 #ifndef FIXED_POINT
-/* in-place radix-2 FFT in FP64, forward, n a power of two */
-static void fft_f64(double *re, double *im, size_t n)
+/* in-place radix-2 FFT in FP64, forward, n a power of two; w: room for n doubles */
+static void fft_f64(double *re, double *im, size_t n, double *w)
 {
     size_t i, j, len, k;
     for (i = 1, j = 0; i < n; ++i) {
@@ -43,11 +45,15 @@ static void fft_f64(double *re, double *im, size_t n)
             im[j] = t;
         }
     }
+    for (k = 0; k < n / 2; ++k) {
+        const double ang = -2.0 * 3.14159265358979323846264338327 * (double)k / (double)n;
+        w[2 * k] = cos(ang);
+        w[2 * k + 1] = sin(ang);
+    }
     for (len = 2; len <= n; len <<= 1)
-        for (k = 0; k < len / 2; ++k) {
-            const double ang = -2.0 * 3.14159265358979323846264338327 * (double)k / (double)len;
-            const double wr = cos(ang), wi = sin(ang);
-            for (i = 0; i < n; i += len) {
+        for (i = 0; i < n; i += len)
+            for (k = 0; k < len / 2; ++k) {
+                const double wr = w[2 * k * (n / len)], wi = w[2 * k * (n / len) + 1];
                 const size_t a = i + k, b = i + k + len / 2;
                 const double xr = re[b] * wr - im[b] * wi, xi = re[b] * wi + im[b] * wr;
                 re[b] = re[a] - xr;
@@ -55,7 +61,32 @@ static void fft_f64(double *re, double *im, size_t n)
                 re[a] += xr;
                 im[a] += xi;
             }
+}
+#endif
+
+#ifndef FIXED_POINT
+/* Transform length for a response of nh taps.  A call's output depends on nfft only through
+ * its sample count (complete blocks of nfft - nh + 1 good samples), so the GPU takes the
+ * length that costs least per good sample: the kernel's time per point of a block (2^26
+ * real samples: ps), times the points per good sample.  1000 taps, default nfft 2048: 4096
+ * points 194 us against 227. */
+static size_t ff_block(size_t nh)
+{
+    static const struct { size_t n; double ps; } len[] = {{256, 4.25}, {512, 3.85}, {1024, 4.31}, {2048, 3.46},
+                                                          {4096, 4.36}, {8192, 5.6}};
+    size_t i, best = 0;
+    double least = 0;
+    for (i = 0; i < sizeof len / sizeof len[0]; ++i) {
+        double cost;
+        if (len[i].n < 2 * nh && len[i].n < 8192)
+            continue;
+        cost = len[i].ps * (double)len[i].n / (double)(len[i].n - nh + 1);
+        if (best == 0 || cost < least) {
+            best = len[i].n;
+            least = cost;
         }
+    }
+    return best;
 }
 #endif
 
@@ -71,7 +102,7 @@ static kiss_fastfir_cfg ff_alloc(const void *h, size_t nh, int real, size_t *pnf
     KF_ERROR("kiss_fastfir_alloc: float builds only (the spectrum is scaled by 1/nfft in float)");
     return NULL;
 #else
-    size_t nfft = pnfft ? *pnfft : 0, i;
+    size_t nfft = pnfft ? *pnfft : 0, nblk, i;
     if (nh < 1)
         return NULL;
     if (nfft == 0) {
@@ -90,8 +121,9 @@ static kiss_fastfir_cfg ff_alloc(const void *h, size_t nh, int real, size_t *pnf
         KF_ERROR("kiss_fastfir_alloc: block length %zu unsupported (powers of two 256..8192, >= taps)", nfft);
         return NULL;
     }
+    nblk = ff_block(nh);
     const size_t samp = real ? sizeof(kiss_fft_scalar) : sizeof(kiss_fft_cpx);
-    const size_t need = sizeof(struct kiss_fastfir_state) + sizeof(kiss_fft_cpx) * nfft + samp * nfft;
+    const size_t need = sizeof(struct kiss_fastfir_state) + 2 * sizeof(double) * nblk + samp * nfft;
     kiss_fastfir_cfg st = NULL;
     if (lenmem == NULL) {
         st = (kiss_fastfir_cfg)malloc(need);
@@ -104,21 +136,25 @@ static kiss_fastfir_cfg ff_alloc(const void *h, size_t nh, int real, size_t *pnf
         return NULL;
     st->nfft = nfft;
     st->ngood = nfft - nh + 1;
+    st->nh = nh;
+    st->nblk = nblk;
     st->real = real;
-    st->H = (kiss_fft_cpx *)(st + 1);
-    st->tmpbuf = (void *)(st->H + nfft);
+    st->H = (double *)(st + 1);
+    st->tmpbuf = (void *)(st->H + 2 * nblk);
 
-    double *re = (double *)calloc(nfft, sizeof(double)), *im = (double *)calloc(nfft, sizeof(double));
-    if (!re || !im) {
+    double *re = (double *)calloc(nblk, sizeof(double)), *im = (double *)calloc(nblk, sizeof(double));
+    double *w = (double *)malloc(nblk * sizeof(double));
+    if (!re || !im || !w) {
         free(re);
         free(im);
+        free(w);
         if (!lenmem)
             free(st);
         return NULL;
     }
     /* the rotated impulse response, kiss_fastfir.c:137-141 */
     for (i = 0; i < nh; ++i) {
-        const size_t at = (i == nh - 1) ? 0 : nfft - nh + 1 + i;
+        const size_t at = (i == nh - 1) ? 0 : nblk - nh + 1 + i;
         if (real) {
             re[at] = ((const kiss_fft_scalar *)h)[i];
         } else {
@@ -126,50 +162,56 @@ static kiss_fastfir_cfg ff_alloc(const void *h, size_t nh, int real, size_t *pnf
             im[at] = ((const kiss_fft_cpx *)h)[i].i;
         }
     }
-    fft_f64(re, im, nfft);
-    for (i = 0; i < nfft; ++i) {
-        st->H[i].r = (kiss_fft_scalar)(re[i] / (double)nfft);
-        st->H[i].i = (kiss_fft_scalar)(im[i] / (double)nfft);
+    fft_f64(re, im, nblk, w);
+    for (i = 0; i < nblk; ++i) {
+        st->H[2 * i] = re[i] / (double)nblk;
+        st->H[2 * i + 1] = im[i] / (double)nblk;
     }
     free(re);
     free(im);
+    free(w);
     return st;
 #endif
 }
 
-/* every complete block of the n samples at in; returns the good samples written */
-static size_t ff_blocks(kiss_fastfir_cfg st, const void *in, void *out, size_t n)
+/* every complete block of the n samples at in; returns the good samples written.  *moved: the
+ * samples after them are at the front of `in` already (rest != 0, device memory) */
+static size_t ff_blocks(kiss_fastfir_cfg st, void *in, void *out, size_t n, int rest, int *moved)
 {
+    *moved = 0;
     if (n < st->nfft)
         return 0;
-    const long long nb = (long long)((n - st->nfft) / st->ngood + 1);
-    if (kfa_fastfir(KF_TYPE, (int)st->nfft, st->real, st->H, in, out, nb, (long long)st->ngood, NULL, 1) != 0) {
+    const size_t nout = ((n - st->nfft) / st->ngood + 1) * st->ngood;
+    if (kfa_fastfir(KF_TYPE, (int)st->nblk, st->real, st->H, (long long)st->nh, in, out, (long long)nout,
+                    rest ? (long long)(n - nout) : 0, moved, NULL, 1) != 0) {
         KF_ERROR("kiss_fastfir: %s", kfa_last_error());
         return 0;
     }
-    return (size_t)nb * st->ngood;
+    return nout;
 }
 
 static size_t ff_run(kiss_fastfir_cfg st, void *inbuf, void *outbuf, size_t n_new, size_t *offset)
 {
     const size_t samp = st->real ? sizeof(kiss_fft_scalar) : sizeof(kiss_fft_cpx);
     const size_t ntot = n_new + *offset;
+    int moved;
     if (n_new == 0) {
         /* flush, kiss_fastfir.c:200-217: complete blocks, then the zero-padded rest */
-        size_t done = ff_blocks(st, inbuf, outbuf, ntot), n = ntot - done, keep;
+        size_t done = ff_blocks(st, inbuf, outbuf, ntot, 0, &moved), n = ntot - done, keep;
         char *tmp = (char *)st->tmpbuf;
         memset(tmp, 0, samp * st->nfft);
         memcpy(tmp, (const char *)inbuf + samp * done, samp * n);
-        if (ff_blocks(st, tmp, tmp, st->nfft) == 0)
+        if (ff_blocks(st, tmp, tmp, st->nfft, 0, &moved) == 0)
             return done;
         /* good samples of the padded block that come from real input */
         keep = n + st->ngood > st->nfft ? n + st->ngood - st->nfft : 0;
         memcpy((char *)outbuf + samp * done, tmp, samp * keep);
         return done + keep;
     }
-    const size_t nwritten = ff_blocks(st, inbuf, outbuf, ntot);
+    const size_t nwritten = ff_blocks(st, inbuf, outbuf, ntot, 1, &moved);
     *offset = ntot - nwritten;
-    memmove(inbuf, (const char *)inbuf + samp * nwritten, samp * *offset);
+    if (!moved)
+        memmove(inbuf, (const char *)inbuf + samp * nwritten, samp * *offset);
     return nwritten;
 }
 

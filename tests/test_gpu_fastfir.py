@@ -129,3 +129,38 @@ def test_device_buffers_one_call():
     want = np.convolve(x.astype(np.float64), h.astype(np.float64), mode="valid")
     assert w == (x.shape[0] - ff.nfft) // ff.ngood * ff.ngood + ff.ngood
     assert rel_l2(yd[:w].cpu().numpy(), want[:w]) <= bound(h, x, ff.nfft, False, want)
+
+
+@pytest.mark.parametrize("nh,nfft,extra", [(1, 256, 0), (40, 256, 3), (200, 512, 311), (1000, 0, 1048), (1000, 0, 6000),
+                                           (1500, 2048, 1), (5000, 8192, 3000)])
+@pytest.mark.parametrize("real", [True, False])
+def test_device_stream_tail(nh, nfft, extra, real):
+    """Device buffers filtered in two calls: the GPU's own block length differs from the
+    plan's, its last block is part empty, and the samples left over are at the front of
+    the input after each call (kiss_fastfir.c:218-239), whatever their number."""
+    import torch
+    lib = kissfft_amd.load("float")
+    rng = np.random.default_rng(nh + extra)
+    shape = (lambda n: (n,)) if real else (lambda n: (n, 2))
+    h = rng.standard_normal(shape(nh)).astype(np.float32)
+    ff = lib.fastfir_alloc(h, real=real, nfft=nfft)
+    n1 = ff.nfft + 5 * ff.ngood + extra % ff.ngood
+    x = rng.standard_normal(shape(2 * n1)).astype(np.float32)
+    xb = torch.zeros(shape(n1 + ff.nfft), device="cuda")
+    yb = torch.full(shape(n1 + ff.nfft), 7.0, device="cuda")
+    done, used = [], 0
+    for k in range(2):
+        print("case fir tail", nh, ff.nfft, real, k, flush=True)
+        xb[ff.offset:ff.offset + n1] = torch.from_numpy(x[k * n1:(k + 1) * n1]).cuda()
+        torch.cuda.synchronize()
+        w = ff.filter(xb, yb, n1)
+        torch.cuda.synchronize()
+        done.append(yb[:w].cpu().numpy())
+        assert (yb[w:] == 7.0).all()  # nothing beyond the good samples is written
+        used += w
+        assert ff.offset == (k + 1) * n1 - used
+        np.testing.assert_array_equal(xb[:ff.offset].cpu().numpy(), x[used:used + ff.offset])
+    y = np.concatenate(done)
+    c = (lambda v: v.astype(np.float64)) if real else (lambda v: v[:, 0] + 1j * v[:, 1].astype(np.float64))
+    want = np.convolve(c(x), c(h), mode="valid")[:used]
+    assert rel_l2(c(y), want) <= 1e-6
