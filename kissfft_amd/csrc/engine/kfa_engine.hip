@@ -1093,6 +1093,8 @@ static int launch_rtile(const TileChoice &tc, RealTileArgs a, long long howmany,
 struct BlueChoice {
     const BlueVariant *v = nullptr;
     DevBuf mem_f, mem_i, mem_chirp, mem_bfft;
+    const BlueVariant *vf = nullptr;  // in a multi-batch (null: v there too), with its stage tables
+    DevBuf fmem_f, fmem_i;
 };
 
 // In-place radix-2 FFT in FP64 (forward: exp(-2*pi*i*j*k/M)), M a power of two.
@@ -1127,7 +1129,8 @@ static void fft_pow2_f64(std::vector<double> &re, std::vector<double> &im)
 }
 
 // The Bluestein variant and tables for a float plan (v == nullptr when the plan has no
-// prime factor above 16 or no registered convolution length fits), decided once per plan.
+// prime factor above 16, above 2048 points none above 50, or no registered convolution
+// length fits), decided once per plan.
 static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
 {
     static const std::shared_ptr<const BlueChoice> none = std::make_shared<const BlueChoice>();
@@ -1137,7 +1140,11 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
     int pmax = 0;
     for (int p : P.radix)
         pmax = std::max(pmax, p);
-    if (pmax <= 16)
+    // Above 2048 points the general kernel's direct sums over a factor up to 50 are the more
+    // exact (6800 = 2^4 5^2 17: 1.41e-7 rel-L2 against Bluestein's 1.84e-7; 5002 = 2 41 61
+    // 1.96e-7 against 1.65e-7, 4093 1.15e-6 against 1.90e-7), and those of 17 .. 31 have
+    // compiled rows.
+    if (pmax <= (P.n > 2048 ? 50 : 16))
         return 0;
     std::lock_guard<std::mutex> g(P.mu);
     if (P.blue_decided) {
@@ -1149,9 +1156,12 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
     auto bc = std::make_shared<BlueChoice>();
     const long long n = P.n;
     for (const BlueVariant &v : blue_registry())
-        if (v.M >= 2 * n - 1 && (!bc->v || v.M < bc->v->M))
+        if (!v.fused && v.M >= 2 * n - 1 && (!bc->v || v.M < bc->v->M))
             bc->v = &v;
     if (bc->v) {
+        for (const BlueVariant &v : blue_registry())
+            if (v.fused && v.M == bc->v->M)
+                bc->vf = &v;
         const int M = bc->v->M;
         const double pi = 3.14159265358979323846264338327;
         const double sg = P.inverse ? 1.0 : -1.0;
@@ -1183,9 +1193,13 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
         const std::vector<unsigned char> tf = float_twiddles(M, 0, M, 1), ti = float_twiddles(M, 1, M, 1);
         int rc;
         RelaxCapture relax;
-        if ((rc = make_stage_table_raw(tf.data(), KFA_F32, M, bc->v->radices, bc->v->tw_pad, 0, bc->mem_f)) ||
-            (rc = make_stage_table_raw(ti.data(), KFA_F32, M, {bc->v->radices.rbegin(), bc->v->radices.rend()},
-                                       bc->v->tw_pad, 0, bc->mem_i)) ||
+        auto stage_tables = [&](const BlueVariant &v, DevBuf &f, DevBuf &i) {
+            const int e = make_stage_table_raw(tf.data(), KFA_F32, M, v.radices, v.tw_pad, 0, f);
+            return e ? e : make_stage_table_raw(ti.data(), KFA_F32, M, {v.radices.rbegin(), v.radices.rend()},
+                                                v.tw_pad, 0, i);
+        };
+        if ((rc = stage_tables(*bc->v, bc->mem_f, bc->mem_i)) ||
+            (bc->vf && (rc = stage_tables(*bc->vf, bc->fmem_f, bc->fmem_i))) ||
             (rc = dev_upload(hw.data(), hw.size() * 4, bc->mem_chirp)) ||
             (rc = dev_upload(hb.data(), hb.size() * 4, bc->mem_bfft)))
             return rc;
@@ -1210,7 +1224,11 @@ static void blue_args(const BlueChoice &bc, int n, BlueArgs &b)
 const BlueVariant *blue_fill(const BlueChoice &bc, int n, BlueArgs &b)
 {
     blue_args(bc, n, b);
-    return bc.v;
+    if (!bc.vf)
+        return bc.v;
+    b.stw_f = bc.fmem_f.get();
+    b.stw_i = bc.fmem_i.get();
+    return bc.vf;
 }
 
 // Whether float plan P runs Bluestein's kernel; its tables are built now rather than at
@@ -1235,9 +1253,9 @@ int blue_launch(DevPlan &P, BlueArgs &b, hipStream_t s)
         return rc;
     if (!bc->v)
         return fail(-2, "no Bluestein kernel for n=%d", P.n);
-    blue_args(*bc, P.n, b);
+    const BlueVariant *v = blue_fill(*bc, P.n, b);
     ++g_launches;
-    return bc->v->launch(b, s) ? fail(-3, "Bluestein kernel launch failed") : 0;
+    return v->launch(b, s) ? fail(-3, "Bluestein kernel launch failed") : 0;
 }
 
 // The plane variant for A x B planes (float) on the current device, or v == nullptr:

@@ -88,6 +88,8 @@ struct BlueVariant {
     size_t lds;
     const char *name;
     int (*launch)(const BlueArgs &, hipStream_t);
+    bool fused;  // only in a multi-batch (kfa_multi.hip: members of its fused launch), where it
+                 // replaces the length's other variant
 };
 
 const std::vector<BlueVariant> &blue_registry();

@@ -217,7 +217,8 @@ int blue_prepare(DevPlan &P, bool *applies, std::shared_ptr<const BlueChoice> *k
 // one Bluestein launch for plan P; b carries buffers, segments, counts and distances
 struct BlueArgs;
 int blue_launch(DevPlan &P, BlueArgs &b, hipStream_t s);
-// fills b's tables from choice bc (plan length n) and returns the variant that runs it
+// fills b's tables from choice bc (plan length n) for an item group of a multi-batch (fused
+// launch or not: both round alike) and returns the variant that runs it there
 struct BlueVariant;
 const BlueVariant *blue_fill(const BlueChoice &bc, int n, BlueArgs &b);
 

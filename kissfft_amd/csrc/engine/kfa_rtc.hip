@@ -4,7 +4,7 @@
 // k_fast (kfa_fast.hpp) for the lengths of the reference's workloads.  Any other length
 // whose line fits one LDS line and whose radices are 2, 3, 4 or 5 (kf_factor's schedule,
 // kiss_fft.c:306-328; float may also regroup the powers of two into radix 8 / 16, and
-// takes the odd radices 7, 11 and 13 as well) gets the same kernel compiled at run time, on
+// takes the odd radices 7, 11 and 13 as well, above 2048 points those up to 31) gets the same kernel compiled at run time, on
 // first use, with the HIP runtime compiler:
 //   * fixed point keeps the plan's own radix schedule (its rounding is part of the result);
 //     float takes a schedule of large radices (16s, then 8 / 4 / 2, then 5s and 3s, then
@@ -394,6 +394,7 @@ std::vector<TileShape> tile_shapes(int n, const std::vector<int> &rad, int type,
 // the tile through LDS for little work).
 std::vector<int> float_schedule(int n, bool tile)
 {
+    const int pmax = !tile && n > 2048 ? 31 : 13;
     int a = 0, b = 0, c = 0;
     while (n % 2 == 0) {
         n /= 2;
@@ -408,8 +409,9 @@ std::vector<int> float_schedule(int n, bool tile)
         ++c;
     }
     std::vector<int> g;
-    for (int p : {7, 11, 13})
-        while (n % p == 0) {
+    // (rows above 2048 points also 17 .. 31: shorter ones run Bluestein's kernel)
+    for (int p : {7, 11, 13, 17, 19, 23, 29, 31})
+        while (p <= pmax && n % p == 0) {
             n /= p;
             g.push_back(p);
         }
@@ -571,7 +573,7 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
         return 0;  // one-stage schedules read and write HBM in one stage (not in-place safe)
     for (int p : rad)
         if (!(p == 2 || p == 3 || p == 4 || p == 5 || p == 7 || p == 11 || p == 13 ||
-              (P.type == KFA_F32 && (p == 8 || p == 16))))
+              (P.type == KFA_F32 && (p == 8 || p == 16 || (p >= 17 && p <= 31)))))
             return 0;
     const int n = P.n;
     const int pmin = *std::min_element(rad.begin(), rad.end());

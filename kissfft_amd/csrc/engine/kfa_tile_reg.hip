@@ -279,7 +279,7 @@ static int launch_blue(const BlueArgs &a, hipStream_t s)
 }
 
 template <int T, int LPB, int... R>
-static void add_blue(std::vector<BlueVariant> &v, const char *name)
+static void add_blue(std::vector<BlueVariant> &v, const char *name, bool fused = false)
 {
     typedef Radices<2, R...> RS;
     static_assert(T * LPB <= 1024, "workgroup too large");
@@ -292,6 +292,7 @@ static void add_blue(std::vector<BlueVariant> &v, const char *name)
     f.lds = (size_t)LPB * conv_slots(RS::N()) * 8;
     f.name = name;
     f.launch = &launch_blue<T, LPB, RS>;
+    f.fused = fused;
     v.push_back(f);
 }
 
@@ -303,9 +304,15 @@ const std::vector<BlueVariant> &blue_registry()
         add_blue<8, 8, 8, 16>(*v, "blue128_816_t8x8");
         add_blue<16, 4, 16, 16>(*v, "blue256_1616_t16x4");
         add_blue<64, 2, 8, 8, 8>(*v, "blue512_888_t64x2");
-        add_blue<64, 2, 16, 16, 4>(*v, "blue1024_16164_t64x2");
-        add_blue<128, 2, 16, 16, 8>(*v, "blue2048_16168_t128x2");
-        add_blue<256, 1, 16, 16, 16>(*v, "blue4096_161616_t256");
+        add_blue<128, 2, 8, 8, 4, 4>(*v, "blue1024_8844_t128x2");
+        // c2c 1009 x4096 27.4 us, 32.2 with 128 threads a line, 30.9 with 16, 16, 8 at 128; but
+        // 64 uneven batches in one fused launch 45.1, 45.1 and 43.4 us
+        add_blue<256, 1, 8, 8, 8, 4>(*v, "blue2048_8884_t256");
+        add_blue<128, 2, 16, 16, 8>(*v, "blue2048_16168_t128x2", true);
+        add_blue<512, 1, 8, 8, 8, 8>(*v, "blue4096_8888_t512");
+        // lengths above 2048: 4093 x8 10.7 ms -> 16 us, 5002 x8 319 -> 23 us against the general kernel
+        add_blue<512, 1, 8, 8, 8, 4, 4>(*v, "blue8192_88844_t512");
+        add_blue<1024, 1, 8, 8, 8, 8, 4>(*v, "blue16384_88884_t1024");
         return v;
     }();
     return *reg;

@@ -131,3 +131,18 @@ def test_short_lengths_compiled(dtype, monkeypatch, capfd):
             assert rel_l2(cplx(X), np.fft.rfft(x.astype(np.float64), axis=-1)) <= ABS_FLOAT_BOUND, n
     err = capfd.readouterr().err
     assert "fast variant rtc_c2c60" in err and "fast variant rtc_r2c49" in err, err[-2000:]
+
+
+@pytest.mark.parametrize("n", [2049, 2176, 2201, 3077, 3162, 3751, 4096 + 1, 4099, 4301, 5002, 6800, 8167, 8191])
+def test_float_lengths_above_2048_with_large_primes(n):
+    """Lengths with prime factors above 13 past 2048 points: factors of 17 .. 31 on rows
+    compiled at run time, above 50 on Bluestein's kernel (8192 and 16384 points)."""
+    lib = kissfft_amd.load("float")
+    x = np.random.default_rng(n).uniform(-1, 1, (3, n, 2)).astype(np.float32)
+    for inv in (False, True):
+        y = np.zeros_like(x)
+        lib.fft_batch(lib.fft_alloc(n, inv), x, y, 3, n, n)
+        z = x[..., 0] + 1j * x[..., 1].astype(np.float64)
+        want = np.fft.ifft(z, axis=-1) * n if inv else np.fft.fft(z, axis=-1)
+        got = y[..., 0] + 1j * y[..., 1].astype(np.float64)
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want), (n, inv)
