@@ -1769,9 +1769,9 @@ static long long balanced_chunk(long long howmany, long long max_chunk)
 
 size_t multipass_bytes_per_transform(DevPlan &P, int fk)
 {
-    if (P.single)
-        return 0;
     const size_t cb = cpx_bytes(P.type);
+    if (P.single)  // (real rows on Bluestein's kernel: the temporary of the split / merge pass)
+        return fk != FK_C2C && blue_real_rows(P) ? cb * (size_t)(P.n + 16) + 256 : 0;
     const size_t c2c = (P.type == KFA_F32 ? 8 : cb) * (size_t)P.n + 256;  // the four-step temporary
     if (fk == FK_C2C)
         return c2c;
@@ -2225,7 +2225,19 @@ int prepare_multipass(DevPlan &P, int fk, hipStream_t s)
     return rc;
 }
 
-// Real rows whose half length needs the multi-pass complex transform.  Float lengths with
+// Real rows with a half length of at most one line that has a prime factor above 50: the
+// complex transform on Bluestein's kernel and the split (merge) as a pass of its own
+// instead of direct sums over the factor (80 x 1126 x34 there and back 1461 -> 62 us).  Smaller
+// factors have compiled rows (to 31) or the more exact direct sums.
+bool blue_real_rows(const DevPlan &P)
+{
+    int pmax = 0;
+    for (int p : P.radix)
+        pmax = std::max(pmax, p);
+    return P.type == KFA_F32 && P.single && pmax > 50 && env_flag("KISSFFT_AMD_BLUESTEIN", true);
+}
+
+// Real rows whose half length needs the multi-pass complex transform (or Bluestein's kernel).  Float lengths with
 // a registered four-step split take the two fused passes of run_real_fourstep; otherwise
 // the complex pass runs into a temporary (nc values per line) and the split (forward) or
 // merge (inverse) runs as its own HBM pass on that temporary.
@@ -2304,6 +2316,8 @@ int run_real_rows(DevPlan &H, const RealTables &R, int inverse, const void *in, 
         ++g_launches;
         return fast_launch(*fc->v, a, s) ? fail(-3, "fast kernel launch failed") : 0;
     }
+    if (blue_real_rows(H))
+        return run_real_multipass(H, R, inverse, in, in_hi, out, out_hi, howmany, s);
     LineLaunch ll{};
     ll.in = in;
     ll.out = out;

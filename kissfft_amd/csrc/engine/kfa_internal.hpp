@@ -167,8 +167,8 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
 // bits), or null: radix outside 2-5, 7, 11, 13 (float also 8, 16), no shape without
 // scratch, or the runtime compiler off
 const TileVariant *rtc_tile(int type, const std::vector<int> &radices, int inverse, int tm);
-// the float schedule of length n (empty: a factor above 13), for a row or a tile kernel
-std::vector<int> float_schedule(int n, bool tile = false);
+// the float schedule of length n (empty: a factor above pmax), for a row or a tile kernel
+std::vector<int> float_schedule(int n, bool tile = false, int pmax = 13);
 // the persisted table of tuned choices (kfa_rtc.hip): key of a decision, lookup, store
 std::string tuned_key(const DevPlan &P, int kind, long long tune_lines);
 bool tuned_lookup(const std::string &key, std::string &name);
@@ -211,6 +211,9 @@ std::vector<unsigned char> float_twiddles(long long n, int inverse, long long co
 int make_stage_table_raw(const unsigned char *h_tw, int type, long long n, const std::vector<int> &rad, int pad,
                          int fmt, DevBuf &out, long long m0 = 1);
 
+// whether real rows of half length P.n run on Bluestein's kernel (the split / merge as a
+// pass of its own)
+bool blue_real_rows(const DevPlan &P);
 // whether a float plan runs Bluestein's kernel (its tables built on return; the caller may
 // hold them in `keep`)
 int blue_prepare(DevPlan &P, bool *applies, std::shared_ptr<const BlueChoice> *keep = nullptr);

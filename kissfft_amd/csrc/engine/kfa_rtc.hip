@@ -4,7 +4,7 @@
 // k_fast (kfa_fast.hpp) for the lengths of the reference's workloads.  Any other length
 // whose line fits one LDS line and whose radices are 2, 3, 4 or 5 (kf_factor's schedule,
 // kiss_fft.c:306-328; float may also regroup the powers of two into radix 8 / 16, and
-// takes the odd radices 7, 11 and 13 as well, above 2048 points those up to 31) gets the same kernel compiled at run time, on
+// takes the odd radices 7, 11 and 13 as well, real and long rows those up to 31) gets the same kernel compiled at run time, on
 // first use, with the HIP runtime compiler:
 //   * fixed point keeps the plan's own radix schedule (its rounding is part of the result);
 //     float takes a schedule of large radices (16s, then 8 / 4 / 2, then 5s and 3s, then
@@ -387,14 +387,13 @@ std::vector<TileShape> tile_shapes(int n, const std::vector<int> &rad, int type,
 }  // namespace
 
 // float: 16s, then one 8 / 4 / 2 for the rest of the power of two, then 5s, then 3s, then
-// the generic odd radices 7, 11, 13 (kfa_fast.hpp's Dft<P>); empty for other factors.
+// the generic odd radices from 7 to pmax (kfa_fast.hpp's Dft<P>); empty for other factors.
 // tile: the odd radices first, which leaves more of the twiddles of the others exact (half of a
 // four-step split of 746496 = 864^2: 1.69e-7 rel-L2 against 1.81e-7 with the order of the rows,
 // and as fast), and 8 and 4 in the place of a 16 and a 2 (a stage of radix 2 would move
 // the tile through LDS for little work).
-std::vector<int> float_schedule(int n, bool tile)
+std::vector<int> float_schedule(int n, bool tile, int pmax)
 {
-    const int pmax = !tile && n > 2048 ? 31 : 13;
     int a = 0, b = 0, c = 0;
     while (n % 2 == 0) {
         n /= 2;
@@ -409,7 +408,6 @@ std::vector<int> float_schedule(int n, bool tile)
         ++c;
     }
     std::vector<int> g;
-    // (rows above 2048 points also 17 .. 31: shorter ones run Bluestein's kernel)
     for (int p : {7, 11, 13, 17, 19, 23, 29, 31})
         while (p <= pmax && n % p == 0) {
             n /= p;
@@ -568,7 +566,10 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
     const int min_n = mv && *mv ? atoi(mv) : 16;
     if (!env_flag("KISSFFT_AMD_RTC", true) || !P.single || P.n < std::max(2, min_n))
         return 0;
-    std::vector<int> rad = P.type == KFA_F32 ? float_schedule(P.n) : P.radix;
+    // factors of 17 .. 31: rows above 2048 points and real ones (shorter complex rows run
+    // Bluestein's kernel)
+    std::vector<int> rad =
+        P.type == KFA_F32 ? float_schedule(P.n, false, P.n > 2048 || kind != FK_C2C ? 31 : 13) : P.radix;
     if (rad.size() < 2)
         return 0;  // one-stage schedules read and write HBM in one stage (not in-place safe)
     for (int p : rad)

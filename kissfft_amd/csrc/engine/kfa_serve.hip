@@ -384,8 +384,8 @@ long long kfa_server_submit(void *srv, int kind, const kfa_cplan *cp, const kfa_
     // decide the compiled variant now, on the server's plan stream, not in the scheduler
     if (r->P->single) {
         const FastChoice *fc;
-        const int fk = kind == KFA_SERVE_R2C ? FK_R2C : kind == KFA_SERVE_C2R ? FK_C2R : FK_C2C;
-        if ((rc = choose_fast(*r->P, fk, S->plan_stream, &fc, howmany)))
+        const int row = kind == KFA_SERVE_R2C ? FK_R2C : kind == KFA_SERVE_C2R ? FK_C2R : FK_C2C;
+        if ((rc = choose_fast(*r->P, row, S->plan_stream, &fc, howmany)))
             return rc;
     }
     side_bytes(S->type, kind, nfft, howmany, r->in_bytes, r->out_bytes);
@@ -394,9 +394,9 @@ long long kfa_server_submit(void *srv, int kind, const kfa_cplan *cp, const kfa_
     r->need = (r->stage_in ? r->in_bytes : 0) + (r->stage_out ? r->out_bytes : 0);
     // multi-pass scratch: the temporaries of one chunk of transforms (the chunking of
     // multi-pass batches bounds them)
-    if (!r->P->single) {
-        const int fk = kind == KFA_SERVE_R2C ? FK_R2C : kind == KFA_SERVE_C2R ? FK_C2R : FK_C2C;
-        const size_t per = multipass_bytes_per_transform(*r->P, fk) + 1024;
+    const int fk = kind == KFA_SERVE_R2C ? FK_R2C : kind == KFA_SERVE_C2R ? FK_C2R : FK_C2C;
+    if (const size_t temp = multipass_bytes_per_transform(*r->P, fk)) {
+        const size_t per = temp + 1024;
         r->need += std::min((size_t)howmany * per, std::max(per, scratch_room()));
     }
     r->t_submit = now_s();
@@ -448,7 +448,7 @@ long long kfa_server_submit_nd(void *srv, int kind, int ndims, const int *dims, 
             return fail(-2, "server submit: real N-D requests need an even last dimension");
         if ((rc = build_cplan(&rp->half, S->dev, r->P)) || (rc = build_rtab(rp, S->dev, r->R)))
             return rc;
-        multipass |= !r->P->single;
+        multipass |= !r->P->single || blue_real_rows(*r->P);
     } else {
         r->P = r->axes[0];
     }

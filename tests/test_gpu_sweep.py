@@ -146,3 +146,24 @@ def test_float_lengths_above_2048_with_large_primes(n):
         want = np.fft.ifft(z, axis=-1) * n if inv else np.fft.fft(z, axis=-1)
         got = y[..., 0] + 1j * y[..., 1].astype(np.float64)
         assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want), (n, inv)
+
+
+@pytest.mark.parametrize("n", [2 * 53, 2 * 68, 2 * 563, 2 * 899, 2 * 1009, 2 * 2047, 2 * 3162, 2 * 4099, 2 * 8191])
+def test_float_real_rows_with_large_primes(n):
+    """Real rows whose half length has prime factors above 13: to 31 on compiled rows, above
+    50 on Bluestein's kernel with the split / merge as a pass of its own; in place too."""
+    import torch
+    lib = kissfft_amd.load("float")
+    x = np.random.default_rng(n).standard_normal((5, n)).astype(np.float32)
+    X = np.zeros((5, n // 2 + 1, 2), np.float32)
+    lib.fftr_batch(lib.fftr_alloc(n), x, X, 5, n, n // 2 + 1)
+    want = np.fft.rfft(x.astype(np.float64), axis=-1)
+    assert rel_l2(cplx(X), want) <= ABS_FLOAT_BOUND
+    z = np.zeros_like(x)
+    lib.fftri_batch(lib.fftr_alloc(n, True), X, z, 5, n // 2 + 1, n)
+    assert rel_l2(z, n * x.astype(np.float64)) <= 2 * ABS_FLOAT_BOUND
+    one = torch.zeros(n + 2, device="cuda")
+    one[:n] = torch.from_numpy(x[0]).cuda()
+    torch.cuda.synchronize()
+    lib.kiss_fftr(lib.fftr_alloc(n), one, one)
+    np.testing.assert_array_equal(one.cpu().numpy().reshape(-1, 2), X[0])
