@@ -1461,6 +1461,8 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
         fc.decided = true;
         return 0;
     }
+    if (P.n < kShortRow && lines_hint * P.n < kShortValues)
+        return 0;  // the general kernel; a larger batch may still decide
     std::vector<const FastVariant *> cand;
     for (const FastVariant &v : fast_registry()) {
         if (v.type != P.type || v.kind != kind || v.n != P.n || v.inverse != P.inverse)
@@ -2603,7 +2605,7 @@ int kfa_c2r(const kfa_rplan *pl, const void *in, long long idist, void *out, lon
 // Whether a column pass of `values` values over lines of n points is worth a kernel
 // compiled for its length on first use (a fraction of a second): any length from 16 points,
 // as for rows, and shorter ones when there is more than a handful of them.
-static bool axis_compiles(long long n, long long values) { return n >= 16 || values >= (1LL << 16); }
+static bool axis_compiles(long long n, long long values) { return n >= kShortRow || values >= kShortValues; }
 
 // One axis of an N-D array batch, dims[k] long, between device buffers (in may equal out).
 static int run_axis(DevPlan &P, const void *in, void *out, long long outer, long long inner,

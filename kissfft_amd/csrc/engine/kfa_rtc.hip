@@ -17,7 +17,9 @@
 //     $XDG_CACHE_HOME/kissfft_amd or ~/.cache/kissfft_amd), keyed by a hash of the source,
 //     the options and the device architecture; KISSFFT_AMD_RTC=0 turns the path off;
 //   * a kernel that would use scratch memory (spilled registers) is not used;
-//   * lines shorter than 16 points (KISSFFT_AMD_RTC_MIN) keep the general kernel.
+//   * complex lines shorter than 16 points (KISSFFT_AMD_RTC_MIN) keep the general kernel, and so
+//     do real rows of a half length below 4; half lengths of 4 .. 15 are compiled when there
+//     is a batch of them (real 15x90x16 x1277 both ways: Q15 518 -> 218 us, float 585 -> 329).
 // The tile kernel k_tile (kfa_tile.hpp) is compiled the same way for the strided lines of
 // N-D axes without a built-in tile, all three scalar kinds, in one shape chosen by rule
 // (tile_shapes), so an axis costs one compilation per direction.  Against the general line
@@ -559,19 +561,20 @@ int fast_launch(const FastVariant &v, const FastArgs &a, hipStream_t s)
 // off, the length has another radix, or nothing compiles).
 int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> &out)
 {
-    // lines from 16 points (KISSFFT_AMD_RTC_MIN): batches of short lines run 3-8 times
+    // lines from 16 points, real half lengths from 4 (kShortRow; KISSFFT_AMD_RTC_MIN): batches
+    // of short lines run 3-8 times
     // faster compiled than on the general kernel (2^29 bytes per side: Q15 120 points
     // 2.88 against 0.37 TB/s, float 60 points 3.96 against 0.78)
     const char *mv = getenv("KISSFFT_AMD_RTC_MIN");
-    const int min_n = mv && *mv ? atoi(mv) : 16;
+    const int min_n = mv && *mv ? atoi(mv) : kind == FK_C2C ? kShortRow : 4;
     if (!env_flag("KISSFFT_AMD_RTC", true) || !P.single || P.n < std::max(2, min_n))
         return 0;
     // factors of 17 .. 31: rows above 2048 points and real ones (shorter complex rows run
     // Bluestein's kernel)
     std::vector<int> rad =
         P.type == KFA_F32 ? float_schedule(P.n, false, P.n > 2048 || kind != FK_C2C ? 31 : 13) : P.radix;
-    if (rad.size() < 2)
-        return 0;  // one-stage schedules read and write HBM in one stage (not in-place safe)
+    if (rad.empty() || (rad.size() < 2 && kind == FK_C2C))
+        return 0;  // one-stage complex rows read and write HBM in one stage (not in-place safe)
     for (int p : rad)
         if (!(p == 2 || p == 3 || p == 4 || p == 5 || p == 7 || p == 11 || p == 13 ||
               (P.type == KFA_F32 && (p == 8 || p == 16 || (p >= 17 && p <= 31)))))

@@ -181,3 +181,34 @@ def test_real_direction_misuse_writes_nothing():
     assert np.all(out == 5.0)
     with pytest.raises(kissfft_amd.KissFFTError):
         lib.fftr_batch(inv_cfg, x, out, 1, 64, 33)
+
+
+@pytest.mark.parametrize("dtype", ["float", "int16_t", "int32_t"])
+@pytest.mark.parametrize("n", [8, 10, 12, 16, 18, 22, 24, 26, 28, 30])
+def test_batches_of_short_real_rows(dtype, n, monkeypatch, capfd):
+    """Real rows of half lengths 4 .. 15 (one or two stages) in a batch large enough to be
+    compiled for, and a few of them on the general kernel: both directions."""
+    lib = kissfft_amd.load(dtype)
+    monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    lib.L.kiss_fft_cleanup()
+    rng = np.random.default_rng(n)
+    b = 70001 * 2 // n
+    x = rng.standard_normal((b, n)).astype(np.float32) if dtype == "float" else \
+        rng.integers(-(1 << 14), 1 << 14, (b, n)).astype(lib.scalar)
+    for k in (3, b):
+        X = np.zeros((k, n // 2 + 1, 2), lib.scalar)
+        z = np.zeros((k, n), lib.scalar)
+        lib.fftr_batch(lib.fftr_alloc(n), x[:k], X, k, n, n // 2 + 1)
+        lib.fftri_batch(lib.fftr_alloc(n, True), X, z, k, n // 2 + 1, n)
+        if dtype == "float":
+            want = np.fft.rfft(x[:k].astype(np.float64), axis=-1)
+            got = X[..., 0] + 1j * X[..., 1].astype(np.float64)
+            assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
+            assert np.linalg.norm(z - n * x[:k].astype(np.float64)) <= 2e-6 * n * np.linalg.norm(x[:k])
+        else:
+            O = Oracle(dtype)
+            np.testing.assert_array_equal(X, O.fftr(x[:k]))
+            np.testing.assert_array_equal(z, O.fftri(X, n))
+    err = capfd.readouterr().err
+    if n // 2 != 11 or dtype == "float":
+        assert f"rtc_r2c{n // 2}" in err and f"rtc_c2r{n // 2}" in err
