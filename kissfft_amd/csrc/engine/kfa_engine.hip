@@ -723,6 +723,8 @@ struct TileCache {
     std::map<std::tuple<int, long long, int, int>, BufPair> rs;                           // dev, nc, n, inv
     // dev, A, B, inv, slab, small (see plane_choice)
     std::map<std::tuple<int, int, int, int, int, int>, std::shared_ptr<const PlaneChoice>> plane;
+    // dev, type, A, B, inv (see fixed_plane)
+    std::map<std::tuple<int, int, int, int, int>, std::shared_ptr<const PlaneChoice>> fplane;
 };
 
 static TileCache &tile_cache()
@@ -1266,8 +1268,9 @@ int blue_launch(DevPlan &P, BlueArgs &b, hipStream_t s)
 // and per size class (up to 128 MiB per side, which the 256 MB Infinity Cache holds
 // between passes, or more: the ranking differs between the two).
 // (KISSFFT_AMD_PLANE=0 turns the plane pass off, KISSFFT_AMD_TILE forces a variant by name.)
+// may_compile: contiguous planes without a built-in variant may take a runtime-compiled one.
 static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long nsub, long long planes,
-                        hipStream_t s, std::shared_ptr<const PlaneChoice> &out)
+                        bool may_compile, hipStream_t s, std::shared_ptr<const PlaneChoice> &out)
 {
     int dev;
     int rc = current_device(&dev);
@@ -1298,6 +1301,17 @@ static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long 
                 cand.push_back(c);
             }
     }
+    if (cand.empty() && !slab && env_flag("KISSFFT_AMD_FAST", true) && env_flag("KISSFFT_AMD_PLANE", true)) {
+        if (!may_compile || stream_capturing(s)) {
+            out = std::make_shared<const PlaneChoice>();
+            return 0;  // the choice stays open
+        }
+        const std::vector<int> ra = float_schedule(A, true), rb = float_schedule(B, true);
+        if (const PlaneVariant *v = rtc_plane(KFA_F32, ra, rb, inverse)) {
+            cand.push_back(std::make_shared<PlaneChoice>());
+            cand.back()->v = v;
+        }
+    }
     for (auto &c : cand) {
         const std::vector<unsigned char> ta = float_twiddles(A, inverse, A, 1), tb = float_twiddles(B, inverse, B, 1);
         if ((rc = make_stage_table_raw(ta.data(), KFA_F32, A, c->v->rad_a, c->v->tw_pad, 0, c->mem_a)) ||
@@ -1326,7 +1340,7 @@ static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long 
                 const PlaneArgs pa =
                     slab ? PlaneArgs{bin.p, bout.p, cand[i]->stw_a, cand[i]->stw_b, tp, rs, sub, (long long)A * rs, B}
                          : plane_args(bin.p, bout.p, cand[i]->stw_a, cand[i]->stw_b, tp, A, B);
-                return cand[i]->v->launch(pa, ts);
+                return plane_launch(*cand[i]->v, pa, ts);
             }, what);
             break;
         }
@@ -1342,6 +1356,56 @@ static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long 
 // Longest half of a four-step split that a tile is compiled for: 8 of its lines (rows of 64
 // bytes) fit a workgroup.
 constexpr long long kTileLongest = 2048;
+
+// Whether `planes` contiguous planes of `values` values run as planes compiled at run time: one
+// pass instead of two, but one workgroup per plane.  Few planes leave most of the device idle
+// where two axis passes would fill it, unless the launches are all that counts; planes that
+// leave a CU room for fewer than four wait on their own barriers (against two passes, us:
+// float 80x60 x64 9.7 / 9.5, x128 9.6 / 11.8, x256 10.6 / 16.5, x1300 38 / 38; 100x45 x1000
+// 25 / 34; 30x40 x1 6.2 / 9.7; Q15 80x60 x1300 27 / 35; but 20x300 x600 33 / 29, Q15 64x96x120
+// x16 83 / 77).
+static bool plane_pays(long long planes, long long values)
+{
+    return values <= 2048 || (planes >= 128 && values <= 5000);
+}
+
+// The compiled plane kernel for the last two axes of a fixed-point N-D transform, columns of
+// plan PA and rows of plan PB (v == nullptr: none), decided once per pair of plans' lengths.
+static int fixed_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, std::shared_ptr<const PlaneChoice> &out)
+{
+    int dev;
+    int rc = current_device(&dev);
+    if (rc)
+        return rc;
+    auto &C = tile_cache();
+    std::lock_guard<std::mutex> g(C.mu);
+    const auto key = std::make_tuple(dev, PA.type, PA.n, PB.n, PA.inverse);
+    auto it = C.fplane.find(key);
+    if (it != C.fplane.end()) {
+        out = it->second;
+        return 0;
+    }
+    if (thread_noalloc())
+        return noalloc_refuse("a plane kernel's tables");
+    auto pc = std::make_shared<PlaneChoice>();
+    out = pc;
+    if (stream_capturing(s))
+        return 0;  // the choice stays open
+    if (PA.single && PB.single && env_flag("KISSFFT_AMD_FAST", true) && env_flag("KISSFFT_AMD_PLANE", true))
+        pc->v = rtc_plane(PA.type, PA.radix, PB.radix, PA.inverse);
+    if (pc->v) {
+        if ((rc = make_stage_table_raw(PA.h_tw.data(), PA.type, PA.n, PA.radix, 2, pc->v->tw_fmt, pc->mem_a)) ||
+            (rc = make_stage_table_raw(PB.h_tw.data(), PB.type, PB.n, PB.radix, 2, pc->v->tw_fmt, pc->mem_b)))
+            return rc;
+        pc->stw_a = pc->mem_a.get();
+        pc->stw_b = pc->mem_b.get();
+        if (env_flag("KISSFFT_AMD_VERBOSE", false))
+            fprintf(stderr, "[kissfft_amd] plane %dx%d inverse=%d type=%d: %s\n", PA.n, PB.n, PA.inverse, PA.type,
+                    pc->v->name);
+    }
+    C.fplane[key] = pc;
+    return 0;
+}
 
 // Float four-step (Bailey) for n = N1*N2 with both halves tile lengths (built in, or
 // compiled at run time), decided once per plan: pass 1 transforms the N1 columns (length N2, stride N1) and
@@ -2690,7 +2754,11 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
         std::vector<int> order{ndims - 2};
         for (int k = 0; k < ndims - 2; ++k)
             order.push_back(k);
-        for (int k : order) {
+        // (built-in variants of any of them first, then a compiled plane of the last two axes)
+        order.push_back(ndims - 2);
+        for (size_t i = 0; i < order.size() && paired < 0; ++i) {
+            const int k = order[i];
+            const bool compile = i + 1 == order.size();
             long long rs = 1;  // in-plane offsets are 32-bit
             for (int j = k + 1; j < ndims; ++j)
                 rs *= dims[j];
@@ -2700,12 +2768,13 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
             for (int j = k + 1; j < ndims - 1; ++j)
                 mid *= dims[j];
             const long long planes = howmany * (total / ((long long)dims[k] * nb));
-            if ((rc = plane_choice(dims[k], nb, P[ndims - 1]->inverse, k != ndims - 2, (int)rs, mid, planes, s, pc)))
-                return rc;
-            if (pc->v && (k == ndims - 2 || pc->v->slab)) {
-                paired = k;
+            if (compile && !plane_pays(planes, (long long)dims[k] * nb))
                 break;
-            }
+            if ((rc = plane_choice(dims[k], nb, P[ndims - 1]->inverse, k != ndims - 2, (int)rs, mid, planes, compile, s,
+                                   pc)))
+                return rc;
+            if (pc->v && (k == ndims - 2 || pc->v->slab))
+                paired = k;
         }
         if (paired >= 0) {
             long long rs = 1, mid = 1;  // row stride; planes per value of the axes before `paired`
@@ -2716,12 +2785,26 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
             const long long planes = howmany * (total / ((long long)dims[paired] * nb));
             const PlaneArgs pa{in, out, pc->stw_a, pc->stw_b, planes, (int)rs, mid, (long long)dims[paired] * rs, nb};
             ++g_launches;
-            if (pc->v->launch(pa, s))
+            if (plane_launch(*pc->v, pa, s))
                 return fail(-3, "plane kernel launch failed");
             src = out;
         }
     }
+    // fixed point: the axes in order, the last two in one pass where a plane of them is compiled
+    std::shared_ptr<const PlaneChoice> fp;
+    if (ndims >= 2 && P[0]->type != KFA_F32) {
+        const long long values = (long long)dims[ndims - 2] * dims[ndims - 1];
+        if (plane_pays(howmany * (total / values), values) &&
+            (rc = fixed_plane(*P[ndims - 2], *P[ndims - 1], s, fp)))
+            return rc;
+    }
     for (int k = 0; k < ndims && rc == 0; ++k) {
+        if (fp && fp->v && k == ndims - 2) {
+            const long long A = dims[k], B = dims[k + 1];
+            ++g_launches;
+            return plane_launch(*fp->v, plane_args(src, out, fp->stw_a, fp->stw_b, howmany * (total / (A * B)), A, B), s)
+                       ? fail(-3, "plane kernel launch failed") : 0;
+        }
         inner /= dims[k];
         if (paired < 0 || (k != paired && k != ndims - 1)) {
             rc = run_axis(*P[k], src, out, outer, inner, s);
@@ -2897,6 +2980,7 @@ void kfa_cleanup(void)
         auto &T = tile_cache();
         std::lock_guard<std::mutex> gt(T.mu);
         T.plane.clear();
+        T.fplane.clear();
         T.choice.clear();
         T.fs.clear();
         T.rs.clear();

@@ -120,20 +120,25 @@ namespace kfa {
 
 struct PlaneArgs;
 
-// Plane variants (kfa_plane.hpp): float, the last two axes A x B of an N-D transform in
-// one pass, one direction.
+// Plane variants (kfa_plane.hpp): the last two axes A x B of an N-D transform in one pass,
+// one direction.  Built in: float; compiled at run time (kfa_rtc.hip): any scalar kind.
 struct PlaneVariant {
+    int type = 0;  // KFA_F32 / KFA_Q15 / KFA_Q31
     int A, B;
     int inverse;
     int TA, TB, NTH;  // threads per column, per row, per workgroup
     std::vector<int> rad_a, rad_b;
     int tw_pad;
+    int tw_fmt = 0;  // see FastVariant
     size_t lds;
+    const void *rtc = nullptr;  // runtime-compiled variant: launched through it
     bool slab;    // also runs slabs of two non-adjacent axes (PlaneArgs rs / nsub / po / pi)
     const char *name;
     int (*launch)(const PlaneArgs &, hipStream_t);
 };
 
 const std::vector<PlaneVariant> &plane_registry();
+// launches variant v (built in or runtime-compiled)
+int plane_launch(const PlaneVariant &v, const PlaneArgs &a, hipStream_t s);
 
 }  // namespace kfa

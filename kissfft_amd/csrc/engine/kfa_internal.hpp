@@ -170,6 +170,9 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
 // bits), or null: radix outside 2-5, 7, 11, 13 (float also 8, 16), no shape without
 // scratch, or the runtime compiler off
 const TileVariant *rtc_tile(int type, const std::vector<int> &radices, int inverse, int tm);
+// the runtime-compiled plane kernel (kfa_plane.hpp) of column schedule ra and row schedule rb,
+// or null (radices as rtc_tile, fixed point 2-5 only; a plane of at most 64 KiB with its tables)
+const PlaneVariant *rtc_plane(int type, const std::vector<int> &ra, const std::vector<int> &rb, int inverse);
 // the float schedule of length n (empty: a factor above pmax), for a row or a tile kernel
 std::vector<int> float_schedule(int n, bool tile = false, int pmax = 13);
 // the persisted table of tuned choices (kfa_rtc.hip): key of a decision, lookup, store

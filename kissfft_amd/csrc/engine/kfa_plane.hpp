@@ -37,6 +37,9 @@ struct PlaneArgs {
     long long pi;
 };
 
+// slots of the plane in LDS, the tables behind it 16-byte aligned
+constexpr int plane_slots(int n, int per16) { return (n + per16 - 1) / per16 * per16; }
+
 // the arguments of contiguous A x B planes
 inline PlaneArgs plane_args(const void *in, void *out, const void *stw_a, const void *stw_b, long long planes,
                             long long A, long long B)
@@ -44,10 +47,10 @@ inline PlaneArgs plane_args(const void *in, void *out, const void *stw_a, const 
     return PlaneArgs{in, out, stw_a, stw_b, planes, (int)B, 1, A * B, 0};
 }
 
-template <bool INV, int T, class RS, int ES, int S>
-__device__ __forceinline__ void plane_stage(F32::store2 *lb, const F32::store2 *stw, int t, bool active)
+template <class A, bool INV, int T, class RS, int ES, int S>
+__device__ __forceinline__ void plane_stage(typename A::store2 *lb, const typename A::store2 *stw, int t, bool active)
 {
-    typedef FastStage<F32, INV, T, RS, S, false> F;
+    typedef FastStage<A, INV, T, RS, S, false> F;
     typename F::C v[F::J][F::p];
     if (active)
         F::template gather<false>(v, lb, ES, t, true);
@@ -59,11 +62,11 @@ __device__ __forceinline__ void plane_stage(F32::store2 *lb, const F32::store2 *
     line_sync<T>();
 }
 
-template <bool INV, int T, class RS, int ES, int... S>
-__device__ __forceinline__ void plane_stages(std::integer_sequence<int, S...>, F32::store2 *lb,
-                                             const F32::store2 *stw, int t, bool active)
+template <class A, bool INV, int T, class RS, int ES, int... S>
+__device__ __forceinline__ void plane_stages(std::integer_sequence<int, S...>, typename A::store2 *lb,
+                                             const typename A::store2 *stw, int t, bool active)
 {
-    (plane_stage<INV, T, RS, ES, S>(lb, stw, t, active), ...);
+    (plane_stage<A, INV, T, RS, ES, S>(lb, stw, t, active), ...);
 }
 
 // Persistent: workgroup g takes planes g, g + G, g + 2G, ... (G = gridDim.x).  PF: the
@@ -74,10 +77,13 @@ __device__ __forceinline__ void plane_stages(std::integer_sequence<int, S...>, F
 // The stage tables are copied to LDS once, so that the stages issue no global loads (a
 // global load's wait would also wait for the prefetch).
 // SLAB: planes addressed through rs / nsub / po / pi (else contiguous A x B planes, p * A * B)
-template <bool INV, int TA, int TB, int NTH, class RA, class RB, bool SLAB, bool PF>
+// Fixed point transforms the columns before the rows, kiss_fftnd's order of the axes (each
+// axis rounds); float the rows first.
+template <class X, bool INV, int TA, int TB, int NTH, class RA, class RB, bool SLAB, bool PF>
 __global__ void __launch_bounds__(NTH) k_plane(PlaneArgs a)
 {
-    typedef F32::store2 St;
+    typedef typename X::store2 St;
+    typedef typename TwEntry<X>::type Ent;
     constexpr int A = RA::N(), B = RB::N();
     constexpr int RSX = (B % 2 == 0) ? B + 1 : B;
     constexpr int E = A * B;
@@ -86,16 +92,17 @@ __global__ void __launch_bounds__(NTH) k_plane(PlaneArgs a)
     static_assert(A * TB <= NTH && B * TA <= NTH, "threads per plane");
     extern __shared__ __align__(16) unsigned char kfa_plane_smem[];
     St *buf = reinterpret_cast<St *>(kfa_plane_smem);
-    St *twa = buf + A * RSX;  // stage tables (after the plane)
-    St *twb = twa + TWA;
+    constexpr int PLANE = plane_slots(A * RSX, (int)(16 / sizeof(St)));
+    Ent *twa = reinterpret_cast<Ent *>(buf + PLANE);  // stage tables (after the plane)
+    Ent *twb = twa + TWA;
     const int tid = threadIdx.x;
     const St *in = reinterpret_cast<const St *>(a.in);
     St *out = reinterpret_cast<St *>(a.out);
 
     for (int i = tid; i < TWA; i += NTH)
-        twa[i] = reinterpret_cast<const St *>(a.stw_a)[i];
+        twa[i] = reinterpret_cast<const Ent *>(a.stw_a)[i];
     for (int i = tid; i < TWB; i += NTH)
-        twb[i] = reinterpret_cast<const St *>(a.stw_b)[i];
+        twb[i] = reinterpret_cast<const Ent *>(a.stw_b)[i];
 
     long long pl = blockIdx.x;
     St v[IT];
@@ -125,20 +132,28 @@ __global__ void __launch_bounds__(NTH) k_plane(PlaneArgs a)
         __syncthreads();
         if (PF && pl + gridDim.x < a.planes)
             load(pl + gridDim.x);  // in flight during the stages below
-        {   // rows: B points, TB threads each
+        auto rows = [&] {  // B points, TB threads each
             const int line = tid / TB;
-            plane_stages<INV, TB, RB, 1>(std::make_integer_sequence<int, RB::K>{},
-                                         buf + (line < A ? line : 0) * RSX, twb, tid - line * TB, line < A);
-        }
-        if constexpr (64 % TB == 0)
-            __syncthreads();  // every row done before the columns read them
-        {   // columns: A points at stride RSX, TA threads each
+            plane_stages<X, INV, TB, RB, 1>(std::make_integer_sequence<int, RB::K>{},
+                                            buf + (line < A ? line : 0) * RSX, reinterpret_cast<const St *>(twb),
+                                            tid - line * TB, line < A);
+            if constexpr (64 % TB == 0)
+                __syncthreads();  // every row done before the columns (or the stores) read them
+        };
+        auto cols = [&] {  // A points at stride RSX, TA threads each
             const int line = tid / TA;
-            plane_stages<INV, TA, RA, RSX>(std::make_integer_sequence<int, RA::K>{}, buf + (line < B ? line : 0),
-                                           twa, tid - line * TA, line < B);
+            plane_stages<X, INV, TA, RA, RSX>(std::make_integer_sequence<int, RA::K>{}, buf + (line < B ? line : 0),
+                                              reinterpret_cast<const St *>(twa), tid - line * TA, line < B);
+            if constexpr (64 % TA == 0)
+                __syncthreads();  // every column done before the rows (or the stores) read it
+        };
+        if constexpr (X::fixed) {
+            cols();
+            rows();
+        } else {
+            rows();
+            cols();
         }
-        if constexpr (64 % TA == 0)
-            __syncthreads();  // every column done before the plane is read out
         {
             St *dst = out + base(pl);
             St w[IT];

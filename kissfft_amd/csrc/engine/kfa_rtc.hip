@@ -52,6 +52,7 @@
 #include "../kfa_engine.h"
 #include "kfa_fast.hpp"
 #include "kfa_internal.hpp"
+#include "kfa_plane.hpp"
 #include "kfa_tile.hpp"
 
 // embedded header sources (generated at build time)
@@ -516,6 +517,125 @@ const TileVariant *rtc_tile(int type, const std::vector<int> &radices, int inver
                 return &it->second->v;
         }
     return nullptr;
+}
+
+namespace {
+
+// One runtime-compiled plane: its variant and its loaded kernel.
+struct RtcPlane {
+    PlaneVariant v;
+    std::string name;
+    hipModule_t mod = nullptr;
+    hipFunction_t fn = nullptr;
+};
+
+std::map<std::string, std::unique_ptr<RtcPlane>> g_planes;  // by name expression, arch, device
+
+// Threads per line, at most `most`, that take the fewest butterfly slots over the stages.
+int plane_threads(int n, const std::vector<int> &rad, int most)
+{
+    int best = 1;
+    long long least = 0;
+    for (int T = 1; T <= most && T <= n; ++T) {
+        long long slots = 0;
+        for (int p : rad)
+            slots += (n / p + T - 1) / T * p;
+        if (!least || slots < least) {
+            best = T;
+            least = slots;
+        }
+    }
+    return best;
+}
+
+}  // namespace
+
+int plane_launch(const PlaneVariant &v, const PlaneArgs &a, hipStream_t s)
+{
+    if (!v.rtc)
+        return v.launch(a, s);
+    if (a.planes <= 0)
+        return 0;
+    if (a.planes > 0x7fffffffLL)
+        return -2;
+    PlaneArgs copy = a;
+    void *params[] = {&copy};
+    return hipModuleLaunchKernel(static_cast<const RtcPlane *>(v.rtc)->fn, (unsigned)a.planes, 1, 1, v.NTH, 1, 1,
+                                 (unsigned)v.lds, s, params, nullptr) == hipSuccess
+               ? 0
+               : -3;
+}
+
+const PlaneVariant *rtc_plane(int type, const std::vector<int> &ra, const std::vector<int> &rb, int inverse)
+{
+    if (!env_flag("KISSFFT_AMD_RTC", true) || ra.empty() || rb.empty())
+        return nullptr;
+    long long A = 1, B = 1, tw = 0;
+    for (int half = 0; half < 2; ++half)
+        for (int p : half ? rb : ra) {
+            if (!(p >= 2 && p <= 5) && !(type == KFA_F32 && (p == 7 || p == 8 || p == 11 || p == 13 || p == 16)))
+                return nullptr;
+            long long &n = half ? B : A;
+            tw += n * ((p - 1 + 1) / 2 * 2) + 2;  // (Radices::tw_len, rows padded to 2 entries)
+            n *= p;
+            if (n > 4096)
+                return nullptr;
+        }
+    const size_t cb = type == KFA_Q15 ? 4 : 8;
+    const size_t slots = ((size_t)A * (B % 2 == 0 ? B + 1 : B) + 3) / 4 * 4;
+    const size_t lds = slots * cb + (size_t)tw * 8;
+    if (lds > 64 * 1024)
+        return nullptr;
+    // threads: about 10 values each, and at least one per line of either axis
+    int NTH = 128;
+    while (NTH < 1024 && (A * B > 10LL * NTH || std::max(A, B) > NTH))
+        NTH *= 2;
+    if (std::max(A, B) > NTH || A * B > 20LL * NTH)
+        return nullptr;
+    const int TA = plane_threads((int)A, ra, NTH / (int)B), TB = plane_threads((int)B, rb, NTH / (int)A);
+    auto list = [](const std::vector<int> &r) {
+        std::string s = "kfa::Radices<2";
+        for (int p : r)
+            s += ", " + std::to_string(p);
+        return s + ">";
+    };
+    const char *arith = type == KFA_F32 ? "kfa::F32" : type == KFA_Q31 ? "kfa::Q31" : "kfa::Q15P";
+    const std::string arch = arch_name();
+    const std::string expr = std::string("&kfa::k_plane<") + arith + ", " + (inverse ? "true" : "false") + ", " +
+                             std::to_string(TA) + ", " + std::to_string(TB) + ", " + std::to_string(NTH) + ", " +
+                             list(ra) + ", " + list(rb) + ", false, false>";
+    std::lock_guard<std::mutex> g(g_rtc_mu);
+    const std::string key = expr + "|" + arch + "|" + std::to_string(current_dev());
+    auto it = g_planes.find(key);
+    if (it == g_planes.end()) {
+        auto rp = std::make_unique<RtcPlane>();
+        if (load_kernel(expr, arch, "#include \"kfa_plane.hpp\"\n", &rp->mod, &rp->fn) == 0) {
+            char nm[96];
+            snprintf(nm, sizeof nm, "rtc_plane%lldx%lld_t%dx%d_%d", A, B, TA, TB, NTH);
+            rp->name = nm;
+            PlaneVariant &v = rp->v;
+            v.type = type;
+            v.A = (int)A;
+            v.B = (int)B;
+            v.inverse = inverse;
+            v.TA = TA;
+            v.TB = TB;
+            v.NTH = NTH;
+            v.rad_a = ra;
+            v.rad_b = rb;
+            v.tw_pad = 2;
+            v.tw_fmt = type == KFA_Q15 ? 1 : 0;
+            v.lds = lds;
+            v.name = rp->name.c_str();
+            v.rtc = rp.get();
+            v.slab = false;
+            v.launch = nullptr;
+        } else {
+            rp.reset();  // remembered as unusable
+        }
+        it = g_planes.emplace(key, std::move(rp)).first;
+    }
+    return it->second ? &it->second->v : nullptr;
 }
 
 std::string tuned_key(const DevPlan &P, int kind, long long tune_lines)

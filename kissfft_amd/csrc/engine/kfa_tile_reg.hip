@@ -160,7 +160,7 @@ template <class RA, class RB>
 constexpr size_t plane_lds()
 {
     constexpr int B = RB::N();
-    return ((size_t)RA::N() * (B % 2 == 0 ? B + 1 : B) + RA::tw_len() + RB::tw_len()) * sizeof(float2);
+    return ((size_t)plane_slots(RA::N() * (B % 2 == 0 ? B + 1 : B), 2) + RA::tw_len() + RB::tw_len()) * sizeof(float2);
 }
 
 // Planes of which one workgroup fills a CU's LDS run persistently (as many workgroups as
@@ -170,7 +170,7 @@ constexpr size_t plane_lds()
 template <bool INV, int TA, int TB, int NTH, class RA, class RB, bool SLAB, bool PF>
 static int launch_plane_as(const PlaneArgs &a, hipStream_t s)
 {
-    const void *fn = (const void *)k_plane<INV, TA, TB, NTH, RA, RB, SLAB, PF>;
+    const void *fn = (const void *)k_plane<F32, INV, TA, TB, NTH, RA, RB, SLAB, PF>;
     constexpr size_t lds = plane_lds<RA, RB>();
     static long long resident = 0;  // 0: one workgroup per plane
     static std::once_flag once;
@@ -187,7 +187,7 @@ static int launch_plane_as(const PlaneArgs &a, hipStream_t s)
     const long long grid = (resident > 0 && a.planes > resident) ? resident : a.planes;
     if (grid > 0x7fffffffLL)
         return -2;
-    hipLaunchKernelGGL((k_plane<INV, TA, TB, NTH, RA, RB, SLAB, PF>), dim3((unsigned)grid), dim3(NTH), lds, s, a);
+    hipLaunchKernelGGL((k_plane<F32, INV, TA, TB, NTH, RA, RB, SLAB, PF>), dim3((unsigned)grid), dim3(NTH), lds, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
