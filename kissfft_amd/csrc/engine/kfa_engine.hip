@@ -2382,7 +2382,9 @@ int run_real_rows(DevPlan &H, const RealTables &R, int inverse, const void *in, 
         ++g_launches;
         return fast_launch(*fc->v, a, s) ? fail(-3, "fast kernel launch failed") : 0;
     }
-    if (blue_real_rows(H))
+    // (a captured call without a workspace of its own keeps the general kernel, which needs
+    // no temporary)
+    if (blue_real_rows(H) && (thread_workspace() || !stream_capturing(s)))
         return run_real_multipass(H, R, inverse, in, in_hi, out, out_hi, howmany, s);
     LineLaunch ll{};
     ll.in = in;

@@ -35,7 +35,7 @@ struct FastChoice {
     void *d_stw = nullptr;
 };
 
-// A float tile variant (kfa_tile.hpp) with its stage table.
+// A tile variant (kfa_tile.hpp; built in, or compiled at run time) with its stage table.
 struct TileChoice {
     const TileVariant *v = nullptr;
     DevBuf stw_mem;

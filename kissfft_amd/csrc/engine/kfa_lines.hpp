@@ -121,8 +121,24 @@ __device__ __forceinline__ void run_stage(const LinePlan &pl, const StageDesc &s
             const long long ug = uadd + (long long)pl.u_mul * u;
             const long long kg = ug + (long long)q1 * sd.mg;
             const long long step = (long long)sd.Ptw * kg % pl.N;
-            C acc = O::fixdiv(O::load(src[cx.idx(line, u * Pl * p + o)]), p);
             long long ti = 0;
+            if constexpr (!A::fixed) {
+                // summed in FP64, rounded once: a float sum of 4099 products is off by 1.1e-6
+                C x = O::load(src[cx.idx(line, u * Pl * p + o)]);
+                double re = x.r, im = x.i;
+                for (int q = 1; q < p; ++q) {
+                    ti += step;
+                    if (ti >= pl.N)
+                        ti -= pl.N;
+                    x = O::load(src[cx.idx(line, u * Pl * p + q * Pl + o)]);
+                    const C t = O::load(tw[ti]);
+                    re = fma((double)x.r, (double)t.r, fma(-(double)x.i, (double)t.i, re));
+                    im = fma((double)x.r, (double)t.i, fma((double)x.i, (double)t.r, im));
+                }
+                dst[cx.idx(line, j)] = O::pack(C{(float)re, (float)im});
+                continue;
+            }
+            C acc = O::fixdiv(O::load(src[cx.idx(line, u * Pl * p + o)]), p);
             for (int q = 1; q < p; ++q) {
                 ti += step;
                 if (ti >= pl.N)

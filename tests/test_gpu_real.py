@@ -212,3 +212,30 @@ def test_batches_of_short_real_rows(dtype, n, monkeypatch, capfd):
     err = capfd.readouterr().err
     if n // 2 != 11 or dtype == "float":
         assert f"rtc_r2c{n // 2}" in err and f"rtc_c2r{n // 2}" in err
+
+
+@pytest.mark.parametrize("n", [2 * 1009, 2 * 4099])
+def test_prime_half_rows_under_capture(n):
+    """Real rows of a prime half length captured by the caller: every replay between eager
+    work gives the transform of the input of that moment, within the float bound."""
+    import torch
+    lib = kissfft_amd.load("float")
+    dev = torch.device("cuda:0")
+    b, st = 5, torch.cuda.Stream()
+    x = torch.from_numpy(np.random.default_rng(n).standard_normal((b, n)).astype(np.float32)).to(dev)
+    X = torch.empty(b, n // 2 + 1, 2, device=dev)
+    cfg = lib.fftr_alloc(n)
+    lib.fftr_batch(cfg, x, X, b, n, n // 2 + 1)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
+        lib.fftr_batch(cfg, x, X, b, n, n // 2 + 1, stream=st)
+    for rep in range(3):
+        x.mul_(1.25).add_(0.5)
+        X.fill_(9.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            g.replay()
+        torch.cuda.synchronize()
+        want = np.fft.rfft(x.cpu().numpy().astype(np.float64), axis=-1)
+        assert rel_l2(cplx(X.cpu().numpy()), want) <= ABS_FLOAT_BOUND, rep

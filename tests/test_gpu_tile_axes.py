@@ -35,6 +35,7 @@ def rnd(rng, dtype, shape):
 def test_compiled_axes(dims, dtype, monkeypatch, capfd):
     lib = kissfft_amd.load(dtype)
     monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    monkeypatch.setenv("KISSFFT_AMD_PLANE", "0")  # an axis each, also where a plane would do
     lib.L.kiss_fft_cleanup()
     x = rnd(np.random.default_rng(sum(dims)), dtype, (2,) + dims + (2,))
     for inv in (False, True):
