@@ -351,11 +351,23 @@ template <bool INV>
 struct Dft<8, INV> {
     __device__ __forceinline__ static void run(Cf *v)
     {
-        const float h = 0.707106781186547524400844362104849039f;
         Cf e[4] = {v[0], v[2], v[4], v[6]};
         Cf o[4] = {v[1], v[3], v[5], v[7]};
         Dft<4, INV>::run(e);
         Dft<4, INV>::run(o);
+        join(v, e, o);
+    }
+    // run() after its first level: v[q] holds x[q] + x[q+4], v[q+4] holds x[q] - x[q+4]
+    __device__ __forceinline__ static void tail(Cf *v)
+    {
+        const Cf r6 = cf_rot<INV>(v[6]), r7 = cf_rot<INV>(v[7]);
+        const Cf e[4] = {cf_add(v[0], v[2]), cf_add(v[4], r6), cf_sub(v[0], v[2]), cf_sub(v[4], r6)};
+        const Cf o[4] = {cf_add(v[1], v[3]), cf_add(v[5], r7), cf_sub(v[1], v[3]), cf_sub(v[5], r7)};
+        join(v, e, o);
+    }
+    __device__ __forceinline__ static void join(Cf *v, const Cf *e, const Cf *o)
+    {
+        const float h = 0.707106781186547524400844362104849039f;
         // o[k] *= W8^k
         Cf o1 = INV ? Cf{h * (o[1].r - o[1].i), h * (o[1].r + o[1].i)}
                     : Cf{h * (o[1].r + o[1].i), h * (o[1].i - o[1].r)};

@@ -74,7 +74,7 @@ static void fft_f64(double *re, double *im, size_t n, double *w)
 static size_t ff_block(size_t nh)
 {
     static const struct { size_t n; double ps; } len[] = {{256, 3.7}, {512, 3.4}, {1024, 3.5}, {2048, 4.0},
-                                                          {4096, 4.25}, {8192, 5.7}};
+                                                          {4096, 5.0}, {8192, 5.7}};
     enum { COUNT = sizeof len / sizeof len[0] };
     double cost[COUNT], least = 0;
     size_t i;
