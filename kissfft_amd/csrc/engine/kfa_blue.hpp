@@ -113,7 +113,7 @@ struct Conv {
     static_assert(RS::N() % T == 0 && RS::K > 1, "threads per line must divide the length");
     // FP64 spectrum, 4096 points: the products stay FP64 through the first level of the
     // inverse and are rounded after it, two roundings less, so that 1000 taps are as exact as
-    // in blocks of 2048 points (1.73e-7 from FP64, 1.75e-7 without).  It costs 92 registers
+    // in blocks of 2048 points (1.73e-7 from FP64, 1.75e-7 without).  It costs 94 registers
     // instead of 78, two workgroups of 512 threads per CU instead of three: 2^26 samples
     // 213 -> 247 us (held to 80 registers the kernel spills).
     static constexpr bool PAIRED = sizeof(HT) == sizeof(Cd) && Mid::p == 8 && RS::N() >= 4096;
@@ -125,21 +125,23 @@ struct Conv {
         Cf m[Mid::J][Mid::p];
         conv_stages<false, T, RS, 0, true>(v, m, buf, stw_f, t);
         // (the inverse's first stage reads element r*NB + b as the forward's last one left it)
+        if constexpr (PAIRED) {
 #pragma unroll
-        for (int j = 0; j < Mid::J; ++j)
+            for (int j = 0; j < Mid::J; ++j)
 #pragma unroll
-            for (int q = 0; q < Mid::p; ++q) {
-                const HT *h = H + t + j * T + q * Mid::NB;
-                if constexpr (PAIRED) {
-                    if (q >= 4)
-                        continue;
+                for (int q = 0; q < 4; ++q) {
+                    const HT *h = H + t + j * T + q * Mid::NB;
                     const Cd a = cd_mul(m[j][q], h[0]), b = cd_mul(m[j][q + 4], h[4 * Mid::NB]);
                     m[j][q] = Cf{(float)(a.r + b.r), (float)(a.i + b.i)};
                     m[j][q + 4] = Cf{(float)(a.r - b.r), (float)(a.i - b.i)};
-                } else {
-                    m[j][q] = conv_mul(m[j][q], h[0]);
                 }
-            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < Mid::J; ++j)
+#pragma unroll
+                for (int q = 0; q < Mid::p; ++q)
+                    m[j][q] = conv_mul(m[j][q], H[t + j * T + q * Mid::NB]);
+        }
         conv_stages<true, T, RI, 0, false, PAIRED>(m, out, buf, stw_i, t);
     }
 };
