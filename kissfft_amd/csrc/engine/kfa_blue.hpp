@@ -115,7 +115,7 @@ struct Conv {
     // inverse and are rounded after it, two roundings less, so that 1000 taps are as exact as
     // in blocks of 2048 points (1.73e-7 from FP64, 1.75e-7 without).  It costs 94 registers
     // instead of 78, two workgroups of 512 threads per CU instead of three: 2^26 samples
-    // 213 -> 247 us (held to 80 registers the kernel spills).
+    // 213 -> 236 us (held to 80 registers the kernel spills).
     static constexpr bool PAIRED = sizeof(HT) == sizeof(Cd) && Mid::p == 8 && RS::N() >= 4096;
 
     __device__ __forceinline__ static void run(Cf (&v)[In::J][In::p], Cf (&out)[Out::J][Out::p], F32::store2 *buf,

@@ -70,7 +70,7 @@ static void fft_f64(double *re, double *im, size_t n, double *w)
  * length that costs least per good sample: the kernel's time per point of a block (ps),
  * times the points per good sample.  A shorter one within a tenth of the least is taken: its
  * transforms round less.  Measured, 2^25 real samples: 30 taps 67 us with 512 or 1024 points,
- * 74 with 2048; 1000 taps 91 us with 4096 points, 119 with 2048, 107 with 8192. */
+ * 74 with 2048; 1000 taps 112 us with 4096 points, 119 with 2048, 107 with 8192. */
 static size_t ff_block(size_t nh)
 {
     static const struct { size_t n; double ps; } len[] = {{256, 3.7}, {512, 3.4}, {1024, 3.5}, {2048, 4.0},
