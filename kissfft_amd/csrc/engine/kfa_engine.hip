@@ -1516,15 +1516,21 @@ static int run_c2c_bailey(const BaileyPlan &bp, long long n, const void *in, lon
 // not disturbed).  The choice is recorded only once its table exists.
 int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, long long lines_hint)
 {
+    // callers read the choice without the lock, so only finished ones are handed out: the
+    // plan's, published whole, or (no decision yet) the empty one
+    static const FastChoice general;
     std::lock_guard<std::mutex> g(P.mu);
-    FastChoice &fc = P.fast[kind];
-    *out = &fc;
-    if (fc.decided)
+    std::shared_ptr<const FastChoice> &slot = P.fast[kind];
+    auto decide = [&](std::shared_ptr<const FastChoice> c) {
+        slot = std::move(c);
+        *out = slot.get();
         return 0;
-    if (!P.single || !env_flag("KISSFFT_AMD_FAST", true)) {
-        fc.decided = true;
+    };
+    *out = slot ? slot.get() : &general;
+    if (slot)
         return 0;
-    }
+    if (!P.single || !env_flag("KISSFFT_AMD_FAST", true))
+        return decide(std::make_shared<const FastChoice>());
     if (P.n < kShortRow && lines_hint * P.n < kShortValues)
         return 0;  // the general kernel; a larger batch may still decide
     std::vector<const FastVariant *> cand;
@@ -1541,10 +1547,8 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
     // stream is being captured: such a plan keeps the general kernel)
     if (cand.empty() && !stream_capturing(s))
         (void)rtc_candidates(P, kind, cand);
-    if (cand.empty()) {
-        fc.decided = true;
-        return 0;
-    }
+    if (cand.empty())
+        return decide(std::make_shared<const FastChoice>());
     std::vector<DevBuf> tabs(cand.size());
     for (size_t i = 0; i < cand.size(); ++i) {
         if ((long long)(cand[i]->tw_len) <= 0)
@@ -1613,14 +1617,14 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
             break;
         }
     }
-    fc.v = cand[best];
-    fc.stw_mem = tabs[best];
-    fc.d_stw = fc.stw_mem.get();
-    fc.decided = true;
+    auto fc = std::make_shared<FastChoice>();
+    fc->v = cand[best];
+    fc->stw_mem = tabs[best];
+    fc->d_stw = fc->stw_mem.get();
     if (env_flag("KISSFFT_AMD_VERBOSE", false))
         fprintf(stderr, "[kissfft_amd] n=%d kind=%d inverse=%d: fast variant %s\n", P.n, kind, P.inverse,
-                fc.v->name);
-    return 0;
+                fc->v->name);
+    return decide(fc);
 }
 
 // ------------------------------------------------------------------------------------

@@ -27,9 +27,9 @@ int dev_upload(const void *host, size_t bytes, DevBuf &out);
 int dev_alloc(size_t bytes, DevBuf &out);
 void free_deferred();
 
-// The fast variant chosen for one transform kind of a plan, with its stage table.
+// The fast variant chosen for one transform kind of a plan, with its stage table (v null:
+// the general kernel).  Never changed once a caller can see it.
 struct FastChoice {
-    bool decided = false;
     const FastVariant *v = nullptr;
     DevBuf stw_mem;
     void *d_stw = nullptr;
@@ -72,7 +72,7 @@ struct DevPlan {
     bool bigp = false;       // first stage radix L1 above one LDS line: a global-memory DFT pass
     LinePlan lp1{}, lp2{};
     std::mutex mu;           // guards the choices below (each decided once)
-    FastChoice fast[3];      // per FK_C2C / FK_R2C / FK_C2R
+    std::shared_ptr<const FastChoice> fast[3];  // per FK_C2C / FK_R2C / FK_C2R; null: undecided
     bool bailey_decided = false;
     std::shared_ptr<const BaileyPlan> bailey;
     bool rfused_decided[2] = {false, false};

@@ -1,0 +1,59 @@
+// Host-only checks of how the engine decides which kernel a plan runs.  No device is
+// needed: plans are filled in by hand and nothing is launched.
+//     choices CASE        exit status 0: the case holds
+#include <cstdio>
+#include <cstring>
+#include <memory>
+
+#include "kfa_engine.h"
+#include "engine/kfa_fast.hpp"
+#include "engine/kfa_internal.hpp"
+
+using namespace kfa;
+
+#define CHECK(x)                                                                      \
+    do {                                                                              \
+        if (!(x)) {                                                                   \
+            fprintf(stderr, "%s:%d: %s does not hold\n", __FILE__, __LINE__, #x);     \
+            return 1;                                                                 \
+        }                                                                             \
+    } while (0)
+
+static void single_plan(DevPlan &P, int type, int n, std::vector<int> radix)
+{
+    P.type = type;
+    P.n = n;
+    P.radix = std::move(radix);
+    P.single = true;
+}
+
+// What choose_fast hands out is read without the plan's lock, so a choice still open must
+// not be the plan's own storage, which a larger batch of the same plan writes.
+static int open_choice_is_not_the_plans()
+{
+    for (int kind : {FK_R2C, FK_C2R}) {
+        DevPlan P;
+        single_plan(P, KFA_F32, 8, {4, 2});
+        const FastChoice *fc = nullptr;
+        CHECK(choose_fast(P, kind, nullptr, &fc, 3) == 0);
+        CHECK(fc && !fc->v && !fc->d_stw);
+        const char *at = reinterpret_cast<const char *>(fc), *p0 = reinterpret_cast<const char *>(&P);
+        CHECK(at < p0 || at >= p0 + sizeof P);
+    }
+    return 0;
+}
+
+int main(int argc, char **argv)
+{
+    static const struct {
+        const char *name;
+        int (*run)();
+    } cases[] = {
+        {"open_choice_is_not_the_plans", open_choice_is_not_the_plans},
+    };
+    for (const auto &c : cases)
+        if (argc == 2 && !strcmp(argv[1], c.name))
+            return c.run();
+    fprintf(stderr, "usage: choices CASE\n");
+    return 2;
+}
