@@ -1531,7 +1531,7 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
         return 0;
     if (!P.single || !env_flag("KISSFFT_AMD_FAST", true))
         return decide(std::make_shared<const FastChoice>());
-    if (P.n < kShortRow && lines_hint * P.n < kShortValues)
+    if (kind != FK_C2C && P.n < kShortRow && lines_hint * P.n < kShortValues)
         return 0;  // the general kernel; a larger batch may still decide
     std::vector<const FastVariant *> cand;
     for (const FastVariant &v : fast_registry()) {

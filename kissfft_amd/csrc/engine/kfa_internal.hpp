@@ -161,7 +161,8 @@ int build_rtab(const kfa_rplan *hp, int dev, std::shared_ptr<RealTables> &out);
 // on a batch sized from lines_hint, the number of lines of the call that asks)
 int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, long long lines_hint = 0);
 
-// rows shorter than this are compiled only for batches of kShortValues values
+// real rows (and N-D axes) shorter than this are compiled only for batches of kShortValues
+// values; no complex row is
 constexpr int kShortRow = 16;
 constexpr long long kShortValues = 1LL << 16;
 // runtime-compiled variants of a plan's length and kind (kfa_rtc.hip), when none is built in

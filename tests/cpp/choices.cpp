@@ -43,6 +43,27 @@ static int open_choice_is_not_the_plans()
     return 0;
 }
 
+// While the no-allocation entry point runs, choices that would allocate are refused.
+struct NoAlloc {
+    NoAlloc() { thread_noalloc() = true; }
+    ~NoAlloc() { thread_noalloc() = false; }
+};
+
+// Complex lines under 16 points have no compiled row: a batch of any size decides that, and
+// the no-allocation entry point then takes batches of any size.
+static int short_complex_lines_are_decided()
+{
+    for (int type : {KFA_F32, KFA_Q15, KFA_Q31}) {
+        DevPlan P;
+        single_plan(P, type, 8, {2, 4});
+        const FastChoice *fc = nullptr;
+        CHECK(choose_fast(P, FK_C2C, nullptr, &fc, 3) == 0 && !fc->v);
+        NoAlloc on;
+        CHECK(choose_fast(P, FK_C2C, nullptr, &fc, 1 << 20) == 0 && !fc->v);
+    }
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     static const struct {
@@ -50,6 +71,7 @@ int main(int argc, char **argv)
         int (*run)();
     } cases[] = {
         {"open_choice_is_not_the_plans", open_choice_is_not_the_plans},
+        {"short_complex_lines_are_decided", short_complex_lines_are_decided},
     };
     for (const auto &c : cases)
         if (argc == 2 && !strcmp(argv[1], c.name))

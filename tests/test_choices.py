@@ -32,5 +32,6 @@ def check(driver, case):
     assert r.returncode == 0, r.stderr
 
 
-def test_open_choice_is_not_the_plans(driver):
-    check(driver, "open_choice_is_not_the_plans")
+@pytest.mark.parametrize("case", ["open_choice_is_not_the_plans", "short_complex_lines_are_decided"])
+def test_choice(driver, case):
+    check(driver, case)
