@@ -1892,7 +1892,7 @@ static int fixed_axis(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoic
 }
 
 // The tile kernels of a multi-pass fixed-point plan's two passes, decided once per plan (as
-// fixed_axis; null: the general kernel).  The second pass reads stage tables of the full
+// fixed_axis, and left open by a no-allocation call too; null: the general kernel).  The second pass reads stage tables of the full
 // length, about 1.3 entries a point, so very long lines keep the general kernel, which
 // reads the one n-point table.
 constexpr int kSplitTableLongest = 1 << 23;
@@ -1905,9 +1905,8 @@ static int fixed_split(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoi
         t1 = t2 = nullptr;
         if (P.type != KFA_F32 && !P.single && !P.bigp && P.n <= kSplitTableLongest &&
             env_flag("KISSFFT_AMD_FAST", true)) {
-            if (thread_noalloc())
-                return noalloc_refuse("the two-pass plan");
-            if (stream_capturing(s))
+            // (the general kernel needs nothing that would have to be allocated)
+            if (thread_noalloc() || stream_capturing(s))
                 return 0;
             std::vector<int> r1, r2;
             long long m = 1;

@@ -64,6 +64,23 @@ static int short_complex_lines_are_decided()
     return 0;
 }
 
+// A long fixed-point line whose two passes are not decided runs on the general kernel under
+// the no-allocation entry point: that kernel reads the plan's own table and nothing else.
+static int fixed_split_needs_no_allocation()
+{
+    for (int type : {KFA_Q15, KFA_Q31}) {
+        DevPlan P;
+        P.type = type;
+        P.n = 1 << 16;
+        P.radix = std::vector<int>(8, 4);
+        P.single = false;
+        P.L1 = P.Q = 256;
+        NoAlloc on;
+        CHECK(prepare_multipass(P, FK_C2C, nullptr) == 0);
+    }
+    return 0;
+}
+
 int main(int argc, char **argv)
 {
     static const struct {
@@ -72,6 +89,7 @@ int main(int argc, char **argv)
     } cases[] = {
         {"open_choice_is_not_the_plans", open_choice_is_not_the_plans},
         {"short_complex_lines_are_decided", short_complex_lines_are_decided},
+        {"fixed_split_needs_no_allocation", fixed_split_needs_no_allocation},
     };
     for (const auto &c : cases)
         if (argc == 2 && !strcmp(argv[1], c.name))
