@@ -723,8 +723,8 @@ struct TileCache {
     std::map<std::tuple<int, long long, int, int>, BufPair> rs;                           // dev, nc, n, inv
     // dev, A, B, inv, slab, small (see plane_choice)
     std::map<std::tuple<int, int, int, int, int, int>, std::shared_ptr<const PlaneChoice>> plane;
-    // dev, type, A, B, inv (see fixed_plane)
-    std::map<std::tuple<int, int, int, int, int>, std::shared_ptr<const PlaneChoice>> fplane;
+    // dev, type, A, B, inv (see compiled_plane)
+    std::map<std::tuple<int, int, int, int, int>, std::shared_ptr<const PlaneChoice>> made_plane;
 };
 
 static TileCache &tile_cache()
@@ -1260,7 +1260,7 @@ int blue_launch(DevPlan &P, BlueArgs &b, hipStream_t s)
     return v->launch(b, s) ? fail(-3, "Bluestein kernel launch failed") : 0;
 }
 
-// The plane variant for A x B planes (float) on the current device, or v == nullptr:
+// The built-in plane variant for A x B planes (float) on the current device, or v == nullptr:
 // contiguous planes of the last two axes, or (slab) an outer axis of length A with the
 // last axis, rows rs values apart and nsub planes per value of the axes before it (the
 // plane geometry of PlaneArgs).  Several candidates are timed once, in the caller's
@@ -1268,9 +1268,8 @@ int blue_launch(DevPlan &P, BlueArgs &b, hipStream_t s)
 // and per size class (up to 128 MiB per side, which the 256 MB Infinity Cache holds
 // between passes, or more: the ranking differs between the two).
 // (KISSFFT_AMD_PLANE=0 turns the plane pass off, KISSFFT_AMD_TILE forces a variant by name.)
-// may_compile: contiguous planes without a built-in variant may take a runtime-compiled one.
 static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long nsub, long long planes,
-                        bool may_compile, hipStream_t s, std::shared_ptr<const PlaneChoice> &out)
+                        hipStream_t s, std::shared_ptr<const PlaneChoice> &out)
 {
     int dev;
     int rc = current_device(&dev);
@@ -1300,17 +1299,6 @@ static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long 
                 c->v = &v;
                 cand.push_back(c);
             }
-    }
-    if (cand.empty() && !slab && env_flag("KISSFFT_AMD_FAST", true) && env_flag("KISSFFT_AMD_PLANE", true)) {
-        if (!may_compile || stream_capturing(s)) {
-            out = std::make_shared<const PlaneChoice>();
-            return 0;  // the choice stays open
-        }
-        const std::vector<int> ra = float_schedule(A, true), rb = float_schedule(B, true);
-        if (const PlaneVariant *v = rtc_plane(KFA_F32, ra, rb, inverse)) {
-            cand.push_back(std::make_shared<PlaneChoice>());
-            cand.back()->v = v;
-        }
     }
     for (auto &c : cand) {
         const std::vector<unsigned char> ta = float_twiddles(A, inverse, A, 1), tb = float_twiddles(B, inverse, B, 1);
@@ -1369,9 +1357,11 @@ static bool plane_pays(long long planes, long long values)
     return values <= 2048 || (planes >= 128 && values <= 5000);
 }
 
-// The compiled plane kernel for the last two axes of a fixed-point N-D transform, columns of
-// plan PA and rows of plan PB (v == nullptr: none), decided once per pair of plans' lengths.
-static int fixed_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, std::shared_ptr<const PlaneChoice> &out)
+// The plane kernel compiled for the last two axes of an N-D transform, columns of plan PA and
+// rows of plan PB (v == nullptr: none), decided once per pair of plans' lengths.  Kept apart
+// from the built-in choices: whether a call may run it depends on the call (plane_pays),
+// not on what an earlier one compiled.
+static int compiled_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, std::shared_ptr<const PlaneChoice> &out)
 {
     int dev;
     int rc = current_device(&dev);
@@ -1380,8 +1370,8 @@ static int fixed_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, std:
     auto &C = tile_cache();
     std::lock_guard<std::mutex> g(C.mu);
     const auto key = std::make_tuple(dev, PA.type, PA.n, PB.n, PA.inverse);
-    auto it = C.fplane.find(key);
-    if (it != C.fplane.end()) {
+    auto it = C.made_plane.find(key);
+    if (it != C.made_plane.end()) {
         out = it->second;
         return 0;
     }
@@ -1391,11 +1381,14 @@ static int fixed_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, std:
     out = pc;
     if (stream_capturing(s))
         return 0;  // the choice stays open
-    if (PA.single && PB.single && env_flag("KISSFFT_AMD_FAST", true) && env_flag("KISSFFT_AMD_PLANE", true))
-        pc->v = rtc_plane(PA.type, PA.radix, PB.radix, PA.inverse);
+    if (PA.single && PB.single && env_flag("KISSFFT_AMD_FAST", true) && env_flag("KISSFFT_AMD_PLANE", true)) {
+        const bool fixed = PA.type != KFA_F32;
+        pc->v = rtc_plane(PA.type, fixed ? PA.radix : float_schedule(PA.n, true),
+                          fixed ? PB.radix : float_schedule(PB.n, true), PA.inverse);
+    }
     if (pc->v) {
-        if ((rc = make_stage_table_raw(PA.h_tw.data(), PA.type, PA.n, PA.radix, 2, pc->v->tw_fmt, pc->mem_a)) ||
-            (rc = make_stage_table_raw(PB.h_tw.data(), PB.type, PB.n, PB.radix, 2, pc->v->tw_fmt, pc->mem_b)))
+        if ((rc = make_stage_table_raw(PA.h_tw.data(), PA.type, PA.n, pc->v->rad_a, 2, pc->v->tw_fmt, pc->mem_a)) ||
+            (rc = make_stage_table_raw(PB.h_tw.data(), PB.type, PB.n, pc->v->rad_b, 2, pc->v->tw_fmt, pc->mem_b)))
             return rc;
         pc->stw_a = pc->mem_a.get();
         pc->stw_b = pc->mem_b.get();
@@ -1403,7 +1396,7 @@ static int fixed_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, std:
             fprintf(stderr, "[kissfft_amd] plane %dx%d inverse=%d type=%d: %s\n", PA.n, PB.n, PA.inverse, PA.type,
                     pc->v->name);
     }
-    C.fplane[key] = pc;
+    C.made_plane[key] = pc;
     return 0;
 }
 
@@ -2749,9 +2742,10 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
     long long outer = howmany, inner = total;
     const void *src = in;
     int rc = 0;
-    int paired = -1;  // float: the axis done together with the last one in a plane pass
+    int paired = -1;  // the axis done together with the last one in a plane pass
     std::shared_ptr<const PlaneChoice> pc;
-    if (ndims >= 2 && P[ndims - 1]->type == KFA_F32) {
+    const bool fixed = P[0]->type != KFA_F32;
+    if (ndims >= 2 && !fixed) {
         // the last axis and one other in one pass when a plane (or slab) of them fits in
         // LDS: the axis before the last first (contiguous planes), then the outer axes from
         // the first (float results do not depend on the order of the axes beyond rounding)
@@ -2759,11 +2753,7 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
         std::vector<int> order{ndims - 2};
         for (int k = 0; k < ndims - 2; ++k)
             order.push_back(k);
-        // (built-in variants of any of them first, then a compiled plane of the last two axes)
-        order.push_back(ndims - 2);
-        for (size_t i = 0; i < order.size() && paired < 0; ++i) {
-            const int k = order[i];
-            const bool compile = i + 1 == order.size();
+        for (int k : order) {
             long long rs = 1;  // in-plane offsets are 32-bit
             for (int j = k + 1; j < ndims; ++j)
                 rs *= dims[j];
@@ -2773,43 +2763,45 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
             for (int j = k + 1; j < ndims - 1; ++j)
                 mid *= dims[j];
             const long long planes = howmany * (total / ((long long)dims[k] * nb));
-            if (compile && !plane_pays(planes, (long long)dims[k] * nb))
-                break;
-            if ((rc = plane_choice(dims[k], nb, P[ndims - 1]->inverse, k != ndims - 2, (int)rs, mid, planes, compile, s,
-                                   pc)))
+            if ((rc = plane_choice(dims[k], nb, P[ndims - 1]->inverse, k != ndims - 2, (int)rs, mid, planes, s, pc)))
                 return rc;
-            if (pc->v && (k == ndims - 2 || pc->v->slab))
+            if (pc->v && (k == ndims - 2 || pc->v->slab)) {
                 paired = k;
-        }
-        if (paired >= 0) {
-            long long rs = 1, mid = 1;  // row stride; planes per value of the axes before `paired`
-            for (int k = paired + 1; k < ndims; ++k)
-                rs *= dims[k];
-            for (int k = paired + 1; k < ndims - 1; ++k)
-                mid *= dims[k];
-            const long long planes = howmany * (total / ((long long)dims[paired] * nb));
-            const PlaneArgs pa{in, out, pc->stw_a, pc->stw_b, planes, (int)rs, mid, (long long)dims[paired] * rs, nb};
-            ++g_launches;
-            if (plane_launch(*pc->v, pa, s))
-                return fail(-3, "plane kernel launch failed");
-            src = out;
+                break;
+            }
         }
     }
-    // fixed point: the axes in order, the last two in one pass where a plane of them is compiled
-    std::shared_ptr<const PlaneChoice> fp;
-    if (ndims >= 2 && P[0]->type != KFA_F32) {
+    if (ndims >= 2 && paired < 0) {
+        // no built-in one: a compiled plane of the last two axes
         const long long values = (long long)dims[ndims - 2] * dims[ndims - 1];
-        if (plane_pays(howmany * (total / values), values) &&
-            (rc = fixed_plane(*P[ndims - 2], *P[ndims - 1], s, fp)))
-            return rc;
-    }
-    for (int k = 0; k < ndims && rc == 0; ++k) {
-        if (fp && fp->v && k == ndims - 2) {
-            const long long A = dims[k], B = dims[k + 1];
-            ++g_launches;
-            return plane_launch(*fp->v, plane_args(src, out, fp->stw_a, fp->stw_b, howmany * (total / (A * B)), A, B), s)
-                       ? fail(-3, "plane kernel launch failed") : 0;
+        if (plane_pays(howmany * (total / values), values)) {
+            if ((rc = compiled_plane(*P[ndims - 2], *P[ndims - 1], s, pc)))
+                return rc;
+            if (pc->v)
+                paired = ndims - 2;
         }
+    }
+    auto plane_pass = [&](const void *from) {
+        const int nb = dims[ndims - 1];
+        long long rs = 1, mid = 1;  // row stride; planes per value of the axes before `paired`
+        for (int k = paired + 1; k < ndims; ++k)
+            rs *= dims[k];
+        for (int k = paired + 1; k < ndims - 1; ++k)
+            mid *= dims[k];
+        const long long planes = howmany * (total / ((long long)dims[paired] * nb));
+        const PlaneArgs pa{from, out, pc->stw_a, pc->stw_b, planes, (int)rs, mid, (long long)dims[paired] * rs, nb};
+        ++g_launches;
+        return plane_launch(*pc->v, pa, s) ? fail(-3, "plane kernel launch failed") : 0;
+    };
+    if (paired >= 0 && !fixed) {
+        if ((rc = plane_pass(in)))
+            return rc;
+        src = out;
+    }
+    // fixed point: the axes in order, the plane in the place of its own
+    for (int k = 0; k < ndims && rc == 0; ++k) {
+        if (fixed && k == paired)
+            return plane_pass(src);
         inner /= dims[k];
         if (paired < 0 || (k != paired && k != ndims - 1)) {
             rc = run_axis(*P[k], src, out, outer, inner, s);
@@ -2985,7 +2977,7 @@ void kfa_cleanup(void)
         auto &T = tile_cache();
         std::lock_guard<std::mutex> gt(T.mu);
         T.plane.clear();
-        T.fplane.clear();
+        T.made_plane.clear();
         T.choice.clear();
         T.fs.clear();
         T.rs.clear();

@@ -50,3 +50,26 @@ def test_compiled_planes(dims, b, dtype, monkeypatch, capfd):
         torch.cuda.synchronize()
         np.testing.assert_array_equal(d.cpu().numpy(), y)
     assert f"plane {dims[-2]}x{dims[-1]} " in capfd.readouterr().err
+
+
+def test_few_planes_after_many():
+    """A call of few planes takes the axis passes whatever ran before it: its launches and its
+    bits are those of the same call in a fresh process, also after a batch of the same
+    planes that is worth a compiled kernel."""
+    lib = kissfft_amd.load("float")
+    dims, many, few = (80, 60), 130, 4
+    x = np.random.default_rng(3).uniform(-1, 1, (many,) + dims + (2,)).astype(np.float32)
+    cfg = lib.fftnd_alloc(dims)
+
+    def run(b):
+        y = np.zeros_like(x[:b])
+        n0 = lib.stats()["launches"]
+        lib.fftnd_batch(cfg, x[:b], y, b)
+        return y, lib.stats()["launches"] - n0
+
+    lib.L.kiss_fft_cleanup()
+    fresh, n_fresh = run(few)
+    _, n_many = run(many)
+    after, n_after = run(few)
+    assert (n_fresh, n_many, n_after) == (2, 1, 2)
+    np.testing.assert_array_equal(after, fresh)
