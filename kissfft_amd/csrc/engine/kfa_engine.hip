@@ -1519,13 +1519,17 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
         *out = slot.get();
         return 0;
     };
-    *out = slot ? slot.get() : &general;
-    if (slot)
+    // A small batch of short real rows runs on the general kernel whatever ran before it (its
+    // float bits must not depend on that); a larger one may still decide.
+    *out = &general;
+    if (kind != FK_C2C && P.n < kShortRow && lines_hint * P.n < kShortValues)
         return 0;
+    if (slot) {
+        *out = slot.get();
+        return 0;
+    }
     if (!P.single || !env_flag("KISSFFT_AMD_FAST", true))
         return decide(std::make_shared<const FastChoice>());
-    if (kind != FK_C2C && P.n < kShortRow && lines_hint * P.n < kShortValues)
-        return 0;  // the general kernel; a larger batch may still decide
     std::vector<const FastVariant *> cand;
     for (const FastVariant &v : fast_registry()) {
         if (v.type != P.type || v.kind != kind || v.n != P.n || v.inverse != P.inverse)

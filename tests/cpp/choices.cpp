@@ -2,6 +2,7 @@
 // needed: plans are filled in by hand and nothing is launched.
 //     choices CASE        exit status 0: the case holds
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
 #include <memory>
 
@@ -39,6 +40,24 @@ static int open_choice_is_not_the_plans()
         CHECK(fc && !fc->v && !fc->d_stw);
         const char *at = reinterpret_cast<const char *>(fc), *p0 = reinterpret_cast<const char *>(&P);
         CHECK(at < p0 || at >= p0 + sizeof P);
+    }
+    return 0;
+}
+
+// A small batch of short real rows runs on the general kernel also after a large one of the
+// same plan was given a compiled kernel.
+static int short_real_rows_do_not_depend_on_the_past()
+{
+    static const FastVariant compiled{};
+    for (int kind : {FK_R2C, FK_C2R}) {
+        DevPlan P;
+        single_plan(P, KFA_F32, 8, {4, 2});
+        auto c = std::make_shared<FastChoice>();
+        c->v = &compiled;
+        P.fast[kind] = c;
+        const FastChoice *fc = nullptr;
+        CHECK(choose_fast(P, kind, nullptr, &fc, 3) == 0 && !fc->v);
+        CHECK(choose_fast(P, kind, nullptr, &fc, 1 << 20) == 0 && fc->v == &compiled);
     }
     return 0;
 }
@@ -88,6 +107,7 @@ int main(int argc, char **argv)
         int (*run)();
     } cases[] = {
         {"open_choice_is_not_the_plans", open_choice_is_not_the_plans},
+        {"short_real_rows_do_not_depend_on_the_past", short_real_rows_do_not_depend_on_the_past},
         {"short_complex_lines_are_decided", short_complex_lines_are_decided},
         {"fixed_split_needs_no_allocation", fixed_split_needs_no_allocation},
     };
