@@ -1522,7 +1522,7 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
     // A small batch of short real rows runs on the general kernel whatever ran before it (its
     // float bits must not depend on that); a larger one may still decide.
     *out = &general;
-    if (kind != FK_C2C && P.n < kShortRow && lines_hint * P.n < kShortValues)
+    if (kind != FK_C2C && P.n < kShortRow && lines_hint * P.n < kShortValues && !rtc_min_set())
         return 0;
     if (slot) {
         *out = slot.get();

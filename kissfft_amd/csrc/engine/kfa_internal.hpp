@@ -165,6 +165,8 @@ int choose_fast(DevPlan &P, int kind, hipStream_t s, const FastChoice **out, lon
 // values; no complex row is
 constexpr int kShortRow = 16;
 constexpr long long kShortValues = 1LL << 16;
+// whether the caller sets the shortest compiled row (KISSFFT_AMD_RTC_MIN): batches of any size then
+bool rtc_min_set();
 // runtime-compiled variants of a plan's length and kind (kfa_rtc.hip), when none is built in
 int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> &out);
 // the runtime-compiled tile kernel of schedule `radices` (kfa_tile.hpp; tm: TM_* mapping

@@ -677,6 +677,12 @@ int fast_launch(const FastVariant &v, const FastArgs &a, hipStream_t s)
     return v.rtc ? rtc_launch(v, a, s) : v.launch(a, s);
 }
 
+bool rtc_min_set()
+{
+    const char *v = getenv("KISSFFT_AMD_RTC_MIN");
+    return v && *v;
+}
+
 // Runtime-compiled candidates for plan P and transform kind `kind` (none when the path is
 // off, the length has another radix, or nothing compiles).
 int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> &out)
@@ -685,8 +691,7 @@ int rtc_candidates(const DevPlan &P, int kind, std::vector<const FastVariant *> 
     // of short lines run 3-8 times
     // faster compiled than on the general kernel (2^29 bytes per side: Q15 120 points
     // 2.88 against 0.37 TB/s, float 60 points 3.96 against 0.78)
-    const char *mv = getenv("KISSFFT_AMD_RTC_MIN");
-    const int min_n = mv && *mv ? atoi(mv) : kind == FK_C2C ? kShortRow : 4;
+    const int min_n = rtc_min_set() ? atoi(getenv("KISSFFT_AMD_RTC_MIN")) : kind == FK_C2C ? kShortRow : 4;
     if (!env_flag("KISSFFT_AMD_RTC", true) || !P.single || P.n < std::max(2, min_n))
         return 0;
     // factors of 17 .. 31: rows above 2048 points and real ones (shorter complex rows run

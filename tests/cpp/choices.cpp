@@ -62,6 +62,18 @@ static int short_real_rows_do_not_depend_on_the_past()
     return 0;
 }
 
+// A caller who sets the shortest compiled row gets it for batches of any size.
+static int shortest_compiled_row_as_set()
+{
+    setenv("KISSFFT_AMD_RTC_MIN", "8", 1);
+    setenv("KISSFFT_AMD_RTC", "0", 1);  // (nothing is compiled here)
+    DevPlan P;
+    single_plan(P, KFA_F32, 8, {4, 2});
+    const FastChoice *fc = nullptr;
+    CHECK(choose_fast(P, FK_R2C, nullptr, &fc, 3) == 0 && P.fast[FK_R2C]);
+    return 0;
+}
+
 // While the no-allocation entry point runs, choices that would allocate are refused.
 struct NoAlloc {
     NoAlloc() { thread_noalloc() = true; }
@@ -108,6 +120,7 @@ int main(int argc, char **argv)
     } cases[] = {
         {"open_choice_is_not_the_plans", open_choice_is_not_the_plans},
         {"short_real_rows_do_not_depend_on_the_past", short_real_rows_do_not_depend_on_the_past},
+        {"shortest_compiled_row_as_set", shortest_compiled_row_as_set},
         {"short_complex_lines_are_decided", short_complex_lines_are_decided},
         {"fixed_split_needs_no_allocation", fixed_split_needs_no_allocation},
     };
