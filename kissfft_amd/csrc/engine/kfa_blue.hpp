@@ -10,7 +10,8 @@
 // i.e. X = w * IFFT_M( FFT_M(x*w, zero-padded) * B ),  B = FFT_M(conj(w) wrapped) / M.
 // One line per T threads, entirely in LDS: the chirp multiply on load, the forward M-point
 // schedule, the pointwise product with B, the inverse schedule, the chirp on store.
-// w (N entries) and B (M entries) are computed in FP64 on the host and rounded once.
+// w (N entries) and B (M entries) are computed in FP64 on the host; B is rounded once, w by
+// the variants that read it in float.
 #pragma once
 
 #include "kfa_tile.hpp"
@@ -150,7 +151,8 @@ struct BlueArgs {
     const void *in;
     void *out;
     const void *stw_f, *stw_i;  // stage tables of the M-point schedule, and of it backwards
-    const void *chirp;          // w[n], n < N
+    const void *chirp;          // w[n], n < N, float2
+    const void *chirp64;        // the same in FP64 (null where no variant of the length reads it)
     const void *bfft;           // B[m], m < M
     int n;
     long long nlines;
@@ -159,8 +161,21 @@ struct BlueArgs {
     FastSeg seg[KFA_MAX_SEG];
 };
 
+// Entries of the chirp table.
+template <bool WIDE>
+struct Chirp {
+    typedef float2 type;
+    __device__ __forceinline__ static const type *of(const BlueArgs &a) { return reinterpret_cast<const type *>(a.chirp); }
+};
+template <>
+struct Chirp<true> {
+    typedef Cd type;
+    __device__ __forceinline__ static const type *of(const BlueArgs &a) { return reinterpret_cast<const type *>(a.chirp64); }
+};
+
 // The Bluestein body for workgroup `blk` of its launch (see k_fast_body).
-template <int T, int LPB, class RS>
+// WIDE: the products with the chirp on load (bit 0) and on store (bit 1) in FP64.
+template <int T, int LPB, int WIDE, class RS>
 __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
 {
     typedef F32::store2 St;
@@ -176,7 +191,8 @@ __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
     const long long gl = blk * LPB + line;
     const bool ok = gl < a.nlines;
     const int n = a.n;
-    const St *chirp = reinterpret_cast<const St *>(a.chirp);
+    const auto *chirp_in = Chirp<(WIDE & 1) != 0>::of(a);
+    const auto *chirp_out = Chirp<(WIDE & 2) != 0>::of(a);
 
     const St *src;
     St *dst;
@@ -187,7 +203,7 @@ __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
 #pragma unroll
         for (int r = 0; r < In::p; ++r) {
             const int i = t + j * T + r * In::NB;
-            v[j][r] = (ok && i < n) ? O::cmul(O::load(src[(long long)i * a.in_el]), O::load(chirp[i])) : O::zero();
+            v[j][r] = (ok && i < n) ? conv_mul(O::load(src[(long long)i * a.in_el]), chirp_in[i]) : O::zero();
         }
     CV::run(v, out, buf, reinterpret_cast<const St *>(a.stw_f), reinterpret_cast<const St *>(a.stw_i),
             reinterpret_cast<const St *>(a.bfft), t);
@@ -199,14 +215,14 @@ __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
         for (int q = 0; q < Out::p; ++q) {
             const int i = t + j * T + q * Out::NB;
             if (i < n)
-                dst[(long long)i * a.out_el] = O::pack(O::cmul(out[j][q], O::load(chirp[i])));
+                dst[(long long)i * a.out_el] = O::pack(conv_mul(out[j][q], chirp_out[i]));
         }
 }
 
-template <int T, int LPB, class RS>
+template <int T, int LPB, int WIDE, class RS>
 __global__ void __launch_bounds__(T *LPB) k_blue(BlueArgs a)
 {
-    k_blue_body<T, LPB, RS>(a, blockIdx.x);
+    k_blue_body<T, LPB, WIDE, RS>(a, blockIdx.x);
 }
 
 }  // namespace kfa

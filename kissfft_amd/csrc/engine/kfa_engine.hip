@@ -1094,7 +1094,7 @@ static int launch_rtile(const TileChoice &tc, RealTileArgs a, long long howmany,
 // ------------------------------------------------------------------------------------
 struct BlueChoice {
     const BlueVariant *v = nullptr;
-    DevBuf mem_f, mem_i, mem_chirp, mem_bfft;
+    DevBuf mem_f, mem_i, mem_chirp, mem_chirp64, mem_bfft;
     const BlueVariant *vf = nullptr;  // in a multi-batch (null: v there too), with its stage tables
     DevBuf fmem_f, fmem_i;
 };
@@ -1167,13 +1167,15 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
         const int M = bc->v->M;
         const double pi = 3.14159265358979323846264338327;
         const double sg = P.inverse ? 1.0 : -1.0;
-        std::vector<double> wr(n), wi(n);
+        std::vector<double> wr(n), wi(n), hw64(2 * n);
         std::vector<float> hw(2 * n);
         for (long long i = 0; i < n; ++i) {
             const long long q = (i * i) % (2 * n);  // n^2 mod 2N: exact phase reduction
             const double ph = sg * pi * (double)q / (double)n;
             wr[i] = cos(ph);
             wi[i] = sin(ph);
+            hw64[2 * i] = wr[i];
+            hw64[2 * i + 1] = wi[i];
             hw[2 * i] = (float)wr[i];
             hw[2 * i + 1] = (float)wi[i];
         }
@@ -1203,6 +1205,8 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
         if ((rc = stage_tables(*bc->v, bc->mem_f, bc->mem_i)) ||
             (bc->vf && (rc = stage_tables(*bc->vf, bc->fmem_f, bc->fmem_i))) ||
             (rc = dev_upload(hw.data(), hw.size() * 4, bc->mem_chirp)) ||
+            ((bc->v->wide || (bc->vf && bc->vf->wide)) &&
+             (rc = dev_upload(hw64.data(), hw64.size() * 8, bc->mem_chirp64))) ||
             (rc = dev_upload(hb.data(), hb.size() * 4, bc->mem_bfft)))
             return rc;
         if (env_flag("KISSFFT_AMD_VERBOSE", false))
@@ -1219,6 +1223,7 @@ static void blue_args(const BlueChoice &bc, int n, BlueArgs &b)
     b.stw_f = bc.mem_f.get();
     b.stw_i = bc.mem_i.get();
     b.chirp = bc.mem_chirp.get();
+    b.chirp64 = bc.mem_chirp64.get();
     b.bfft = bc.mem_bfft.get();
     b.n = n;
 }

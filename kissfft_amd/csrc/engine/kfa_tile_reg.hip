@@ -262,23 +262,23 @@ const std::vector<PlaneVariant> &plane_registry()
     return *reg;
 }
 
-template <int T, int LPB, class RS>
+template <int T, int LPB, int WIDE, class RS>
 static int launch_blue(const BlueArgs &a, hipStream_t s)
 {
     const size_t lds = (size_t)LPB * conv_slots(RS::N()) * sizeof(float2);
     static std::once_flag once;
     std::call_once(once, [=] {
-        (void)hipFuncSetAttribute((const void *)k_blue<T, LPB, RS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        (void)hipFuncSetAttribute((const void *)k_blue<T, LPB, WIDE, RS>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)lds);
     });
     const long long blocks = (a.nlines + LPB - 1) / LPB;
     if (blocks <= 0)
         return 0;
-    hipLaunchKernelGGL((k_blue<T, LPB, RS>), dim3((unsigned)blocks), dim3(T * LPB), lds, s, a);
+    hipLaunchKernelGGL((k_blue<T, LPB, WIDE, RS>), dim3((unsigned)blocks), dim3(T * LPB), lds, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-template <int T, int LPB, int... R>
+template <int T, int LPB, int WIDE, int... R>
 static void add_blue(std::vector<BlueVariant> &v, const char *name, bool fused = false)
 {
     typedef Radices<2, R...> RS;
@@ -291,7 +291,8 @@ static void add_blue(std::vector<BlueVariant> &v, const char *name, bool fused =
     f.tw_pad = 2;
     f.lds = (size_t)LPB * conv_slots(RS::N()) * 8;
     f.name = name;
-    f.launch = &launch_blue<T, LPB, RS>;
+    f.wide = WIDE;
+    f.launch = &launch_blue<T, LPB, WIDE, RS>;
     f.fused = fused;
     v.push_back(f);
 }
@@ -300,19 +301,26 @@ const std::vector<BlueVariant> &blue_registry()
 {
     static std::vector<BlueVariant> *reg = [] {
         auto *v = new std::vector<BlueVariant>();
-        add_blue<8, 8, 8, 8>(*v, "blue64_88_t8x8");
-        add_blue<8, 8, 8, 16>(*v, "blue128_816_t8x8");
-        add_blue<16, 4, 16, 16>(*v, "blue256_1616_t16x4");
-        add_blue<64, 2, 8, 8, 8>(*v, "blue512_888_t64x2");
-        add_blue<128, 2, 8, 8, 4, 4>(*v, "blue1024_8844_t128x2");
+        // The chirp on load in FP64 (third argument 1) for 64, 128, 512 points and the fused
+        // 2048: with both products in float they are 0.4 .. 1 % less exact than with the line
+        // staged through LDS between the steps (512 points 1.411e-7 rel-L2 against 1.405e-7, now
+        // 1.385e-7; 2048 fused 1.617e-7 against 1.610e-7, now 1.595e-7).  On load and store
+        // it takes 3 % of the time of 64 .. 512 points, on load alone 1-2 %; 64 uneven batches in
+        // one fused launch 43.4 / 43.9 / 44.3 us with none, load, both.  Both (3) from 8192 points,
+        // where it costs nothing that can be measured: -2.8 % of the error.
+        add_blue<8, 8, 1, 8, 8>(*v, "blue64_88_t8x8");
+        add_blue<8, 8, 1, 8, 16>(*v, "blue128_816_t8x8");
+        add_blue<16, 4, 0, 16, 16>(*v, "blue256_1616_t16x4");
+        add_blue<64, 2, 1, 8, 8, 8>(*v, "blue512_888_t64x2");
+        add_blue<128, 2, 0, 8, 8, 4, 4>(*v, "blue1024_8844_t128x2");
         // c2c 1009 x4096 27.4 us, 32.2 with 128 threads a line, 30.9 with 16, 16, 8 at 128; but
         // 64 uneven batches in one fused launch 45.1, 45.1 and 43.4 us
-        add_blue<256, 1, 8, 8, 8, 4>(*v, "blue2048_8884_t256");
-        add_blue<128, 2, 16, 16, 8>(*v, "blue2048_16168_t128x2", true);
-        add_blue<512, 1, 8, 8, 8, 8>(*v, "blue4096_8888_t512");
+        add_blue<256, 1, 0, 8, 8, 8, 4>(*v, "blue2048_8884_t256");
+        add_blue<128, 2, 1, 16, 16, 8>(*v, "blue2048_16168_t128x2", true);
+        add_blue<512, 1, 0, 8, 8, 8, 8>(*v, "blue4096_8888_t512");
         // lengths above 2048: 4093 x8 10.7 ms -> 16 us, 5002 x8 319 -> 23 us against the general kernel
-        add_blue<512, 1, 8, 8, 8, 4, 4>(*v, "blue8192_88844_t512");
-        add_blue<1024, 1, 8, 8, 8, 8, 4>(*v, "blue16384_88884_t1024");
+        add_blue<512, 1, 3, 8, 8, 8, 4, 4>(*v, "blue8192_88844_t512");
+        add_blue<1024, 1, 3, 8, 8, 8, 8, 4>(*v, "blue16384_88884_t1024");
         return v;
     }();
     return *reg;
