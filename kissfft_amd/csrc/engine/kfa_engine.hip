@@ -1130,23 +1130,39 @@ static void fft_pow2_f64(std::vector<double> &re, std::vector<double> &im)
     }
 }
 
-// The Bluestein variant and tables for a float plan (v == nullptr when the plan has no
-// prime factor above 16, above 2048 points none above 50, or no registered convolution
-// length fits), decided once per plan.
+static int largest_radix(const DevPlan &P)
+{
+    return *std::max_element(P.radix.begin(), P.radix.end());
+}
+
+// Whether Bluestein's convolution is at least as exact as float butterflies that sum the
+// products of the plan's largest factor directly, which is what the reference computes.  It is 5 to
+// 1800 times faster than direct sums (4028 = 4 19 53 x256 18 against 177 us, 4093 x64 16 us against
+// 10.7 ms), but its error does not depend on the factor: it grows with the filled part of the
+// M points, 2n / M, where a direct sum's grows with the factor.  Over all 1832 lengths to 8192
+// with a largest factor of 53 .. 97, complex ones and real halves, its error is at most 1.00 times
+// that of float direct sums for factors above 73, and at most 0.99 times for 53 .. 73 up to
+// 2n / M = 0.7, from where it reaches 1.12 (8162 = 2 7 11 53: 1.96e-7 against 1.74e-7).  The lengths
+// it is not taken for run on the general kernel, whose sums are FP64 (8162: 0.7e-7).
+static bool blue_exact(const DevPlan &P)
+{
+    const int p = largest_radix(P);
+    long long M = 64;
+    while (M < 2LL * P.n - 1)
+        M *= 2;
+    return p > 73 || (p > 50 && 20LL * P.n <= 7 * M);
+}
+
+// The Bluestein variant and tables for a float plan, decided once per plan.  v == nullptr: up to
+// 2048 points the plan has no prime factor above 16; above, the direct sums are the more
+// exact (blue_exact) or no registered convolution length fits.
 static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
 {
     static const std::shared_ptr<const BlueChoice> none = std::make_shared<const BlueChoice>();
     out = none;
     if (P.type != KFA_F32 || !P.single || !env_flag("KISSFFT_AMD_BLUESTEIN", true))
         return 0;
-    int pmax = 0;
-    for (int p : P.radix)
-        pmax = std::max(pmax, p);
-    // Above 2048 points the general kernel's direct sums over a factor up to 50 are the more
-    // exact (6800 = 2^4 5^2 17: 1.41e-7 rel-L2 against Bluestein's 1.84e-7; 5002 = 2 41 61
-    // 1.96e-7 against 1.65e-7, 4093 1.15e-6 against 1.90e-7), and those of 17 .. 31 have
-    // compiled rows.
-    if (pmax <= (P.n > 2048 ? 50 : 16))
+    if (P.n > 2048 ? !blue_exact(P) : largest_radix(P) <= 16)
         return 0;
     std::lock_guard<std::mutex> g(P.mu);
     if (P.blue_decided) {
@@ -2296,16 +2312,13 @@ int prepare_multipass(DevPlan &P, int fk, hipStream_t s)
     return rc;
 }
 
-// Real rows with a half length of at most one line that has a prime factor above 50: the
-// complex transform on Bluestein's kernel and the split (merge) as a pass of its own
-// instead of direct sums over the factor (80 x 1126 x34 there and back 1461 -> 62 us).  Smaller
-// factors have compiled rows (to 31) or the more exact direct sums.
+// Real rows with a half length of at most one line for which Bluestein's kernel is exact enough
+// (blue_exact): the complex transform on it and the split (merge) as a pass of its own
+// instead of direct sums over the factor (80 x 1126 x34 there and back 1461 -> 62 us).  Factors to 31
+// have compiled rows.
 bool blue_real_rows(const DevPlan &P)
 {
-    int pmax = 0;
-    for (int p : P.radix)
-        pmax = std::max(pmax, p);
-    return P.type == KFA_F32 && P.single && pmax > 50 && env_flag("KISSFFT_AMD_BLUESTEIN", true);
+    return P.type == KFA_F32 && P.single && blue_exact(P) && env_flag("KISSFFT_AMD_BLUESTEIN", true);
 }
 
 // Real rows whose half length needs the multi-pass complex transform (or Bluestein's kernel).  Float lengths with

@@ -74,6 +74,31 @@ static int shortest_compiled_row_as_set()
     return 0;
 }
 
+// Lengths whose direct sums are more exact than Bluestein's convolution keep them: factors up to
+// 73 in a convolution that is more than 0.7 full.
+static int bluestein_only_where_exact()
+{
+    const struct {
+        std::vector<int> radix;
+        bool real;  // Bluestein for real rows of this half length
+    } v[] = {{{53, 19}, false},         {{53, 19, 2}, false}, {{53, 19, 4}, false}, {{53, 11, 7}, false},
+             {{53, 5, 5, 3, 2}, false}, {{53, 17, 9}, false}, {{73, 109}, true},    {{53, 53}, true},
+             {{79, 101}, true},         {{1021, 2}, true},    {{47, 47}, false},    {{61, 16, 4}, false}};
+    for (const auto &x : v) {
+        DevPlan P;
+        int n = 1;
+        for (int p : x.radix)
+            n *= p;
+        single_plan(P, KFA_F32, n, x.radix);
+        CHECK(blue_real_rows(P) == x.real);
+        if (x.real || n <= 2048)
+            continue;
+        bool applies = true;  // complex lines: no table is built (there is no device here)
+        CHECK(blue_prepare(P, &applies) == 0 && !applies);
+    }
+    return 0;
+}
+
 // While the no-allocation entry point runs, choices that would allocate are refused.
 struct NoAlloc {
     NoAlloc() { thread_noalloc() = true; }
@@ -121,6 +146,7 @@ int main(int argc, char **argv)
         {"open_choice_is_not_the_plans", open_choice_is_not_the_plans},
         {"short_real_rows_do_not_depend_on_the_past", short_real_rows_do_not_depend_on_the_past},
         {"shortest_compiled_row_as_set", shortest_compiled_row_as_set},
+        {"bluestein_only_where_exact", bluestein_only_where_exact},
         {"short_complex_lines_are_decided", short_complex_lines_are_decided},
         {"fixed_split_needs_no_allocation", fixed_split_needs_no_allocation},
     };

@@ -167,3 +167,26 @@ def test_float_real_rows_with_large_primes(n):
     torch.cuda.synchronize()
     lib.kiss_fftr(lib.fftr_alloc(n), one, one)
     np.testing.assert_array_equal(one.cpu().numpy().reshape(-1, 2), X[0])
+
+
+@pytest.mark.parametrize("n", [1007, 2014, 4028, 4081, 7950, 8109, 8162])
+def test_factor_53_is_as_exact_as_direct_sums(n):
+    """Lengths with a factor of 53 in a nearly full convolution keep direct sums, summed in FP64:
+    a stage rounds its inputs' twiddle products and its result, so 3 or 4 stages stay within
+    sqrt(2 * 4) * 2^-24 * 0.6 = 1.0e-7; 1.5e-7 leaves half as much again.  Float sums are at
+    1.7e-7 and Bluestein's convolution at 1.9e-7.  Real rows of this half length, and complex
+    lines of it above 2048 points."""
+    lib = kissfft_amd.load("float")
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((16, 2 * n)).astype(np.float32)
+    X = np.zeros((16, n + 1, 2), np.float32)
+    lib.fftr_batch(lib.fftr_alloc(2 * n), x, X, 16, 2 * n, n + 1)
+    assert rel_l2(cplx(X), np.fft.rfft(x.astype(np.float64), axis=-1)) <= 1.5e-7
+    if n <= 2048:
+        return
+    z = x.reshape(16, n, 2)
+    for inv in (False, True):
+        y = np.zeros_like(z)
+        lib.fft_batch(lib.fft_alloc(n, inv), z, y, 16, n, n)
+        want = np.fft.ifft(cplx(z), axis=-1) * n if inv else np.fft.fft(cplx(z), axis=-1)
+        assert rel_l2(cplx(y), want) <= 1.5e-7, inv
