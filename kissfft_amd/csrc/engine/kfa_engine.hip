@@ -314,6 +314,25 @@ void free_deferred()
         (void)hipFree(p);  // waits for the device before freeing
 }
 
+// The device's stream for table uploads, non-blocking: a copy on the legacy stream would end a
+// capture under way on any blocking stream, also the one whose call needs the table.
+static int upload_stream(hipStream_t *s)
+{
+    static std::mutex mu;
+    static std::map<int, hipStream_t> streams;
+    int dev = 0;
+    KFA_HIP(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> g(mu);
+    auto it = streams.find(dev);
+    if (it == streams.end()) {
+        hipStream_t t = nullptr;
+        KFA_HIP(hipStreamCreateWithFlags(&t, hipStreamNonBlocking));  // default priority
+        it = streams.emplace(dev, t).first;
+    }
+    *s = it->second;
+    return 0;
+}
+
 int dev_upload(const void *host, size_t bytes, DevBuf &out)
 {
     if (thread_noalloc())
@@ -321,8 +340,13 @@ int dev_upload(const void *host, size_t bytes, DevBuf &out)
     void *p = nullptr;
     KFA_HIP(hipMalloc(&p, bytes ? bytes : 1));
     out = DevBuf(p, defer_free);
-    if (bytes && host)
-        KFA_HIP(hipMemcpy(p, host, bytes, hipMemcpyHostToDevice));
+    if (bytes && host) {
+        hipStream_t s = nullptr;
+        if (int rc = upload_stream(&s))
+            return rc;
+        KFA_HIP(hipMemcpyAsync(p, host, bytes, hipMemcpyHostToDevice, s));
+        KFA_HIP(hipStreamSynchronize(s));
+    }
     return 0;
 }
 

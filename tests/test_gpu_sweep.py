@@ -190,3 +190,28 @@ def test_factor_53_is_as_exact_as_direct_sums(n):
         lib.fft_batch(lib.fft_alloc(n, inv), z, y, 16, n, n)
         want = np.fft.ifft(cplx(z), axis=-1) * n if inv else np.fft.fft(cplx(z), axis=-1)
         assert rel_l2(cplx(y), want) <= 1.5e-7, inv
+
+
+def test_tables_made_under_capture():
+    """A call captured on a blocking stream whose length needs tables that no call has made yet
+    (4093: Bluestein's): they are uploaded without ending the capture, and every replay
+    gives the transform of the input of that moment."""
+    import torch
+    n, b = 4093, 4
+    lib = kissfft_amd.load("float")
+    lib.L.kiss_fft_cleanup()
+    x = torch.from_numpy(np.random.default_rng(n).uniform(-1, 1, (b, n, 2)).astype(np.float32)).cuda()
+    y = torch.empty_like(x)
+    cfg, st, g = lib.fft_alloc(n), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    lib.fft_batch(cfg, x, y, 0, n, n)  # (the device plan alone)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
+        lib.fft_batch(cfg, x, y, b, n, n, stream=st)
+    for rep in range(3):
+        x.mul_(1.25).add_(0.25)
+        y.fill_(9.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            g.replay()
+        torch.cuda.synchronize()
+        assert rel_l2(cplx(y.cpu().numpy()), np.fft.fft(cplx(x.cpu().numpy()), axis=-1)) <= ABS_FLOAT_BOUND, rep
