@@ -1482,15 +1482,11 @@ static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPl
         if (n % N1 == 0 && n / N1 <= kTileLongest && (made1 == 0 || score(N1) < score(made1)) &&
             float_schedule((int)N1, true).size() > 1 && !float_schedule((int)(n / N1), true).empty())
             made1 = N1;
-    if (made1 && (best1 == 0 || score(best1) > 1.5 * score(made1))) {
-        if (stream_capturing(s))
-            return 0;  // nothing is compiled now: the choice stays open
-        best1 = made1;
-    }
-    if (best1) {
+    // the split of N1 columns, or null: a tile of it cannot be had
+    auto build = [&](long long N1, std::shared_ptr<const BaileyPlan> &plan) {
         auto bp = std::make_shared<BaileyPlan>();
-        bp->N1 = best1;
-        bp->N2 = n / best1;
+        bp->N1 = N1;
+        bp->N2 = n / N1;
         BufPair tw;
         int rc;
         if ((rc = tile_choice((int)bp->N1, P.inverse, TILE_ROWS_TO_COLS, s, bp->c2)) ||
@@ -1499,9 +1495,30 @@ static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPl
             return rc;
         bp->tw_hi = tw.first;
         bp->tw_lo = tw.second;
-        if (bp->c1->v && bp->c2->v)
-            P.bailey = bp;
+        if (bp->c1->v && bp->c2->v) {
+            plan = bp;
+            if (env_flag("KISSFFT_AMD_VERBOSE", false))
+                fprintf(stderr, "[kissfft_amd] four-step n=%lld inverse=%d: columns %s, rows %s\n", n, P.inverse,
+                        bp->c1->v->name, bp->c2->v->name);
+        }
+        return 0;
+    };
+    int rc;
+    if (made1 && (best1 == 0 || score(best1) > 1.5 * score(made1))) {
+        if (stream_capturing(s)) {
+            // nothing is compiled now: the built-in split, if there is one, for this call (the plan
+            // keeps it, a graph may hold its tables), and the choice stays open
+            if (best1 && !P.bailey_builtin && (rc = build(best1, P.bailey_builtin)))
+                return rc;
+            out = P.bailey_builtin;
+            return 0;
+        }
+        if ((rc = build(made1, P.bailey)))
+            return rc;
     }
+    // (a compiled one may not be had: no runtime compiler, or no shape without scratch)
+    if (!P.bailey && best1 && (rc = build(best1, P.bailey)))
+        return rc;
     P.bailey_decided = true;
     out = P.bailey;
     return 0;

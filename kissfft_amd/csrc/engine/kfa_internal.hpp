@@ -75,6 +75,7 @@ struct DevPlan {
     std::shared_ptr<const FastChoice> fast[3];  // per FK_C2C / FK_R2C / FK_C2R; null: undecided
     bool bailey_decided = false;
     std::shared_ptr<const BaileyPlan> bailey;
+    std::shared_ptr<const BaileyPlan> bailey_builtin;  // for captured calls while the choice is open
     bool rfused_decided[2] = {false, false};
     std::shared_ptr<const RealFusedPlan> rfused[2];  // per direction
     bool blue_decided = false;

@@ -5,6 +5,8 @@ fixed-point builds' reference-order split, whose second pass reads its own rows 
 full-length twiddle tables (TM_REF in kfa_tile.hpp).  Fixed point is bit-exact against the
 oracle, float within the float bar of FP64; contiguous and strided input, both directions.
 """
+import re
+
 import numpy as np
 import pytest
 
@@ -53,3 +55,58 @@ def test_two_pass_lines(n, dtype, monkeypatch, capfd):
     else:
         np.testing.assert_array_equal(ys, Oracle(dtype).fft(xd))
     assert "tile" in capfd.readouterr().err
+
+
+def float_error(y, x):
+    return rel_l2(cplx(y), np.fft.fft(cplx(x), axis=-1))
+
+
+# 96 x 512 and 96 x 1024: built-in halves, less balanced than a split that can be compiled
+@pytest.mark.parametrize("n", [49152, 98304])
+def test_builtin_split_without_the_compiler(n, monkeypatch, capfd):
+    """With the runtime compiler off a length whose preferred split would be compiled runs its
+    built-in one, not the general kernel."""
+    lib = kissfft_amd.load("float")
+    x = rnd(np.random.default_rng(n), "float", (2, n, 2))
+    y = np.zeros_like(x)
+    monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    monkeypatch.setenv("KISSFFT_AMD_RTC", "0")
+    lib.L.kiss_fft_cleanup()
+    try:
+        lib.fft_batch(lib.fft_alloc(n), x, y, 2, n, n)
+    finally:
+        lib.L.kiss_fft_cleanup()
+    assert float_error(y, x) <= ABS_FLOAT_BOUND
+    split = re.findall(rf"four-step n={n} inverse=0: columns h?tile(\d+)_\S+, rows h?tile(\d+)_", capfd.readouterr().err)
+    assert len(split) == 1 and int(split[0][0]) * int(split[0][1]) == n, split
+
+
+def test_captured_first_call_runs_the_builtin_split(monkeypatch, capfd):
+    """A first call under capture compiles nothing: it takes the built-in split, and a later
+    eager call still gets the compiled one.  Every replay, also after that call, gives the
+    transform of the input of that moment."""
+    import torch
+    n, b = 98304, 2
+    lib = kissfft_amd.load("float")
+    monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    lib.L.kiss_fft_cleanup()
+    x = torch.from_numpy(rnd(np.random.default_rng(5), "float", (b, n, 2))).cuda()
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    cfg, st, g = lib.fft_alloc(n), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    lib.fft_batch(cfg, x, y, 0, n, n)  # (the device plan alone)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
+        lib.fft_batch(cfg, x, y, b, n, n, stream=st)
+    err = capfd.readouterr().err
+    assert re.search(rf"four-step n={n} inverse=0: columns h?tile\d+_\S+, rows h?tile\d+_", err), err
+    for rep in range(3):
+        x.mul_(1.25).add_(0.25)
+        y.fill_(9.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            g.replay()
+        torch.cuda.synchronize()
+        assert float_error(y.cpu().numpy(), x.cpu().numpy()) <= ABS_FLOAT_BOUND, rep
+        lib.fft_batch(cfg, x, z, b, n, n)
+        assert float_error(z.cpu().numpy(), x.cpu().numpy()) <= ABS_FLOAT_BOUND, rep
+    assert re.search(rf"four-step n={n} inverse=0: columns .*rtc_tile", capfd.readouterr().err)
