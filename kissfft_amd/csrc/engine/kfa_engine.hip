@@ -74,32 +74,36 @@ size_t cpx_bytes(int type) { return type == KFA_Q15 ? 4 : 8; }
 static std::mutex g_pool_mu;
 static std::map<int, hipMemPool_t> g_pools;
 
-hipError_t scratch_alloc(void **p, size_t bytes, hipStream_t s)
+static hipError_t scratch_pool(hipMemPool_t *pool)
 {
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess)
         return e;
-    hipMemPool_t pool;
-    {
-        std::lock_guard<std::mutex> g(g_pool_mu);
-        auto it = g_pools.find(dev);
-        if (it == g_pools.end()) {
-            hipMemPoolProps props = {};
-            props.allocType = hipMemAllocationTypePinned;
-            props.handleTypes = hipMemHandleTypeNone;
-            props.location.type = hipMemLocationTypeDevice;
-            props.location.id = dev;
-            if ((e = hipMemPoolCreate(&pool, &props)) != hipSuccess)
-                return e;
-            uint64_t keep = ~0ULL;
-            (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-            g_pools[dev] = pool;
-        } else {
-            pool = it->second;
-        }
+    std::lock_guard<std::mutex> g(g_pool_mu);
+    auto it = g_pools.find(dev);
+    if (it == g_pools.end()) {
+        hipMemPoolProps props = {};
+        props.allocType = hipMemAllocationTypePinned;
+        props.handleTypes = hipMemHandleTypeNone;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id = dev;
+        if ((e = hipMemPoolCreate(pool, &props)) != hipSuccess)
+            return e;
+        uint64_t keep = ~0ULL;
+        (void)hipMemPoolSetAttribute(*pool, hipMemPoolAttrReleaseThreshold, &keep);
+        g_pools[dev] = *pool;
+    } else {
+        *pool = it->second;
     }
-    return hipMallocFromPoolAsync(p, bytes ? bytes : 1, pool, s);
+    return hipSuccess;
+}
+
+hipError_t scratch_alloc(void **p, size_t bytes, hipStream_t s)
+{
+    hipMemPool_t pool;
+    const hipError_t e = scratch_pool(&pool);
+    return e == hipSuccess ? hipMallocFromPoolAsync(p, bytes ? bytes : 1, pool, s) : e;
 }
 
 static void scratch_trim()
@@ -254,6 +258,9 @@ int StreamMem::get(size_t bytes, hipStream_t s)
     put();
     s_ = s;
     if (!stream_capturing(s)) {
+        // (the pool cannot be created under capture: an eager call has it ready for a captured one)
+        hipMemPool_t pool;
+        KFA_HIP(scratch_pool(&pool));
         int dev = 0;
         KFA_HIP(hipGetDevice(&dev));
         bool wait = false;

@@ -5,12 +5,16 @@ fixed-point builds' reference-order split, whose second pass reads its own rows 
 full-length twiddle tables (TM_REF in kfa_tile.hpp).  Fixed point is bit-exact against the
 oracle, float within the float bar of FP64; contiguous and strided input, both directions.
 """
+import os
 import re
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
 import kissfft_amd
+from conftest import ROOT
 from helpers import ABS_FLOAT_BOUND, cplx, rel_l2
 from oracle import Oracle
 
@@ -93,7 +97,9 @@ def test_captured_first_call_runs_the_builtin_split(monkeypatch, capfd):
     x = torch.from_numpy(rnd(np.random.default_rng(5), "float", (b, n, 2))).cuda()
     y, z = torch.empty_like(x), torch.empty_like(x)
     cfg, st, g = lib.fft_alloc(n), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    lib.fft_batch(lib.fft_alloc(65536), x, y, 1, 65536, 65536)  # (the pool of captured temporaries)
     lib.fft_batch(cfg, x, y, 0, n, n)  # (the device plan alone)
+    capfd.readouterr()
     torch.cuda.synchronize()
     with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
         lib.fft_batch(cfg, x, y, b, n, n, stream=st)
@@ -110,3 +116,35 @@ def test_captured_first_call_runs_the_builtin_split(monkeypatch, capfd):
         lib.fft_batch(cfg, x, z, b, n, n)
         assert float_error(z.cpu().numpy(), x.cpu().numpy()) <= ABS_FLOAT_BOUND, rep
     assert re.search(rf"four-step n={n} inverse=0: columns .*rtc_tile", capfd.readouterr().err)
+
+
+CAPTURED = """
+import numpy as np, torch, kissfft_amd
+n, b = 65536, 3
+lib = kissfft_amd.load("int16_t")
+x = torch.from_numpy(np.random.default_rng(1).integers(-9999, 9999, (b, n, 2)).astype(np.int16)).cuda()
+y, want = torch.empty_like(x), torch.empty_like(x)
+cfg, st, g = lib.fft_alloc(n), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+lib.fft_batch(cfg, x, want, b, n, n)
+torch.cuda.synchronize()
+with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
+    lib.fft_batch(cfg, x, y, b, n, n, stream=st)
+for rep in range(3):
+    x.add_(7)
+    lib.fft_batch(cfg, x, want, b, n, n)
+    y.zero_()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(st):
+        g.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(y, want), rep
+print("same")
+"""
+
+
+def test_capture_after_one_eager_call():
+    """In a fresh process one eager call is all the preparation that a captured call of the same
+    kind needs: its temporary comes from the graph's pool, which no call has used before."""
+    r = subprocess.run([sys.executable, "-c", CAPTURED], capture_output=True, text=True, timeout=110, cwd=ROOT,
+                       env=dict(os.environ, PYTHONPATH=ROOT))
+    assert r.returncode == 0 and "same" in r.stdout, r.stderr[-2000:]
