@@ -1468,8 +1468,12 @@ static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPl
         P.bailey_decided = true;
         return 0;
     }
-    if (thread_noalloc())
-        return noalloc_refuse("the four-step plan");
+    if (thread_noalloc()) {
+        if (!P.bailey_open)
+            return noalloc_refuse("the four-step plan");
+        out = P.bailey_builtin;  // as the captured call that left the choice open
+        return 0;
+    }
     const long long n = P.n;
     // the most balanced split, among the built-in lengths and among those that a tile can be
     // compiled for; a built-in one is taken unless its longer half is over 1.5 times the other's
@@ -1517,6 +1521,7 @@ static int bailey_plan(DevPlan &P, hipStream_t s, std::shared_ptr<const BaileyPl
             // keeps it, a graph may hold its tables), and the choice stays open
             if (best1 && !P.bailey_builtin && (rc = build(best1, P.bailey_builtin)))
                 return rc;
+            P.bailey_open = true;
             out = P.bailey_builtin;
             return 0;
         }

@@ -73,7 +73,7 @@ struct DevPlan {
     LinePlan lp1{}, lp2{};
     std::mutex mu;           // guards the choices below (each decided once)
     std::shared_ptr<const FastChoice> fast[3];  // per FK_C2C / FK_R2C / FK_C2R; null: undecided
-    bool bailey_decided = false;
+    bool bailey_decided = false, bailey_open = false;  // (open: a captured call came first)
     std::shared_ptr<const BaileyPlan> bailey;
     std::shared_ptr<const BaileyPlan> bailey_builtin;  // for captured calls while the choice is open
     bool rfused_decided[2] = {false, false};

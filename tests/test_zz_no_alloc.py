@@ -76,3 +76,31 @@ def test_noalloc_refusals():
     lib.fft_batch(cfg, big, bout, 1, n, n)
     with pytest.raises(kissfft_amd.KissFFTError, match="static"):
         lib.fft_batch_noalloc(cfg, big, bout, 1, n, n)
+
+
+@pytest.mark.parametrize("n", [98304, 19683])
+def test_noalloc_after_a_captured_call(n):
+    """A plan whose only call so far was captured has its four-step choice open where the
+    preferred split would be compiled (98304 has a built-in one too, 19683 none): the
+    no-allocation entry point runs it as that call did, and a replay still agrees."""
+    import torch
+    lib = kissfft_amd.load("float")
+    lib.L.kiss_fft_cleanup()
+    x = torch.from_numpy(np.random.default_rng(n).uniform(-1, 1, (2, n, 2)).astype(np.float32)).cuda()
+    y, z = torch.empty_like(x), torch.empty_like(x)
+    cfg, st, g = lib.fft_alloc(n), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    lib.fft_batch(lib.fft_alloc(16384), x, y, 1, 16384, 16384)  # (the pool of captured temporaries)
+    lib.fft_batch(cfg, x, y, 0, n, n)  # (the device plan alone)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=st, capture_error_mode="thread_local"):
+        lib.fft_batch(cfg, x, y, 2, n, n, stream=st)
+    lib.fft_batch_noalloc(cfg, x, z, 2, n, n, stream=st)
+    st.synchronize()
+    assert rel_l2(cplx(z.cpu().numpy()), np.fft.fft(cplx(x.cpu().numpy()), axis=-1)) <= ABS_FLOAT_BOUND
+    for _ in range(3):
+        y.fill_(9.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, z)
