@@ -1962,29 +1962,52 @@ static int fixed_axis(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoic
     return 0;
 }
 
-// The tile kernels of a multi-pass fixed-point plan's two passes, decided once per plan (as
-// fixed_axis, and left open by a no-allocation call too; null: the general kernel).  The second pass reads stage tables of the full
-// length, about 1.3 entries a point, so very long lines keep the general kernel, which
-// reads the one n-point table.
-constexpr int kSplitTableLongest = 1 << 23;
+// Most entries of the second pass's stage tables (8 bytes each; 4 with unpacked Q15): what 2^23
+// points of radices 2 to 5 take, about 1.3 a point.  A generic radix p keeps p (p - 1) per column
+// of its stage, p - 1 a point (7^8 would take 8.0 entries a point, 369 MB), and what is
+// above keeps the general kernel, which reads the one n-point table.
+constexpr long long kSplitTableEntries = 12LL << 20;
+constexpr int kSplitLongest = 1 << 23;
 
+// The radices of a multi-pass plan's two passes.
+static void split_radices(const DevPlan &P, std::vector<int> &r1, std::vector<int> &r2)
+{
+    long long m = 1;
+    for (int p : P.radix) {
+        (m < P.L1 ? r1 : r2).push_back(p);
+        m *= p;
+    }
+}
+
+bool split_tables_fit(const DevPlan &P)
+{
+    std::vector<int> r1, r2;
+    split_radices(P, r1, r2);
+    long long m = P.L1, entries = 0;
+    for (int p : r2) {  // (make_stage_table_raw, rows padded to two entries)
+        entries += m * ((p - 1 + 1) / 2 * 2) + 2;
+        if (p > 5)
+            entries += m * p * (p - 1);
+        m *= p;
+    }
+    return P.n <= kSplitLongest && entries <= kSplitTableEntries;
+}
+
+// The tile kernels of a multi-pass fixed-point plan's two passes, decided once per plan (as
+// fixed_axis, and left open by a no-allocation call too; null: the general kernel).  The
+// second pass reads stage tables of the full length.
 static int fixed_split(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoice> &t1,
                        std::shared_ptr<const TileChoice> &t2)
 {
     std::lock_guard<std::mutex> g(P.mu);
     if (!P.split_decided) {
         t1 = t2 = nullptr;
-        if (P.type != KFA_F32 && !P.single && !P.bigp && P.n <= kSplitTableLongest &&
-            env_flag("KISSFFT_AMD_FAST", true)) {
+        if (P.type != KFA_F32 && !P.single && !P.bigp && split_tables_fit(P) && env_flag("KISSFFT_AMD_FAST", true)) {
             // (the general kernel needs nothing that would have to be allocated)
             if (thread_noalloc() || stream_capturing(s))
                 return 0;
             std::vector<int> r1, r2;
-            long long m = 1;
-            for (int p : P.radix) {
-                (m < P.L1 ? r1 : r2).push_back(p);
-                m *= p;
-            }
+            split_radices(P, r1, r2);
             std::shared_ptr<const TileChoice> a, b;
             if (int rc = fixed_tile(P, r1, 1, 0, a))
                 return rc;

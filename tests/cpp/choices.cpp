@@ -99,6 +99,32 @@ static int bluestein_only_where_exact()
     return 0;
 }
 
+// The tables of a long fixed-point line's second pass are bounded by their size: generic radices
+// keep p - 1 entries a point and stage, the others 1.3 a point in all.
+static int split_tables_are_bounded()
+{
+    auto fits = [](int p, int k1, int k2) {
+        DevPlan P;
+        P.type = KFA_Q31;
+        P.single = false;
+        P.n = P.L1 = P.Q = 1;
+        for (int k = 0; k < k1 + k2; ++k) {
+            P.radix.push_back(p);
+            P.n *= p;
+            (k < k1 ? P.L1 : P.Q) *= p;
+        }
+        return split_tables_fit(P);
+    };
+    CHECK(fits(4, 4, 4));    // 65536 points, 0.7 MB
+    CHECK(fits(4, 5, 6));    // 2^22 points, 45 MB
+    CHECK(fits(5, 4, 5));    // 1953125 points
+    CHECK(fits(7, 3, 4));    // 823543 points, 6.6 M entries
+    CHECK(!fits(7, 4, 4));   // 5764801 points, 46 M entries
+    CHECK(!fits(13, 3, 3));  // 4826809 points, 67 M entries
+    CHECK(!fits(4, 6, 6));   // 2^24 points
+    return 0;
+}
+
 // While the no-allocation entry point runs, choices that would allocate are refused.
 struct NoAlloc {
     NoAlloc() { thread_noalloc() = true; }
@@ -147,6 +173,7 @@ int main(int argc, char **argv)
         {"short_real_rows_do_not_depend_on_the_past", short_real_rows_do_not_depend_on_the_past},
         {"shortest_compiled_row_as_set", shortest_compiled_row_as_set},
         {"bluestein_only_where_exact", bluestein_only_where_exact},
+        {"split_tables_are_bounded", split_tables_are_bounded},
         {"short_complex_lines_are_decided", short_complex_lines_are_decided},
         {"fixed_split_needs_no_allocation", fixed_split_needs_no_allocation},
     };
