@@ -2767,6 +2767,16 @@ int kfa_c2r(const kfa_rplan *pl, const void *in, long long idist, void *out, lon
 // as for rows, and shorter ones when there is more than a handful of them.
 static bool axis_compiles(long long n, long long values) { return n >= kShortRow || values >= kShortValues; }
 
+// The tile kernel of an axis that is not the last (null or v null: the general kernel).
+static int axis_tile(DevPlan &P, long long outer, long long inner, hipStream_t s,
+                     std::shared_ptr<const TileChoice> &tc)
+{
+    tc = nullptr;
+    if (!axis_compiles(P.n, outer * inner * P.n))
+        return 0;
+    return P.type == KFA_F32 ? tile_choice(P.n, P.inverse, TILE_COLS, s, tc, inner, outer) : fixed_axis(P, s, tc);
+}
+
 // One axis of an N-D array batch, dims[k] long, between device buffers (in may equal out).
 static int run_axis(DevPlan &P, const void *in, void *out, long long outer, long long inner,
                     hipStream_t s)
@@ -2785,26 +2795,22 @@ static int run_axis(DevPlan &P, const void *in, void *out, long long outer, long
         }
         return 0;
     }
-    if (axis_compiles(len, outer * inner * len)) {
-        std::shared_ptr<const TileChoice> tc;
-        int rc = P.type == KFA_F32 ? tile_choice((int)len, P.inverse, TILE_COLS, s, tc, inner, outer)
-                                   : fixed_axis(P, s, tc);
-        if (rc)
-            return rc;
-        if (tc && tc->v) {
-            TileArgs a{};
-            a.in = in;
-            a.out = out;
-            a.nlines = outer * inner;
-            a.nlo = inner;
-            a.in_hi = len * inner;
-            a.in_lo = 1;
-            a.in_el = inner;
-            a.out_hi = len * inner;
-            a.out_lo = 1;
-            a.out_el = inner;
-            return launch_tile(*tc, a, s);
-        }
+    std::shared_ptr<const TileChoice> tc;
+    if (int rc = axis_tile(P, outer, inner, s, tc))
+        return rc;
+    if (tc && tc->v) {
+        TileArgs a{};
+        a.in = in;
+        a.out = out;
+        a.nlines = outer * inner;
+        a.nlo = inner;
+        a.in_hi = len * inner;
+        a.in_lo = 1;
+        a.in_el = inner;
+        a.out_hi = len * inner;
+        a.out_lo = 1;
+        a.out_el = inner;
+        return launch_tile(*tc, a, s);
     }
     LineLaunch ll{};
     ll.in = in;
@@ -2827,23 +2833,20 @@ static int run_axis(DevPlan &P, const void *in, void *out, long long outer, long
 
 namespace kfa {
 
-// Complex N-D transform of `howmany` arrays between device buffers: axis 0 first, as
-// kiss_fftnd.c:181-186 does (fixed point rounds per axis, so the order is part of the
-// result); the first axis reads the input, later axes run in place on the output.
-int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, const void *in, void *out,
-           long long howmany, hipStream_t s)
+// The plane pass of a complex N-D transform: the axis done together with the last one
+// (paired; -1: every axis has a pass of its own) and its kernel.
+static int nd_plane(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, long long howmany,
+                    hipStream_t s, int &paired, std::shared_ptr<const PlaneChoice> &pc)
 {
     const int ndims = (int)P.size();
     long long total = 1;
     for (int k = 0; k < ndims; ++k)
         total *= dims[k];
-    long long outer = howmany, inner = total;
-    const void *src = in;
-    int rc = 0;
-    int paired = -1;  // the axis done together with the last one in a plane pass
-    std::shared_ptr<const PlaneChoice> pc;
-    const bool fixed = P[0]->type != KFA_F32;
-    if (ndims >= 2 && !fixed) {
+    int rc;
+    paired = -1;
+    if (ndims < 2)
+        return 0;
+    if (P[0]->type == KFA_F32) {
         // the last axis and one other in one pass when a plane (or slab) of them fits in
         // LDS: the axis before the last first (contiguous planes), then the outer axes from
         // the first (float results do not depend on the order of the axes beyond rounding)
@@ -2865,20 +2868,39 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
                 return rc;
             if (pc->v && (k == ndims - 2 || pc->v->slab)) {
                 paired = k;
-                break;
+                return 0;
             }
         }
     }
-    if (ndims >= 2 && paired < 0) {
-        // no built-in one: a compiled plane of the last two axes
-        const long long values = (long long)dims[ndims - 2] * dims[ndims - 1];
-        if (plane_pays(howmany * (total / values), values)) {
-            if ((rc = compiled_plane(*P[ndims - 2], *P[ndims - 1], s, pc)))
-                return rc;
-            if (pc->v)
-                paired = ndims - 2;
-        }
+    // no built-in one: a compiled plane of the last two axes
+    const long long values = (long long)dims[ndims - 2] * dims[ndims - 1];
+    if (plane_pays(howmany * (total / values), values)) {
+        if ((rc = compiled_plane(*P[ndims - 2], *P[ndims - 1], s, pc)))
+            return rc;
+        if (pc->v)
+            paired = ndims - 2;
     }
+    return 0;
+}
+
+// Complex N-D transform of `howmany` arrays between device buffers: axis 0 first, as
+// kiss_fftnd.c:181-186 does (fixed point rounds per axis, so the order is part of the
+// result); the first axis reads the input, later axes run in place on the output.
+int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, const void *in, void *out,
+           long long howmany, hipStream_t s)
+{
+    const int ndims = (int)P.size();
+    long long total = 1;
+    for (int k = 0; k < ndims; ++k)
+        total *= dims[k];
+    long long outer = howmany, inner = total;
+    const void *src = in;
+    int paired;
+    std::shared_ptr<const PlaneChoice> pc;
+    int rc = nd_plane(P, dims, howmany, s, paired, pc);
+    if (rc)
+        return rc;
+    const bool fixed = P[0]->type != KFA_F32;
     auto plane_pass = [&](const void *from) {
         const int nb = dims[ndims - 1];
         long long rs = 1, mid = 1;  // row stride; planes per value of the axes before `paired`
@@ -2905,6 +2927,67 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
             rc = run_axis(*P[k], src, out, outer, inner, s);
             src = out;
         }
+        outer *= dims[k];
+    }
+    return rc;
+}
+
+// Decides now what `lines` lines of plan P will run on (fk: FK_*; real kinds with P the half-length
+// plan), so that run_c2c / run_real_rows find every choice made.
+int prepare_rows(DevPlan &P, int fk, long long lines, hipStream_t s)
+{
+    if (!P.single)
+        return prepare_multipass(P, fk, s);
+    const FastChoice *fc = nullptr;
+    bool blue = false;
+    int rc = choose_fast(P, fk, s, &fc, lines);
+    if (rc || fc->v)
+        return rc;
+    if (fk == FK_C2C)
+        return blue_prepare(P, &blue);
+    return blue_real_rows(P) ? prepare_rows(P, FK_C2C, lines, s) : 0;
+}
+
+// ... and one axis (run_axis),
+static int prepare_axis(DevPlan &P, long long outer, long long inner, hipStream_t s)
+{
+    if (inner == 1 || !P.single)
+        return prepare_rows(P, FK_C2C, inner == 1 ? outer : inner, s);
+    std::shared_ptr<const TileChoice> tc;
+    return axis_tile(P, outer, inner, s, tc);
+}
+
+// ... an N-D transform (run_nd),
+int prepare_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, long long howmany, hipStream_t s)
+{
+    const int ndims = (int)P.size();
+    int paired;
+    std::shared_ptr<const PlaneChoice> pc;
+    int rc = nd_plane(P, dims, howmany, s, paired, pc);
+    long long outer = howmany, inner = 1;
+    for (int k = 0; k < ndims; ++k)
+        inner *= dims[k];
+    for (int k = 0; k < ndims && rc == 0; ++k) {
+        inner /= dims[k];
+        if (paired < 0 || (k != paired && k != ndims - 1))
+            rc = prepare_axis(*P[k], outer, inner, s);
+        outer *= dims[k];
+    }
+    return rc;
+}
+
+// ... a real N-D transform (run_ndr).
+int prepare_ndr(DevPlan &H, const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, int inverse,
+                long long howmany, hipStream_t s)
+{
+    long long outer = howmany, inner = dims[P.size()] / 2 + 1, rows = 1;
+    for (size_t k = 0; k < P.size(); ++k)
+        rows *= dims[k];
+    inner *= rows;
+    int rc = prepare_rows(H, inverse ? FK_C2R : FK_R2C, rows * howmany, s);
+    for (size_t k = 0; k < P.size() && rc == 0; ++k) {
+        inner /= dims[k];
+        rc = prepare_axis(*P[k], outer, inner, s);
         outer *= dims[k];
     }
     return rc;

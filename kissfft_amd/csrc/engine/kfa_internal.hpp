@@ -197,6 +197,12 @@ int run_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, cons
            long long howmany, hipStream_t s);
 int run_ndr(DevPlan &H, const RealTables &R, const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims,
             int inverse, const void *in, void *out, long long howmany, hipStream_t s);
+// every choice of kernels those calls would make on first use, made now (kernels compiled and
+// timed, tables built) on the caller's thread
+int prepare_rows(DevPlan &P, int fk, long long lines, hipStream_t s);
+int prepare_nd(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, long long howmany, hipStream_t s);
+int prepare_ndr(DevPlan &H, const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, int inverse,
+                long long howmany, hipStream_t s);
 
 // A caller buffer: used in place when the device can access it, else staged through a
 // stream-ordered device copy (stage_in copies host -> device; finish_out device -> host).

@@ -314,6 +314,22 @@ void Server::run()
 
 using namespace kfa;
 
+// The server's device on the submitting thread, whose plans and tables are built there.
+struct OnDevice {
+    int prev = -1;
+    explicit OnDevice(int dev)
+    {
+        int cur = dev;
+        if (hipGetDevice(&cur) == hipSuccess && cur != dev && hipSetDevice(dev) == hipSuccess)
+            prev = cur;
+    }
+    ~OnDevice()
+    {
+        if (prev >= 0)
+            (void)hipSetDevice(prev);
+    }
+};
+
 extern "C" {
 
 void *kfa_server_create(int type, long long budget_bytes, int nstreams, int max_group)
@@ -363,6 +379,7 @@ long long kfa_server_submit(void *srv, int kind, const kfa_cplan *cp, const kfa_
     Server *S = static_cast<Server *>(srv);
     if (!S || !in || !out || howmany <= 0 || nfft <= 0)
         return fail(-2, "server submit: bad arguments");
+    const OnDevice here(S->dev);
     auto r = std::make_shared<ServeReq>();
     r->kind = kind;
     r->n = nfft;
@@ -381,20 +398,17 @@ long long kfa_server_submit(void *srv, int kind, const kfa_cplan *cp, const kfa_
         if ((rc = build_cplan(cp, S->dev, r->P)))
             return rc;
     }
-    // decide the compiled variant now, on the server's plan stream, not in the scheduler
-    if (r->P->single) {
-        const FastChoice *fc;
-        const int row = kind == KFA_SERVE_R2C ? FK_R2C : kind == KFA_SERVE_C2R ? FK_C2R : FK_C2C;
-        if ((rc = choose_fast(*r->P, row, S->plan_stream, &fc, howmany)))
-            return rc;
-    }
+    // compile, time and build what the request will run on now, on the submitting thread: in the
+    // scheduler every other request would wait for it
+    const int fk = kind == KFA_SERVE_R2C ? FK_R2C : kind == KFA_SERVE_C2R ? FK_C2R : FK_C2C;
+    if ((rc = prepare_rows(*r->P, fk, howmany, S->plan_stream)))
+        return rc;
     side_bytes(S->type, kind, nfft, howmany, r->in_bytes, r->out_bytes);
     r->stage_in = !device_accessible(in);
     r->stage_out = !device_accessible(out);
     r->need = (r->stage_in ? r->in_bytes : 0) + (r->stage_out ? r->out_bytes : 0);
     // multi-pass scratch: the temporaries of one chunk of transforms (the chunking of
     // multi-pass batches bounds them)
-    const int fk = kind == KFA_SERVE_R2C ? FK_R2C : kind == KFA_SERVE_C2R ? FK_C2R : FK_C2C;
     if (const size_t temp = multipass_bytes_per_transform(*r->P, fk)) {
         const size_t per = temp + 1024;
         r->need += std::min((size_t)howmany * per, std::max(per, scratch_room()));
@@ -419,6 +433,7 @@ long long kfa_server_submit_nd(void *srv, int kind, int ndims, const int *dims, 
     Server *S = static_cast<Server *>(srv);
     if (!S || !in || !out || howmany <= 0 || ndims <= 0 || !dims || kind < 0 || kind > 3)
         return fail(-2, "server submit: bad arguments");
+    const OnDevice here(S->dev);
     const bool real = kind == KFA_SERVE_R2C || kind == KFA_SERVE_C2R;
     auto r = std::make_shared<ServeReq>();
     r->nd = true;
@@ -452,6 +467,10 @@ long long kfa_server_submit_nd(void *srv, int kind, int ndims, const int *dims, 
     } else {
         r->P = r->axes[0];
     }
+    rc = real ? prepare_ndr(*r->P, r->axes, dims, kind == KFA_SERVE_C2R, howmany, S->plan_stream)
+              : prepare_nd(r->axes, dims, howmany, S->plan_stream);
+    if (rc)
+        return rc;
     const size_t cb = cpx_bytes(S->type), sb = cb / 2;
     const long long last = dims[ndims - 1];
     const size_t cpx_all = cb * (size_t)(total / last * (last / 2 + 1)) * (size_t)howmany;

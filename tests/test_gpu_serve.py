@@ -4,6 +4,7 @@ Each request's result must be identical whether it runs alone (a batched call) o
 a mixed stream served concurrently; host-buffer requests are staged through the server's
 HBM budget and admitted only when they fit; requests larger than the budget fail cleanly.
 """
+import re
 import sys
 
 import numpy as np
@@ -181,4 +182,39 @@ def test_q15_nd_served_bit_exact():
     Y = np.zeros((2, 8, 21, 2), np.int16)
     srv.wait(srv.submit_nd(R2C, (8, 40), xr, Y, 2))
     np.testing.assert_array_equal(Y, O.fftndr(xr, (8, 40)))
+    srv.close()
+
+
+@pytest.mark.parametrize("dtype", ["float", "int16_t"])
+def test_submit_prepares_the_kernels(dtype, monkeypatch, capfd):
+    """Kernels are compiled by the submitting thread, not by the scheduler, where every other
+    request would wait: they are there when submit returns, also for requests that the
+    scheduler never launches (a server of one byte refuses them all)."""
+    lib = kissfft_amd.load(dtype)
+    monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    lib.L.kiss_fft_cleanup()
+    srv = lib.server(1, 1, 8)
+
+    def report(submit, *shapes):
+        x, y = (np.zeros(s, lib.scalar) for s in shapes)
+        capfd.readouterr()
+        ticket = submit(x, y)
+        err = capfd.readouterr().err
+        with pytest.raises(kissfft_amd.KissFFTError, match="budget"):
+            srv.wait(ticket)
+        return err
+
+    n = 54000  # two passes, 225 x 240
+    err = report(lambda x, y: srv.submit(C2C_FWD, n, x, y, 2), (2, n, 2), (2, n, 2))
+    say(err)
+    assert len(set(re.findall(r"tile n=(\d+)", err))) == 2, err
+    dims = (45, 36, 84, 60)  # two axes and a compiled plane too large for few arrays: four axes
+    err = report(lambda x, y: srv.submit_nd(C2C_FWD, dims, x, y, 1), dims + (2,), dims + (2,))
+    say(err)
+    assert f"plane {dims[2]}x{dims[3]}" in err or f"tile n={dims[2]}" in err, err
+    assert f"tile n={dims[0]}" in err and f"tile n={dims[1]}" in err, err
+    dims = (50, 66, 90)  # real rows of 45 bins, axes of 50 and 66
+    err = report(lambda x, y: srv.submit_nd(R2C, dims, x, y, 3), (3,) + dims, (3, 50, 66, 46, 2))
+    say(err)
+    assert "rtc_r2c45" in err and "tile n=50" in err and "tile n=66" in err, err
     srv.close()
