@@ -746,8 +746,11 @@ struct PlaneChoice {
 
 typedef std::pair<DevBuf, DevBuf> BufPair;
 
+// A choice that is missing is made (kernels compiled and timed, tables built) under `build`
+// alone: lookups, which take `mu` for a moment, go on meanwhile.
 struct TileCache {
-    std::mutex mu;
+    std::mutex build;
+    std::mutex mu;  // guards the maps; taken after `build`
     // dev, n, inv, mode, inner, small (see tile_choice)
     std::map<std::tuple<int, int, int, int, long long, int>, std::shared_ptr<const TileChoice>> choice;
     std::map<std::tuple<int, long long, int, int>, BufPair> fs;                           // dev, N, inv, wide -> hi, lo
@@ -762,6 +765,25 @@ static TileCache &tile_cache()
 {
     static TileCache *c = new TileCache();
     return *c;
+}
+
+// The choice under `key`, if it is made.
+template <class Map, class Value>
+static bool find_choice(TileCache &C, const Map &map, const typename Map::key_type &key, Value &out)
+{
+    std::lock_guard<std::mutex> g(C.mu);
+    auto it = map.find(key);
+    if (it == map.end())
+        return false;
+    out = it->second;
+    return true;
+}
+
+template <class Map, class Value>
+static void keep_choice(TileCache &C, Map &map, const typename Map::key_type &key, const Value &v)
+{
+    std::lock_guard<std::mutex> g(C.mu);
+    map[key] = v;
 }
 
 // The tile variant for (n, inverse, mode) on the current device, or v == nullptr.
@@ -944,15 +966,14 @@ static int tile_choice(int n, int inverse, int mode, hipStream_t s, std::shared_
     if (rc)
         return rc;
     auto &C = tile_cache();
-    std::lock_guard<std::mutex> g(C.mu);
     const bool geo = mode == TILE_COLS && inner > 0 && outer > 0;
     const int small = geo && 8.0 * n * (double)inner * (double)outer <= (double)(128 << 20);
     const auto key = std::make_tuple(dev, n, inverse, mode, geo ? inner : 0LL, small);
-    auto it = C.choice.find(key);
-    if (it != C.choice.end()) {
-        out = it->second;
+    if (find_choice(C, C.choice, key, out))
         return 0;
-    }
+    std::lock_guard<std::mutex> g(C.build);
+    if (find_choice(C, C.choice, key, out))
+        return 0;
     if (thread_noalloc())
         return noalloc_refuse("a tile kernel's tables");
     std::vector<std::shared_ptr<TileChoice>> cand;
@@ -993,7 +1014,7 @@ static int tile_choice(int n, int inverse, int mode, hipStream_t s, std::shared_
     std::shared_ptr<const TileChoice> tc = cand.empty() ? std::make_shared<const TileChoice>() : cand[best];
     if (tc->v && env_flag("KISSFFT_AMD_VERBOSE", false))
         fprintf(stderr, "[kissfft_amd] tile n=%d inverse=%d mode=%d: %s\n", n, inverse, mode, tc->v->name);
-    C.choice[key] = tc;
+    keep_choice(C, C.choice, key, tc);
     out = tc;
     return 0;
 }
@@ -1328,14 +1349,13 @@ static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long 
     if (rc)
         return rc;
     auto &C = tile_cache();
-    std::lock_guard<std::mutex> g(C.mu);
     const bool small = 8.0 * A * B * (double)planes <= (double)(128 << 20);
     const auto key = std::make_tuple(dev, A, B, inverse, (int)slab, (int)small);
-    auto it = C.plane.find(key);
-    if (it != C.plane.end()) {
-        out = it->second;
+    if (find_choice(C, C.plane, key, out))
         return 0;
-    }
+    std::lock_guard<std::mutex> g(C.build);
+    if (find_choice(C, C.plane, key, out))
+        return 0;
     if (thread_noalloc())
         return noalloc_refuse("a plane kernel's tables");
     std::vector<std::shared_ptr<PlaneChoice>> cand;
@@ -1388,7 +1408,7 @@ static int plane_choice(int A, int B, int inverse, bool slab, int rs, long long 
     std::shared_ptr<const PlaneChoice> pc = cand.empty() ? std::make_shared<const PlaneChoice>() : cand[best];
     if (pc->v && env_flag("KISSFFT_AMD_VERBOSE", false))
         fprintf(stderr, "[kissfft_amd] plane %dx%d inverse=%d: %s\n", A, B, inverse, pc->v->name);
-    C.plane[key] = pc;
+    keep_choice(C, C.plane, key, pc);
     out = pc;
     return 0;
 }
@@ -1420,13 +1440,12 @@ static int compiled_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, s
     if (rc)
         return rc;
     auto &C = tile_cache();
-    std::lock_guard<std::mutex> g(C.mu);
     const auto key = std::make_tuple(dev, PA.type, PA.n, PB.n, PA.inverse);
-    auto it = C.made_plane.find(key);
-    if (it != C.made_plane.end()) {
-        out = it->second;
+    if (find_choice(C, C.made_plane, key, out))
         return 0;
-    }
+    std::lock_guard<std::mutex> g(C.build);
+    if (find_choice(C, C.made_plane, key, out))
+        return 0;
     if (thread_noalloc())
         return noalloc_refuse("a plane kernel's tables");
     auto pc = std::make_shared<PlaneChoice>();
@@ -1448,7 +1467,7 @@ static int compiled_plane(const DevPlan &PA, const DevPlan &PB, hipStream_t s, s
             fprintf(stderr, "[kissfft_amd] plane %dx%d inverse=%d type=%d: %s\n", PA.n, PB.n, PA.inverse, PA.type,
                     pc->v->name);
     }
-    C.made_plane[key] = pc;
+    keep_choice(C, C.made_plane, key, std::shared_ptr<const PlaneChoice>(pc));
     return 0;
 }
 

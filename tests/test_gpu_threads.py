@@ -9,6 +9,7 @@ in a server, or while other threads transform, must not disturb them.
 """
 import sys
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -208,3 +209,45 @@ def test_cleanup_while_other_threads_transform():
     for t in th:
         t.join()
     assert not errors, errors[:5]
+
+
+def test_decided_nd_calls_go_on_while_another_compiles(monkeypatch, tmp_path):
+    """A thread whose N-D call compiles a kernel (some tenths of a second, nothing on disk) does
+    not hold up another thread's calls of shapes that are decided."""
+    monkeypatch.setenv("KISSFFT_AMD_CACHE", str(tmp_path))
+    lib = kissfft_amd.load("float")
+    rng = np.random.default_rng(9)
+    dims, new = (50, 64, 6), (5, 243, 19)
+    x = rng.uniform(-1, 1, (2,) + dims + (2,)).astype(np.float32)
+    xn = rng.uniform(-1, 1, (2,) + new + (2,)).astype(np.float32)
+    cfg, cfg_new = lib.fftnd_alloc(dims), lib.fftnd_alloc(new, True)
+    want = np.zeros_like(x)
+    lib.fftnd_batch(cfg, x, want, 2)
+    ends, bad, stop, started = [], [], threading.Event(), threading.Event()
+
+    def other():
+        y = np.zeros_like(x)
+        while not stop.is_set():
+            lib.fftnd_batch(cfg, x, y, 2)
+            ends.append(time.perf_counter())
+            if not np.array_equal(y, want):
+                bad.append(len(ends))
+            started.set()
+
+    t = threading.Thread(target=other)
+    t.start()
+    try:
+        assert started.wait(30)
+        t0 = time.perf_counter()
+        lib.fftnd_batch(cfg_new, xn, np.zeros_like(xn), 2)
+        t1 = time.perf_counter()
+    finally:
+        stop.set()
+        t.join()
+    during = [t0] + [e for e in ends if t0 < e < t1] + [t1]
+    gap = max(b - a for a, b in zip(during, during[1:]))
+    say("compiling call", round(t1 - t0, 3), "s; the other thread's longest call in it", round(gap, 3), "s of",
+        len(during) - 2)
+    assert not bad
+    assert t1 - t0 > 0.1, "nothing was compiled"
+    assert gap < 0.4 * (t1 - t0)
