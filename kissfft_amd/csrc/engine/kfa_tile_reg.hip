@@ -313,11 +313,17 @@ const std::vector<BlueVariant> &blue_registry()
         add_blue<16, 4, 0, 16, 16>(*v, "blue256_1616_t16x4");
         add_blue<64, 2, 1, 8, 8, 8>(*v, "blue512_888_t64x2");
         add_blue<128, 2, 0, 8, 8, 4, 4>(*v, "blue1024_8844_t128x2");
+        // The last argument true: only in a multi-batch, whose fused launch runs members of one
+        // workgroup size, shares their registers and LDS among them, and is 256 threads wide with
+        // most row kernels; 16 values a thread there, 8 in a launch of their own.
         // c2c 1009 x4096 27.4 us, 32.2 with 128 threads a line, 30.9 with 16, 16, 8 at 128; but
         // 64 uneven batches in one fused launch 45.1, 45.1 and 43.4 us
         add_blue<256, 1, 0, 8, 8, 8, 4>(*v, "blue2048_8884_t256");
         add_blue<128, 2, 1, 16, 16, 8>(*v, "blue2048_16168_t128x2", true);
         add_blue<512, 1, 0, 8, 8, 8, 8>(*v, "blue4096_8888_t512");
+        // lengths 1009 and 1997 among six lists in one multi-batch: both fused 20.9 us, 28.5 with 512
+        // threads for 1997, which leaves 1009 a launch of its own; without 1009 18.7 against 18.0
+        add_blue<256, 1, 0, 8, 8, 8, 8>(*v, "blue4096_8888_t256", true);
         // lengths above 2048: 4093 x8 10.7 ms -> 16 us, 5002 x8 319 -> 23 us against the general kernel
         add_blue<512, 1, 3, 8, 8, 8, 4, 4>(*v, "blue8192_88844_t512");
         add_blue<1024, 1, 3, 8, 8, 8, 8, 4>(*v, "blue16384_88884_t1024");

@@ -346,3 +346,28 @@ def test_graph_capture_with_multipass_items():
                 got = got if k == C2R else cplx(got)
                 assert rel_l2(got, fp64_ref(k, n, xs)) <= ABS_FLOAT_BOUND, (k, n)
         m.close()
+
+
+def test_bluestein_groups_of_two_sizes_share_the_fused_launch():
+    """Prime lengths whose convolutions have 2048 and 4096 points run in one fused launch, with
+    a compiled-row group: every group is in it and every result is a transform."""
+    import torch
+    lib = kissfft_amd.load("float")
+    rng = np.random.default_rng(77)
+    items, keep = [], []
+    for kind, n, b in ((0, 1009, 7), (1, 1021, 5), (0, 1997, 6), (1, 2039, 4), (0, 1024, 20)):
+        x = torch.from_numpy(rng.uniform(-1, 1, (b, n, 2)).astype(np.float32)).cuda()
+        y = torch.empty_like(x)
+        items.append((kind, n, x, y, b))
+        keep.append((kind, n, x, y))
+    torch.cuda.synchronize()
+    m = kissfft_amd.MultiBatch(lib, items)
+    info = m.info()
+    assert info["bluestein_items"] == 4 and info["fused_groups"] == 5, info
+    m.exec()
+    torch.cuda.synchronize()
+    for kind, n, x, y in keep:
+        z = cplx(x.cpu().numpy())
+        want = np.fft.ifft(z, axis=-1) * n if kind else np.fft.fft(z, axis=-1)
+        assert rel_l2(cplx(y.cpu().numpy()), want) <= ABS_FLOAT_BOUND, n
+    m.close()
