@@ -1,8 +1,8 @@
 // kfa_conv.hip -- fast FIR filtering by overlap-scrap (k_conv in kfa_blue.hpp).
 //
 // The filter spectrum (N complex FP64, scaled by 1/N) comes from the host layer; the engine
-// keeps a device copy per (device, N, spectrum contents) together with the stage tables
-// of the N-point schedule, and runs every complete block of a call in one launch.
+// keeps a device copy per (device, N, impulse response), and the stage tables of an N-point
+// schedule once for all of them, and runs every complete block of a call in one launch.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -19,20 +19,48 @@
 
 namespace kfa {
 
+typedef std::pair<DevBuf, DevBuf> BufPair;
+
 struct ConvPlan {
     const ConvVariant *v = nullptr;
-    DevBuf mem_f, mem_i, mem_h;
+    BufPair stages;  // forward, inverse
+    DevBuf mem_h;
+};
+
+// Device plans by the response itself (its samples' bytes): at most 1/2 of the spectrum's, and of a
+// real one 1/4, to compare per call, and nothing is copied for the look-up (2^16 samples through
+// 1000 taps 23.2 -> 21.2 us, 4000 taps 31.5 -> 27.5).
+struct ConvKey {
+    int dev, nfft, real;
+    std::string taps;
+};
+struct ConvRef {
+    int dev, nfft, real;
+    const char *taps;
+    size_t bytes;
+};
+struct ConvLess {
+    typedef void is_transparent;
+    static ConvRef ref(const ConvKey &k) { return {k.dev, k.nfft, k.real, k.taps.data(), k.taps.size()}; }
+    static const ConvRef &ref(const ConvRef &k) { return k; }
+    template <class X, class Y>
+    bool operator()(const X &x, const Y &y) const
+    {
+        const ConvRef &a = ref(x), &b = ref(y);
+        const auto ka = std::make_tuple(a.dev, a.nfft, a.real, a.bytes), kb = std::make_tuple(b.dev, b.nfft, b.real, b.bytes);
+        return ka != kb ? ka < kb : memcmp(a.taps, b.taps, a.bytes) < 0;
+    }
 };
 
 static std::mutex g_conv_mu;
-static std::map<std::tuple<int, int, int, std::string>, std::shared_ptr<const ConvPlan>> g_conv;
+static std::map<ConvKey, std::shared_ptr<const ConvPlan>, ConvLess> g_conv;
+static std::map<std::pair<int, const ConvVariant *>, BufPair> g_conv_stages;  // per device
 
-static int conv_plan(int dev, int nfft, int real, const void *H, std::shared_ptr<const ConvPlan> &out)
+static int conv_plan(int dev, int nfft, int real, const void *H, const void *h, size_t bytes,
+                     std::shared_ptr<const ConvPlan> &out)
 {
-    const std::string key_h((const char *)H, (size_t)nfft * 16);
     std::lock_guard<std::mutex> g(g_conv_mu);
-    const auto key = std::make_tuple(dev, nfft, real, key_h);
-    auto it = g_conv.find(key);
+    auto it = g_conv.find(ConvRef{dev, nfft, real, (const char *)h, bytes});
     if (it != g_conv.end()) {
         out = it->second;
         return 0;
@@ -45,14 +73,20 @@ static int conv_plan(int dev, int nfft, int real, const void *H, std::shared_ptr
         }
     if (!cp->v)
         return fail(-2, "fast convolution: no kernel for block length %d (powers of two 256..8192)", nfft);
-    const std::vector<unsigned char> tf = float_twiddles(nfft, 0, nfft, 1), ti = float_twiddles(nfft, 1, nfft, 1);
     int rc;
-    if ((rc = make_stage_table_raw(tf.data(), KFA_F32, nfft, cp->v->radices, cp->v->tw_pad, 0, cp->mem_f)) ||
-        (rc = make_stage_table_raw(ti.data(), KFA_F32, nfft, {cp->v->radices.rbegin(), cp->v->radices.rend()},
-                                   cp->v->tw_pad, 0, cp->mem_i)) ||
-        (rc = dev_upload(H, (size_t)nfft * 16, cp->mem_h)))
+    BufPair &st = g_conv_stages[{dev, cp->v}];
+    if (!st.first || !st.second) {
+        const std::vector<unsigned char> tf = float_twiddles(nfft, 0, nfft, 1), ti = float_twiddles(nfft, 1, nfft, 1);
+        const std::vector<int> &rad = cp->v->radices;
+        if ((rc = make_stage_table_raw(tf.data(), KFA_F32, nfft, rad, cp->v->tw_pad, 0, st.first)) ||
+            (rc = make_stage_table_raw(ti.data(), KFA_F32, nfft, {rad.rbegin(), rad.rend()}, cp->v->tw_pad, 0,
+                                       st.second)))
+            return rc;
+    }
+    cp->stages = st;
+    if ((rc = dev_upload(H, (size_t)nfft * 16, cp->mem_h)))
         return rc;
-    g_conv[key] = cp;
+    g_conv.emplace(ConvKey{dev, nfft, real, std::string((const char *)h, bytes)}, cp);
     out = cp;
     return 0;
 }
@@ -83,14 +117,15 @@ void conv_release()
 {
     std::lock_guard<std::mutex> g(g_conv_mu);
     g_conv.clear();
+    g_conv_stages.clear();
 }
 
 }  // namespace kfa
 
 using namespace kfa;
 
-extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, long long nh, void *in, void *out,
-                           long long nout, long long keep, int *moved, void *stream, int sync)
+extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, const void *h, long long nh, void *in,
+                           void *out, long long nout, long long keep, int *moved, void *stream, int sync)
 {
     *moved = 0;
     if (type != KFA_F32)
@@ -103,7 +138,7 @@ extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, long lon
     if (rc || nout == 0)
         return rc;
     std::shared_ptr<const ConvPlan> cp;
-    if ((rc = conv_plan(dev, nfft, real, H, cp)))
+    if ((rc = conv_plan(dev, nfft, real, H, h, (size_t)nh * (real ? 4 : 8), cp)))
         return rc;
     const size_t sb = real ? 4 : 8;
     Operand I, O;
@@ -114,8 +149,8 @@ extern "C" int kfa_fastfir(int type, int nfft, int real, const void *H, long lon
         ConvArgs a{};
         a.in = I.dev;
         a.out = O.dev;
-        a.stw_f = cp->mem_f.get();
-        a.stw_i = cp->mem_i.get();
+        a.stw_f = cp->stages.first.get();
+        a.stw_i = cp->stages.second.get();
         a.H = cp->mem_h.get();
         a.ngood = nfft - nh + 1;
         a.nin = nout + nh - 1;

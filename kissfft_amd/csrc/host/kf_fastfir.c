@@ -23,6 +23,7 @@ struct kiss_fastfir_state {
     size_t nblk;      /* points of the GPU's transforms (ff_block) */
     int real;
     double *H;        /* nblk FP64 pairs, spectrum / nblk */
+    void *taps;       /* the nh samples of the impulse response */
     void *tmpbuf;     /* nfft samples, the flush block */
 };
 
@@ -123,7 +124,7 @@ static kiss_fastfir_cfg ff_alloc(const void *h, size_t nh, int real, size_t *pnf
     }
     nblk = ff_block(nh);
     const size_t samp = real ? sizeof(kiss_fft_scalar) : sizeof(kiss_fft_cpx);
-    const size_t need = sizeof(struct kiss_fastfir_state) + 2 * sizeof(double) * nblk + samp * nfft;
+    const size_t need = sizeof(struct kiss_fastfir_state) + 2 * sizeof(double) * nblk + samp * (nh + nfft);
     kiss_fastfir_cfg st = NULL;
     if (lenmem == NULL) {
         st = (kiss_fastfir_cfg)malloc(need);
@@ -140,7 +141,9 @@ static kiss_fastfir_cfg ff_alloc(const void *h, size_t nh, int real, size_t *pnf
     st->nblk = nblk;
     st->real = real;
     st->H = (double *)(st + 1);
-    st->tmpbuf = (void *)(st->H + 2 * nblk);
+    st->taps = (void *)(st->H + 2 * nblk);
+    st->tmpbuf = (void *)((char *)st->taps + samp * nh);
+    memcpy(st->taps, h, samp * nh);
 
     double *re = (double *)calloc(nblk, sizeof(double)), *im = (double *)calloc(nblk, sizeof(double));
     double *w = (double *)malloc(nblk * sizeof(double));
@@ -182,8 +185,8 @@ static size_t ff_blocks(kiss_fastfir_cfg st, void *in, void *out, size_t n, int 
     if (n < st->nfft)
         return 0;
     const size_t nout = ((n - st->nfft) / st->ngood + 1) * st->ngood;
-    if (kfa_fastfir(KF_TYPE, (int)st->nblk, st->real, st->H, (long long)st->nh, in, out, (long long)nout,
-                    rest ? (long long)(n - nout) : 0, moved, NULL, 1) != 0) {
+    if (kfa_fastfir(KF_TYPE, (int)st->nblk, st->real, st->H, st->taps, (long long)st->nh, in, out,
+                    (long long)nout, rest ? (long long)(n - nout) : 0, moved, NULL, 1) != 0) {
         KF_ERROR("kiss_fastfir: %s", kfa_last_error());
         return 0;
     }

@@ -132,11 +132,11 @@ KFA_HIDDEN void kfa_multi_destroy(void *m);
 
 /* Fast FIR by overlap-scrap: out[t] = sum_i h[i] in[t + nh-1 - i], t < nout, from nout + nh-1
  * samples at in, by transforms of nfft points.  H: nfft FP64 pairs (host), the spectrum of the
- * rotated impulse response scaled by 1/nfft.  real: samples are scalars.  Where `in` is device
+ * rotated impulse response h scaled by 1/nfft.  real: samples and h are scalars.  Where `in` is device
  * memory the `keep` samples from in[nout] on are moved to its front as well, behind the
  * convolution, and *moved is set. */
-KFA_HIDDEN int kfa_fastfir(int type, int nfft, int real, const void *H, long long nh, void *in, void *out,
-                           long long nout, long long keep, int *moved, void *stream, int sync);
+KFA_HIDDEN int kfa_fastfir(int type, int nfft, int real, const void *H, const void *h, long long nh, void *in,
+                           void *out, long long nout, long long keep, int *moved, void *stream, int sync);
 
 #ifdef __cplusplus
 }

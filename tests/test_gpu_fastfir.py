@@ -164,3 +164,28 @@ def test_device_stream_tail(nh, nfft, extra, real):
     c = (lambda v: v.astype(np.float64)) if real else (lambda v: v[:, 0] + 1j * v[:, 1].astype(np.float64))
     want = np.convolve(c(x), c(h), mode="valid")[:used]
     assert rel_l2(c(y), want) <= 1e-6
+
+
+@pytest.mark.parametrize("nh", [9, 300])
+def test_filters_of_one_length_and_one_place(nh):
+    """Filters of the same length differ by their responses alone, also when one is planned in
+    the memory of another: each call runs the response its cfg was planned from."""
+    import ctypes
+    lib = kissfft_amd.load("float")
+    rng = np.random.default_rng(nh)
+    taps = [rng.standard_normal(nh).astype(np.float32) for _ in range(2)]
+    taps.append(taps[0].copy())
+    taps[2][nh - 1] += 1.0  # the same but for the last tap
+    need, nfft = ctypes.c_size_t(0), ctypes.c_size_t(0)
+    lib.L.kiss_fastfir_alloc_real(taps[0].ctypes.data, nh, ctypes.byref(nfft), None, ctypes.byref(need))
+    mem = ctypes.create_string_buffer(need.value + 64)
+    at = (ctypes.addressof(mem) + 63) & ~63
+    n = 6000
+    x = rng.standard_normal(n).astype(np.float32)
+    for k in (0, 1, 2, 0, 2, 1):
+        size, nfft = ctypes.c_size_t(need.value), ctypes.c_size_t(0)
+        assert lib.L.kiss_fastfir_alloc_real(taps[k].ctypes.data, nh, ctypes.byref(nfft), at, ctypes.byref(size)) == at
+        buf, y, off = x.copy(), np.zeros(n, np.float32), ctypes.c_size_t(0)
+        w = lib.L.kiss_fastfir_real(at, buf.ctypes.data, y.ctypes.data, n, ctypes.byref(off))
+        want = np.convolve(x.astype(np.float64), taps[k].astype(np.float64), mode="valid")[:w]
+        assert w > 0 and rel_l2(y[:w], want) <= 1e-6, k
