@@ -1423,9 +1423,13 @@ constexpr long long kTileLongest = 2048;
 // leave a CU room for fewer than four wait on their own barriers (against two passes, us:
 // float 80x60 x64 9.7 / 9.5, x128 9.6 / 11.8, x256 10.6 / 16.5, x1300 38 / 38; 100x45 x1000
 // 25 / 34; 30x40 x1 6.2 / 9.7; Q15 80x60 x1300 27 / 35; but 20x300 x600 33 / 29, Q15 64x96x120
-// x16 83 / 77).
-static bool plane_pays(long long planes, long long values)
+// x16 83 / 77).  A plane of a few values leaves most of its workgroup's 128 threads idle, which
+// many of them pay for (float x2^20: 2x2 302 us against 79 in two axis passes, 4x4 323 / 228,
+// 4x8 506 / 583; x16384: 2x2 5.7 / 7.7).  One launch takes 2^31 - 1 workgroups.
+bool plane_pays(long long planes, long long values)
 {
+    if (planes > 0x7fffffffLL || (values < 32 && planes > 16384))
+        return false;
     return values <= 2048 || (planes >= 128 && values <= 5000);
 }
 

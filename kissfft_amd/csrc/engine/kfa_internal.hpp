@@ -153,6 +153,8 @@ size_t multipass_bytes_per_transform(DevPlan &P, int fk);
 // decides every lazily built choice a multi-pass transform of P will use (tile variants,
 // four-step tables), so that later calls allocate nothing but their scratch
 int prepare_multipass(DevPlan &P, int fk, hipStream_t s);
+// whether `planes` planes of `values` values run as planes compiled at run time
+bool plane_pays(long long planes, long long values);
 // whether the stage tables of a long fixed-point plan's second pass are of a size to keep
 bool split_tables_fit(const DevPlan &P);
 bool device_accessible(const void *p);

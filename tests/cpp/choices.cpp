@@ -125,6 +125,16 @@ static int split_tables_are_bounded()
     return 0;
 }
 
+// Many planes of a few values, and more planes than one launch takes, keep an axis per pass.
+static int compiled_planes_where_they_pay()
+{
+    CHECK(!plane_pays(1 << 20, 2 * 2) && !plane_pays(1 << 20, 5 * 5));
+    CHECK(plane_pays(16384, 2 * 2) && plane_pays(1 << 20, 4 * 8));
+    CHECK(!plane_pays(1LL << 31, 16 * 16) && plane_pays((1LL << 31) - 1, 16 * 16));
+    CHECK(plane_pays(1, 2048) && !plane_pays(1, 2049) && plane_pays(128, 5000) && !plane_pays(128, 5001));
+    return 0;
+}
+
 // While the no-allocation entry point runs, choices that would allocate are refused.
 struct NoAlloc {
     NoAlloc() { thread_noalloc() = true; }
@@ -174,6 +184,7 @@ int main(int argc, char **argv)
         {"shortest_compiled_row_as_set", shortest_compiled_row_as_set},
         {"bluestein_only_where_exact", bluestein_only_where_exact},
         {"split_tables_are_bounded", split_tables_are_bounded},
+        {"compiled_planes_where_they_pay", compiled_planes_where_they_pay},
         {"short_complex_lines_are_decided", short_complex_lines_are_decided},
         {"fixed_split_needs_no_allocation", fixed_split_needs_no_allocation},
     };

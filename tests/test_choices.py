@@ -34,6 +34,7 @@ def check(driver, case):
 
 @pytest.mark.parametrize("case", ["open_choice_is_not_the_plans", "short_real_rows_do_not_depend_on_the_past",
                                   "shortest_compiled_row_as_set", "short_complex_lines_are_decided", "fixed_split_needs_no_allocation",
-                                  "bluestein_only_where_exact", "split_tables_are_bounded"])
+                                  "bluestein_only_where_exact", "split_tables_are_bounded",
+                                  "compiled_planes_where_they_pay"])
 def test_choice(driver, case):
     check(driver, case)
