@@ -11,13 +11,16 @@
  *   kiss_fastfir_alloc(h, nh, &nfft, mem, lenmem)
  *       nfft <= 0 (or NULL): the next power of two at least twice nh-1, at least 1024
  *       (complex) or 2048 (real) -- kiss_fastfir.c:77-89.  Supported block lengths are
- *       powers of two from 256 to 8192 (one block is transformed in LDS).  mem/lenmem:
- *       the reference's size-query protocol; the cfg is one free()-able block.
+ *       powers of two from 256 to 8192.  mem/lenmem: the reference's size-query protocol;
+ *       the cfg is one free()-able block (it holds the response and its spectrum).
  *   kiss_fastfir(cfg, inbuf, outbuf, n_new, &offset)
  *       filters the offset + n_new samples at the front of inbuf: every complete block
  *       (nfft samples in, nfft-nh+1 good samples out) in one GPU launch; returns the
  *       number of output samples written and moves the unprocessed input samples to the
- *       front of inbuf, setting offset to their count.  n_new == 0 flushes: the remaining
+ *       front of inbuf, setting offset to their count.  nfft sets how many samples a call
+ *       completes; the GPU's transforms have a length of their own, chosen from nh (256 to
+ *       8192 points, one in LDS per workgroup or less), so an infinity or NaN among the
+ *       samples spreads over the outputs of that transform (two of them for real samples).  n_new == 0 flushes: the remaining
  *       samples are zero-padded and filtered.  Buffers may be host or device memory.
  *
  * Differences: float builds only (the reference scales the spectrum by 1/nfft in float,

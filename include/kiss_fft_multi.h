@@ -10,11 +10,13 @@
  * is assigned, once, to a launch:
  *   - items whose (kind, length) has a compiled row kernel are grouped by (kind, length)
  *     into one launch of that kernel (up to 64 items per launch, one segment each);
- *   - float lengths with a prime factor above 16 (e.g. 1009) run Bluestein's kernel,
- *     grouped by length the same way;
- *   - every other item of at most one LDS line (generic prime radices, fixed-point lengths
- *     without a compiled kernel) joins a single persistent launch that walks a table of
- *     all of them, any mix of lengths and kinds together;
+ *   - complex float lengths that the batched calls run on Bluestein's kernel (a prime factor
+ *     above 16 up to 2048 points, e.g. 1009; most with one above 50 up to 8192) run it here,
+ *     grouped by length the same way, with the workgroup size of the fused launch;
+ *   - every other item of at most one LDS line (other lengths with large primes, real rows of
+ *     such half lengths included, and lengths without a compiled kernel) joins a single
+ *     persistent launch that walks a table of all of them, any mix of lengths and kinds
+ *     together;
  *   - items longer than one LDS line (float 8192 complex / 16384 real, Q15 16384 / 32768)
  *     run as their own multi-pass launches, their temporaries in a workspace the
  *     multi-batch allocates at creation;

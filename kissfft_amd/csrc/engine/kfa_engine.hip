@@ -1958,10 +1958,16 @@ static int fixed_tile(const DevPlan &P, const std::vector<int> &rad, long long m
     if (int rc = make_stage_table_raw(P.h_tw.data(), P.type, P.n, rad, v->tw_pad, v->tw_fmt, tc->stw_mem, m0))
         return rc;
     tc->d_stw = tc->stw_mem.get();
-    if (env_flag("KISSFFT_AMD_VERBOSE", false))
-        fprintf(stderr, "[kissfft_amd] tile n=%d of %d inverse=%d type=%d: %s\n", v->n, P.n, P.inverse, P.type, v->name);
     out = tc;
     return 0;
+}
+
+// The engine's report of tile tc for (part of) fixed-point plan P.
+static void report_tile(const DevPlan &P, const std::shared_ptr<const TileChoice> &tc)
+{
+    if (tc && env_flag("KISSFFT_AMD_VERBOSE", false))
+        fprintf(stderr, "[kissfft_amd] tile n=%d of %d inverse=%d type=%d: %s\n", tc->v->n, P.n, P.inverse, P.type,
+                tc->v->name);
 }
 
 // The tile kernel for the lines of fixed-point plan P as strided columns, decided once per
@@ -1980,6 +1986,7 @@ static int fixed_axis(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoic
     if (env_flag("KISSFFT_AMD_FAST", true))
         if (int rc = fixed_tile(P, P.radix, 1, 0, P.axis))
             return rc;
+    report_tile(P, P.axis);
     P.axis_decided = true;
     out = P.axis;
     return 0;
@@ -2040,6 +2047,8 @@ static int fixed_split(DevPlan &P, hipStream_t s, std::shared_ptr<const TileChoi
             if (a && b) {
                 P.split1 = a;
                 P.split2 = b;
+                report_tile(P, a);
+                report_tile(P, b);
             }
         }
         P.split_decided = true;

@@ -14,7 +14,7 @@
 // A thread's line is the lane's for every stage but a ROWS first stage, so a butterfly's
 // operands sit TL values apart in LDS and a wave touches TL neighbouring values per
 // element: the LDS rows are as free of bank conflicts as the HBM rows are contiguous
-// (tile_pos).
+// (TilePos).
 //
 // TWID multiplies element e of line l by W^(lo*e), W = exp(-+2*pi*i/tw_n), on the way out:
 // the twiddle step between the two passes of the four-step split (Bailey, "FFTs in

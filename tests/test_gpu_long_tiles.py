@@ -148,3 +148,23 @@ def test_capture_after_one_eager_call():
     r = subprocess.run([sys.executable, "-c", CAPTURED], capture_output=True, text=True, timeout=110, cwd=ROOT,
                        env=dict(os.environ, PYTHONPATH=ROOT))
     assert r.returncode == 0 and "same" in r.stdout, r.stderr[-2000:]
+
+
+@pytest.mark.parametrize("dtype", ["float", "int16_t", "int32_t"])
+@pytest.mark.parametrize("n", [18750, 19683, 65536, 98304, 2 ** 18 * 3])
+def test_both_passes_run_on_tiles(n, dtype, monkeypatch, capfd):
+    """The engine reports a pair of tiles only when both are there, and then runs both: two
+    lines of its report per fixed-point plan, one naming both tiles per float plan."""
+    lib = kissfft_amd.load(dtype)
+    monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    lib.L.kiss_fft_cleanup()
+    x = rnd(np.random.default_rng(n), dtype, (1, n, 2))
+    for inv in (False, True):
+        capfd.readouterr()
+        lib.fft_batch(lib.fft_alloc(n, inv), x, np.zeros_like(x), 1, n, n)
+        err = capfd.readouterr().err
+        if dtype == "float":
+            assert len(re.findall(rf"four-step n={n} inverse={int(inv)}: columns \S*tile\S+, rows \S*tile", err)) == 1, err
+        else:
+            halves = [int(h) for h in re.findall(rf"tile n=(\d+) of {n} inverse={int(inv)} ", err)]
+            assert len(halves) == 2 and halves[0] * halves[1] == n, err

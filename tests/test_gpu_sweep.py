@@ -215,3 +215,18 @@ def test_tables_made_under_capture():
             g.replay()
         torch.cuda.synchronize()
         assert rel_l2(cplx(y.cpu().numpy()), np.fft.fft(cplx(x.cpu().numpy()), axis=-1)) <= ABS_FLOAT_BOUND, rep
+
+
+@pytest.mark.parametrize("n,path", [(2176, "fast variant rtc_c2c2176"), (3162, "fast variant rtc_c2c3162"), (2809, "Bluestein blue8192"),
+                                    (4093, "Bluestein blue8192"), (5002, "Bluestein blue16384"), (8191, "Bluestein blue16384")])
+def test_large_prime_lengths_take_their_path(n, path, monkeypatch, capfd):
+    """Above 2048 points: rows compiled for factors of 17 .. 31, Bluestein's kernel for larger
+    ones where it is exact enough (2809 = 53^2 in a convolution 0.69 full)."""
+    lib = kissfft_amd.load("float")
+    monkeypatch.setenv("KISSFFT_AMD_VERBOSE", "1")
+    lib.L.kiss_fft_cleanup()
+    x = np.random.default_rng(n).uniform(-1, 1, (2, n, 2)).astype(np.float32)
+    y = np.zeros_like(x)
+    lib.fft_batch(lib.fft_alloc(n), x, y, 2, n, n)
+    assert rel_l2(cplx(y), np.fft.fft(cplx(x), axis=-1)) <= ABS_FLOAT_BOUND
+    assert path in capfd.readouterr().err
