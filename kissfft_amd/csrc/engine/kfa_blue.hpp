@@ -10,8 +10,8 @@
 // i.e. X = w * IFFT_M( FFT_M(x*w, zero-padded) * B ),  B = FFT_M(conj(w) wrapped) / M.
 // One line per T threads, entirely in LDS: the chirp multiply on load, the forward M-point
 // schedule, the pointwise product with B, the inverse schedule, the chirp on store.
-// w (N entries) and B (M entries) are computed in FP64 on the host; B is rounded once, w by
-// the variants that read it in float.
+// w (N entries) and B (M entries) are computed in FP64 on the host; B is rounded once, w as the
+// variant asks (CHIRP_*).
 #pragma once
 
 #include "kfa_tile.hpp"
@@ -152,7 +152,7 @@ struct BlueArgs {
     void *out;
     const void *stw_f, *stw_i;  // stage tables of the M-point schedule, and of it backwards
     const void *chirp;          // w[n], n < N, float2
-    const void *chirp64;        // the same in FP64 (null where no variant of the length reads it)
+    const void *chirp_wide;     // the same as the variant's CHIRP asks (null where none does)
     const void *bfft;           // B[m], m < M
     int n;
     long long nlines;
@@ -161,21 +161,41 @@ struct BlueArgs {
     FastSeg seg[KFA_MAX_SEG];
 };
 
-// Entries of the chirp table.
-template <bool WIDE>
-struct Chirp {
+// How the products with the chirp are made (template argument CHIRP):
+//   CHIRP_F32   float entries;
+//   CHIRP_PAIR  on load, entries of two floats, the value and what float leaves of it: the
+//               product is rounded, the table is not;
+//   CHIRP_F64   on load and store in FP64, rounded once.
+enum { CHIRP_F32 = 0, CHIRP_PAIR = 1, CHIRP_F64 = 2 };
+
+struct ChirpPair {
+    float r, i, rest_r, rest_i;
+};
+__device__ __forceinline__ Cf conv_mul(Cf v, ChirpPair w)
+{
+    const float r = __builtin_fmaf(v.r, w.rest_r, -(v.i * w.rest_i));
+    const float i = __builtin_fmaf(v.r, w.rest_i, v.i * w.rest_r);
+    return Cf{__builtin_fmaf(v.r, w.r, __builtin_fmaf(-v.i, w.i, r)), __builtin_fmaf(v.r, w.i, __builtin_fmaf(v.i, w.r, i))};
+}
+
+template <int CHIRP>
+struct ChirpTable {
     typedef float2 type;
     __device__ __forceinline__ static const type *of(const BlueArgs &a) { return reinterpret_cast<const type *>(a.chirp); }
 };
 template <>
-struct Chirp<true> {
+struct ChirpTable<CHIRP_PAIR> {
+    typedef ChirpPair type;
+    __device__ __forceinline__ static const type *of(const BlueArgs &a) { return reinterpret_cast<const type *>(a.chirp_wide); }
+};
+template <>
+struct ChirpTable<CHIRP_F64> {
     typedef Cd type;
-    __device__ __forceinline__ static const type *of(const BlueArgs &a) { return reinterpret_cast<const type *>(a.chirp64); }
+    __device__ __forceinline__ static const type *of(const BlueArgs &a) { return reinterpret_cast<const type *>(a.chirp_wide); }
 };
 
 // The Bluestein body for workgroup `blk` of its launch (see k_fast_body).
-// WIDE: the products with the chirp on load (bit 0) and on store (bit 1) in FP64.
-template <int T, int LPB, int WIDE, class RS>
+template <int T, int LPB, int CHIRP, class RS>
 __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
 {
     typedef F32::store2 St;
@@ -191,8 +211,8 @@ __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
     const long long gl = blk * LPB + line;
     const bool ok = gl < a.nlines;
     const int n = a.n;
-    const auto *chirp_in = Chirp<(WIDE & 1) != 0>::of(a);
-    const auto *chirp_out = Chirp<(WIDE & 2) != 0>::of(a);
+    const auto *chirp_in = ChirpTable<CHIRP>::of(a);
+    const auto *chirp_out = ChirpTable<CHIRP == CHIRP_F64 ? CHIRP_F64 : CHIRP_F32>::of(a);
 
     const St *src;
     St *dst;
@@ -219,10 +239,10 @@ __device__ __forceinline__ void k_blue_body(const BlueArgs &a, long long blk)
         }
 }
 
-template <int T, int LPB, int WIDE, class RS>
+template <int T, int LPB, int CHIRP, class RS>
 __global__ void __launch_bounds__(T *LPB) k_blue(BlueArgs a)
 {
-    k_blue_body<T, LPB, WIDE, RS>(a, blockIdx.x);
+    k_blue_body<T, LPB, CHIRP, RS>(a, blockIdx.x);
 }
 
 }  // namespace kfa

@@ -1146,7 +1146,7 @@ static int launch_rtile(const TileChoice &tc, RealTileArgs a, long long howmany,
 // ------------------------------------------------------------------------------------
 struct BlueChoice {
     const BlueVariant *v = nullptr;
-    DevBuf mem_f, mem_i, mem_chirp, mem_chirp64, mem_bfft;
+    DevBuf mem_f, mem_i, mem_chirp, mem_chirp_wide, mem_bfft;
     const BlueVariant *vf = nullptr;  // in a multi-batch (null: v there too), with its stage tables
     DevBuf fmem_f, fmem_i;
 };
@@ -1235,17 +1235,28 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
         const int M = bc->v->M;
         const double pi = 3.14159265358979323846264338327;
         const double sg = P.inverse ? 1.0 : -1.0;
-        std::vector<double> wr(n), wi(n), hw64(2 * n);
+        std::vector<double> wr(n), wi(n);
         std::vector<float> hw(2 * n);
         for (long long i = 0; i < n; ++i) {
             const long long q = (i * i) % (2 * n);  // n^2 mod 2N: exact phase reduction
             const double ph = sg * pi * (double)q / (double)n;
             wr[i] = cos(ph);
             wi[i] = sin(ph);
-            hw64[2 * i] = wr[i];
-            hw64[2 * i + 1] = wi[i];
             hw[2 * i] = (float)wr[i];
             hw[2 * i + 1] = (float)wi[i];
+        }
+        // (a length's variants ask for one wide form at most)
+        const int wide = std::max(bc->v->chirp, bc->vf ? bc->vf->chirp : (int)CHIRP_F32);
+        std::vector<double> hwide(wide != CHIRP_F32 ? 2 * n : 0);
+        for (long long i = 0; i < (long long)hwide.size() / 2; ++i) {
+            if (wide == CHIRP_F64) {
+                hwide[2 * i] = wr[i];
+                hwide[2 * i + 1] = wi[i];
+            } else {
+                const float pair[4] = {hw[2 * i], hw[2 * i + 1], (float)(wr[i] - hw[2 * i]),
+                                       (float)(wi[i] - hw[2 * i + 1])};
+                memcpy(&hwide[2 * i], pair, 16);
+            }
         }
         std::vector<double> br(M, 0.0), bi(M, 0.0);
         for (long long m = 0; m < n; ++m) {
@@ -1273,8 +1284,7 @@ static int blue_choice(DevPlan &P, std::shared_ptr<const BlueChoice> &out)
         if ((rc = stage_tables(*bc->v, bc->mem_f, bc->mem_i)) ||
             (bc->vf && (rc = stage_tables(*bc->vf, bc->fmem_f, bc->fmem_i))) ||
             (rc = dev_upload(hw.data(), hw.size() * 4, bc->mem_chirp)) ||
-            ((bc->v->wide || (bc->vf && bc->vf->wide)) &&
-             (rc = dev_upload(hw64.data(), hw64.size() * 8, bc->mem_chirp64))) ||
+            (wide != CHIRP_F32 && (rc = dev_upload(hwide.data(), hwide.size() * 8, bc->mem_chirp_wide))) ||
             (rc = dev_upload(hb.data(), hb.size() * 4, bc->mem_bfft)))
             return rc;
         if (env_flag("KISSFFT_AMD_VERBOSE", false))
@@ -1291,7 +1301,7 @@ static void blue_args(const BlueChoice &bc, int n, BlueArgs &b)
     b.stw_f = bc.mem_f.get();
     b.stw_i = bc.mem_i.get();
     b.chirp = bc.mem_chirp.get();
-    b.chirp64 = bc.mem_chirp64.get();
+    b.chirp_wide = bc.mem_chirp_wide.get();
     b.bfft = bc.mem_bfft.get();
     b.n = n;
 }

@@ -82,8 +82,8 @@ struct BlueArgs;
 // Bluestein variants (kfa_blue.hpp): one convolution length M, float.
 struct BlueVariant {
     int M;
-    int T, LPB;  // (k_blue<T, LPB, wide, Radices<tw_pad, radices...>>)
-    int wide;    // products with the chirp in FP64: 1 on load, 2 on store
+    int T, LPB;  // (k_blue<T, LPB, chirp, Radices<tw_pad, radices...>>)
+    int chirp;   // CHIRP_* (kfa_blue.hpp)
     std::vector<int> radices;
     int tw_pad;
     size_t lds;

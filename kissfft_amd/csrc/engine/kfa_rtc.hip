@@ -832,7 +832,7 @@ int rtc_fused(const std::vector<FusedMember> &m, int NT, hipFunction_t *fn)
               << (unit ? "true" : "false") << ">(*static_cast<const kfa::FastArgs *>(t.arg[" << i << "]), " << blk
               << ");\n";
         } else {
-            k << "kfa::k_blue_body<" << bv->T << ", " << bv->LPB << ", " << bv->wide << ", kfa::Radices<" << bv->tw_pad << rs
+            k << "kfa::k_blue_body<" << bv->T << ", " << bv->LPB << ", " << bv->chirp << ", kfa::Radices<" << bv->tw_pad << rs
               << ">>(*static_cast<const kfa::BlueArgs *>(t.arg[" << i << "]), " << blk << ");\n";
         }
         k << "        return;\n    }\n";

@@ -262,23 +262,23 @@ const std::vector<PlaneVariant> &plane_registry()
     return *reg;
 }
 
-template <int T, int LPB, int WIDE, class RS>
+template <int T, int LPB, int CHIRP, class RS>
 static int launch_blue(const BlueArgs &a, hipStream_t s)
 {
     const size_t lds = (size_t)LPB * conv_slots(RS::N()) * sizeof(float2);
     static std::once_flag once;
     std::call_once(once, [=] {
-        (void)hipFuncSetAttribute((const void *)k_blue<T, LPB, WIDE, RS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        (void)hipFuncSetAttribute((const void *)k_blue<T, LPB, CHIRP, RS>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)lds);
     });
     const long long blocks = (a.nlines + LPB - 1) / LPB;
     if (blocks <= 0)
         return 0;
-    hipLaunchKernelGGL((k_blue<T, LPB, WIDE, RS>), dim3((unsigned)blocks), dim3(T * LPB), lds, s, a);
+    hipLaunchKernelGGL((k_blue<T, LPB, CHIRP, RS>), dim3((unsigned)blocks), dim3(T * LPB), lds, s, a);
     return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
-template <int T, int LPB, int WIDE, int... R>
+template <int T, int LPB, int CHIRP, int... R>
 static void add_blue(std::vector<BlueVariant> &v, const char *name, bool fused = false)
 {
     typedef Radices<2, R...> RS;
@@ -291,8 +291,8 @@ static void add_blue(std::vector<BlueVariant> &v, const char *name, bool fused =
     f.tw_pad = 2;
     f.lds = (size_t)LPB * conv_slots(RS::N()) * 8;
     f.name = name;
-    f.wide = WIDE;
-    f.launch = &launch_blue<T, LPB, WIDE, RS>;
+    f.chirp = CHIRP;
+    f.launch = &launch_blue<T, LPB, CHIRP, RS>;
     f.fused = fused;
     v.push_back(f);
 }
@@ -301,32 +301,31 @@ const std::vector<BlueVariant> &blue_registry()
 {
     static std::vector<BlueVariant> *reg = [] {
         auto *v = new std::vector<BlueVariant>();
-        // The chirp on load in FP64 (third argument 1) for 64, 128, 512 points and the fused
-        // 2048: with both products in float they are 0.4 .. 1 % less exact than with the line
-        // staged through LDS between the steps (512 points 1.411e-7 rel-L2 against 1.405e-7, now
-        // 1.385e-7; 2048 fused 1.617e-7 against 1.610e-7, now 1.595e-7).  On load and store
-        // it takes 3 % of the time of 64 .. 512 points, on load alone 1-2 %; 64 uneven batches in
-        // one fused launch 43.4 / 43.9 / 44.3 us with none, load, both.  Both (3) from 8192 points,
+        // CHIRP_PAIR for 64, 128, 512 points and the fused 2048: with float entries they are 0.4 ..
+        // 1 % less exact than with the line staged through LDS between the steps (ratio of the
+        // errors over 286 lengths: 64 points 1.007, now 0.985, 128 1.010 / 0.992, 512 1.005 / 0.993,
+        // fused 2048 1.0045 / 0.997).  64 uneven batches in one fused launch 36.8 us with float
+        // entries, 37.4 with pairs, 38.2 with FP64 products on load.  CHIRP_F64 from 8192 points,
         // where it costs nothing that can be measured: -2.8 % of the error.
-        add_blue<8, 8, 1, 8, 8>(*v, "blue64_88_t8x8");
-        add_blue<8, 8, 1, 8, 16>(*v, "blue128_816_t8x8");
-        add_blue<16, 4, 0, 16, 16>(*v, "blue256_1616_t16x4");
-        add_blue<64, 2, 1, 8, 8, 8>(*v, "blue512_888_t64x2");
-        add_blue<128, 2, 0, 8, 8, 4, 4>(*v, "blue1024_8844_t128x2");
+        add_blue<8, 8, CHIRP_PAIR, 8, 8>(*v, "blue64_88_t8x8");
+        add_blue<8, 8, CHIRP_PAIR, 8, 16>(*v, "blue128_816_t8x8");
+        add_blue<16, 4, CHIRP_F32, 16, 16>(*v, "blue256_1616_t16x4");
+        add_blue<64, 2, CHIRP_PAIR, 8, 8, 8>(*v, "blue512_888_t64x2");
+        add_blue<128, 2, CHIRP_F32, 8, 8, 4, 4>(*v, "blue1024_8844_t128x2");
         // The last argument true: only in a multi-batch, whose fused launch runs members of one
         // workgroup size, shares their registers and LDS among them, and is 256 threads wide with
         // most row kernels; 16 values a thread there, 8 in a launch of their own.
         // c2c 1009 x4096 27.4 us, 32.2 with 128 threads a line, 30.9 with 16, 16, 8 at 128; but
         // 64 uneven batches in one fused launch 45.1, 45.1 and 43.4 us
-        add_blue<256, 1, 0, 8, 8, 8, 4>(*v, "blue2048_8884_t256");
-        add_blue<128, 2, 1, 16, 16, 8>(*v, "blue2048_16168_t128x2", true);
-        add_blue<512, 1, 0, 8, 8, 8, 8>(*v, "blue4096_8888_t512");
+        add_blue<256, 1, CHIRP_F32, 8, 8, 8, 4>(*v, "blue2048_8884_t256");
+        add_blue<128, 2, CHIRP_PAIR, 16, 16, 8>(*v, "blue2048_16168_t128x2", true);
+        add_blue<512, 1, CHIRP_F32, 8, 8, 8, 8>(*v, "blue4096_8888_t512");
         // lengths 1009 and 1997 among six lists in one multi-batch: both fused 20.9 us, 28.5 with 512
         // threads for 1997, which leaves 1009 a launch of its own; without 1009 18.7 against 18.0
-        add_blue<256, 1, 0, 8, 8, 8, 8>(*v, "blue4096_8888_t256", true);
+        add_blue<256, 1, CHIRP_F32, 8, 8, 8, 8>(*v, "blue4096_8888_t256", true);
         // lengths above 2048: 4093 x8 10.7 ms -> 16 us, 5002 x8 319 -> 23 us against the general kernel
-        add_blue<512, 1, 3, 8, 8, 8, 4, 4>(*v, "blue8192_88844_t512");
-        add_blue<1024, 1, 3, 8, 8, 8, 8, 4>(*v, "blue16384_88884_t1024");
+        add_blue<512, 1, CHIRP_F64, 8, 8, 8, 4, 4>(*v, "blue8192_88844_t512");
+        add_blue<1024, 1, CHIRP_F64, 8, 8, 8, 8, 4>(*v, "blue16384_88884_t1024");
         return v;
     }();
     return *reg;
