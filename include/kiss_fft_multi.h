@@ -31,7 +31,8 @@
  * KISSFFT_AMD_MULTI_PERSISTENT=1 at creation puts every single-pass item into the
  * persistent launch.  Results equal the per-item batched calls of the fixed-point builds
  * bit for bit, and the float builds' within the float tolerance.  Items must not share
- * output memory.  kiss_fft_cleanup() invalidates every multi-batch.
+ * output memory.  A multi-batch holds the device plans and tables it uses: kiss_fft_cleanup()
+ * does not invalidate it.
  */
 #ifndef KISS_FFT_MULTI_H
 #define KISS_FFT_MULTI_H

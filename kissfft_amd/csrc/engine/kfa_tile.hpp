@@ -96,7 +96,7 @@ constexpr int tile_pitch()
 // The kernel streams: what bounds it is the access pattern of its column side.  Measured
 // against the form that staged the tile through LDS on both sides of the stages (same
 // sizes, alternating runs): 64x96x120 x16 74.3 -> 72.0 us, real 1024x1000 x32 forward and
-// inverse 270 -> 263 us, c2c 2^20 x64 488 -> 483 us.
+// inverse 270 -> 263 us; c2c 2^20 x64 474 -> 412 us together with HALF.
 //
 // HALF hands one component over at a time (real parts, then imaginary parts through the
 // same space): half the LDS per line, so twice the lines fit a workgroup.  For lengths whose
