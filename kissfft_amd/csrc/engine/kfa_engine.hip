@@ -2875,6 +2875,16 @@ static int run_axis(DevPlan &P, const void *in, void *out, long long outer, long
 
 namespace kfa {
 
+// Whether a built-in plane (or slab) of these lengths exists: asked before plane_choice, whose
+// look-ups cost a call about half a microsecond each.
+static bool plane_built_in(int A, int B, int inverse, bool slab)
+{
+    for (const PlaneVariant &v : plane_registry())
+        if (v.A == A && v.B == B && v.inverse == inverse && (!slab || v.slab))
+            return true;
+    return false;
+}
+
 // The plane pass of a complex N-D transform: the axis done together with the last one
 // (paired; -1: every axis has a pass of its own) and its kernel.
 static int nd_plane(const std::vector<std::shared_ptr<DevPlan>> &P, const int *dims, long long howmany,
@@ -2897,6 +2907,8 @@ static int nd_plane(const std::vector<std::shared_ptr<DevPlan>> &P, const int *d
         for (int k = 0; k < ndims - 2; ++k)
             order.push_back(k);
         for (int k : order) {
+            if (!plane_built_in(dims[k], nb, P[ndims - 1]->inverse, k != ndims - 2))
+                continue;
             long long rs = 1;  // in-plane offsets are 32-bit
             for (int j = k + 1; j < ndims; ++j)
                 rs *= dims[j];
