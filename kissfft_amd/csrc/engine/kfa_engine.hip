@@ -1193,16 +1193,17 @@ static int largest_radix(const DevPlan &P)
 // 10.7 ms), but its error does not depend on the factor: it grows with the filled part of the
 // M points, 2n / M, where a direct sum's grows with the factor.  Over all 1832 lengths to 8192
 // with a largest factor of 53 .. 97, complex ones and real halves, its error is at most 1.00 times
-// that of float direct sums for factors above 73, and at most 0.99 times for 53 .. 73 up to
-// 2n / M = 0.7, from where it reaches 1.12 (8162 = 2 7 11 53: 1.96e-7 against 1.74e-7).  The lengths
-// it is not taken for run on the general kernel, whose sums are FP64 (8162: 0.7e-7).
+// that of float direct sums for factors above 73, and at most 0.99 times for 53 .. 73 up to 2n / M =
+// 0.70 .. 0.90, a hundredth more for each unit of the factor; taken for all it would reach 1.12 (8162 = 2 7 11 53:
+// 1.96e-7 against 1.74e-7).  The lengths it is not taken for run on the general kernel, whose
+// sums are FP64 (8162: 0.7e-7).
 static bool blue_exact(const DevPlan &P)
 {
     const int p = largest_radix(P);
     long long M = 64;
     while (M < 2LL * P.n - 1)
         M *= 2;
-    return p > 73 || (p > 50 && 20LL * P.n <= 7 * M);
+    return p > 73 || (p > 50 && 200LL * P.n <= (17 + p) * M);
 }
 
 // The Bluestein variant and tables for a float plan, decided once per plan.  v == nullptr: up to

@@ -74,8 +74,8 @@ static int shortest_compiled_row_as_set()
     return 0;
 }
 
-// Lengths whose direct sums are more exact than Bluestein's convolution keep them: factors up to
-// 73 in a convolution that is more than 0.7 full.
+// Lengths whose direct sums are more exact than Bluestein's convolution keep them: factors of 53
+// to 73 in a convolution that is more than 0.70 to 0.90 full.
 static int bluestein_only_where_exact()
 {
     const struct {
@@ -83,7 +83,8 @@ static int bluestein_only_where_exact()
         bool real;  // Bluestein for real rows of this half length
     } v[] = {{{53, 19}, false},         {{53, 19, 2}, false}, {{53, 19, 4}, false}, {{53, 11, 7}, false},
              {{53, 5, 5, 3, 2}, false}, {{53, 17, 9}, false}, {{73, 109}, true},    {{53, 53}, true},
-             {{79, 101}, true},         {{1021, 2}, true},    {{47, 47}, false},    {{61, 16, 4}, false}};
+             {{79, 101}, true},         {{1021, 2}, true},    {{47, 47}, false},    {{61, 16, 4}, false},
+             {{71, 16, 3}, true},       {{67, 53}, false}};
     for (const auto &x : v) {
         DevPlan P;
         int n = 1;
